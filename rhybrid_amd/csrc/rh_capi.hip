@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cfloat>
 #include <fstream>
 #include <iomanip>
@@ -80,6 +81,7 @@ struct Timer {
     struct Pending {
         hipEvent_t e0, e1;
         int species;  // the species the launch worked on, -1 for none
+        const char* also;  // a second name the launch is listed under
     };
     std::vector<Pending> pending;
     double ms = 0;
@@ -196,25 +198,29 @@ __global__ void k_dn_scatter(int nc, const float* __restrict__ y, const float* _
 template <typename Real>
 class Sim final : public Ctx {
 public:
-    // Per species: the sorted store (a, sub) and the destination of the next
-    // sort (d, sub_new), swapped after every sort; cnt_tile holds the 16-bit
-    // slot counts of pass 0 and then, for pass 1, each slot's offset inside
-    // its destination subcell's range (sub_new holds the ranges' starts).
+    // Per species: the store (a) with its tiles' slot tables (tab, live), and
+    // the destination of the next push (dst, tab_new, live_new), swapped after
+    // it.  `cap` places hold the segments; app_cap more, after them, the
+    // appendix of injected particles that wait for their first push.
     struct Species {
         rh_species_desc d;
         size_t cap = 0;
         DevBuf<Real> a[6], dst[6];
         DevBuf<uint8_t> a_lc, dst_lc;
-        DevBuf<uint32_t> sub, sub_new;
-        DevBuf<uint16_t> cnt_tile;
+        size_t app_cap = 0;
+        DevBuf<uint32_t> tab, tab_new;
+        DevBuf<uint8_t> live, live_new;
+        DevBuf<uint32_t> dtab, tile_list, seg_loc, seg_blk;  // k_tile_lists' input and output
+        DevBuf<uint32_t> scal;              // DevScalar
+        bool lists = false;    // particles may wait in neighbours' segments
+        bool compact = true;   // the segments hold no empty places
+        double np_est = 0;     // about how many particles there are
+        std::array<uint32_t, FILL_CLASSES> tile_fill{};  // of the store as last looked at (k_tile_fill)
+        double fill_np = 0;    // np_est then
         DevBuf<Real> partial;  // deposit: per-tile ghost partials (ntiles x next x 4)
-        // per tile, 1 if it held particles at the push (its slot table was
-        // written)
-        DevBuf<uint8_t> live_src;
         DevBuf<double> ave_n, ave_v;  // temporal averages: running charge and current sums (FP64)
         bool deposited = false;
-        bool pushed = false;  // pass 0 done, pass 1 pending
-        PushParams pp{};      // parameters of the pending push
+        bool pushed = false;  // pushed into the other store, not yet swapped in
         // injector: listed cells in subcell-key order, their rates
         // (exosphere), per tile the first listed cell, per listed cell the
         // offset of its new particles past the store's end
@@ -226,9 +232,6 @@ public:
         DevBuf<uint32_t> inj_cbeg, inj_off;
         DevBuf<unsigned long long> inj_total;
         bool inj_pending = false;  // injected particles wait past the store's end
-        // at least 4 particles per cell at the end of the last rh_step call
-        // (the move's occupancy cap pays for such species only)
-        bool dense = true;
         // log counters: the push's own counters (maxVi per species), per
         // boundary cell (escapes, sum v^2, impacts, sum v^2), per injection
         // place sum v^2; host carries of the accumulators when their layout
@@ -240,20 +243,23 @@ public:
         double log_maxvi0 = 0;
         int64_t log_inj0 = 0;
         InjAppendix appendix() const {
-            return inj_pending ? InjAppendix{inj_cbeg.p, inj_off.p} : InjAppendix{nullptr, nullptr};
+            if (!inj_pending) return InjAppendix{nullptr, nullptr, 0, 0, 0};
+            const bool at_end = inj.kind == INJ_UNIFORM;
+            return InjAppendix{inj_cbeg.p, inj_off.p, at_end ? 0xFFFFFFFFu : (uint32_t)app_cap, (uint32_t)inj_slots,
+                               at_end ? 1 : 0};
         }
         PArrays<Real> A() { return {a[0].p, a[1].p, a[2].p, a[3].p, a[4].p, a[5].p, a_lc.p}; }
         PArrays<Real> Dst() { return {dst[0].p, dst[1].p, dst[2].p, dst[3].p, dst[4].p, dst[5].p, dst_lc.p}; }
         void swap_stores() {
             for (int q = 0; q < 6; ++q) std::swap(a[q].p, dst[q].p);
             std::swap(a_lc.p, dst_lc.p);
-            std::swap(sub.p, sub_new.p);
+            std::swap(tab.p, tab_new.p);
+            std::swap(live.p, live_new.p);
         }
         // the species' own stream for the particle phase of a step, the event
-        // that marks the end of its work there, and its scan's block sums
+        // that marks the end of its work there
         hipStream_t ss = nullptr;
         hipEvent_t done = nullptr;
-        std::vector<DevBuf<uint32_t>> scan_lv;
         Species() = default;
         Species(const Species&) = delete;
         Species& operator=(const Species&) = delete;
@@ -276,6 +282,8 @@ public:
     DevBuf<uint8_t> flg[RH_N_FLAGS];
     DevBuf<uint8_t> flg_fu;       // the fused field update's three inner flags in one byte per cell
     DevBuf<int> ext_cells, bc_cells;
+    DevBuf<int> bc_beg;             // per boundary cell its ranges (k_boundary)
+    DevBuf<CellRange> bc_range;
     int n_ext = 0, n_bc = 0;
     DevBuf<unsigned long long> dcount;
     DevBuf<double> diag_partial;
@@ -286,7 +294,8 @@ public:
     DevBuf<uint8_t> dep_count;
     DevBuf<uint16_t> dep_tlist;  // deposit gather lists of cell-target terms (next x 32)
     DevBuf<uint8_t> dep_tcount;
-    int kbits = 12;
+    DevBuf<uint16_t> slot_dir, slot_of;  // the tile shape's slots (tile_slots)
+    DevBuf<uint32_t> slot_code;          // and its extended cells' codes (tile_codes)
     bool timing = false;
     std::string timing_only;  // when not empty, only launches of this name are timed
     std::map<std::string, Timer> timers;
@@ -308,16 +317,11 @@ public:
             RH_HIP(hipGetDevice(&dev));
             RH_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
             lds_limit = (size_t)lds;
-            int lds_cu = 0;
-            RH_HIP(hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev));
-            lds_per_cu = (size_t)lds_cu;
         }
         choose_tiles(gd->tile);
         // dynamic LDS above the default 64 KiB (FP64 tiles of 64 cells)
         RH_HIP(hipFuncSetAttribute((const void*)k_deposit<Real>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)deposit_lds_bytes<Real>(g)));
-        RH_HIP(hipFuncSetAttribute((const void*)k_push_move<Real>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)std::max(push_move_lds_bytes<Real>(g), move_lds_bytes())));
         RH_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         ls = stream;
         RH_HIP(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming));
@@ -367,8 +371,18 @@ public:
         zero_u32.alloc(1);
         RH_HIP(hipMemsetAsync(zero_u32.p, 0, sizeof(uint32_t), stream));
         alloc_scan_levels(scan_lv);
-        kbits = 1;
-        while ((1 << kbits) < g.extk) ++kbits;
+        {
+            std::vector<uint16_t> dir(28), slot((size_t)g.next);
+            tile_slots(g, dir.data(), slot.data());
+            slot_dir.alloc(dir.size());
+            slot_of.alloc(slot.size());
+            RH_HIP(hipMemcpy(slot_dir.p, dir.data(), dir.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+            RH_HIP(hipMemcpy(slot_of.p, slot.data(), slot.size() * sizeof(uint16_t), hipMemcpyHostToDevice));
+            std::vector<uint32_t> code(2 * (size_t)g.next);
+            tile_codes(g, slot.data(), code.data(), code.data() + g.next);
+            slot_code.alloc(code.size());
+            RH_HIP(hipMemcpy(slot_code.p, code.data(), code.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        }
         RH_HIP(hipStreamSynchronize(stream));
     }
 
@@ -399,23 +413,6 @@ public:
     }
 
     size_t lds_limit = 65536;  // the device's LDS per workgroup (queried at creation)
-    size_t lds_per_cu = 0;     // and per CU
-
-    // The move pass (pass 1 of k_push_move) runs with at most MOVE_WG_PER_CU
-    // workgroups per CU, set through its dynamic LDS request: with fewer
-    // tiles' scattered stores in flight per CU it runs faster (the 128x96x96
-    // box: 500 us per launch at the 7 workgroups its registers allow, 483 at
-    // 5 or 6, 474 at 4, 526 at 3).  The push pass keeps the full occupancy,
-    // and so does the move of a species with fewer than 4 particles per cell
-    // (at the end of the last rh_step call): its move is set by a few crowded
-    // tiles, which the cap only starts later.
-    static constexpr int MOVE_WG_PER_CU = 4;
-    size_t move_lds_bytes(const Species* S_ = nullptr) const {
-        const size_t need = push_move_lds_bytes<Real>(g);
-        if (lds_per_cu == 0 || (S_ && !S_->dense)) return need;
-        const size_t cap = lds_per_cu / MOVE_WG_PER_CU - 1024;  // below the share, so MOVE_WG_PER_CU fit
-        return std::min(lds_limit, std::max(need, cap));
-    }
 
     // LDS of the largest per-tile kernels for a tile shape
     size_t tile_lds_bytes(const int* t) const {
@@ -425,7 +422,8 @@ public:
         h.ex = t[0] + 2; h.ey = t[1] + 2; h.ez = t[2] + 2;
         h.next = h.ex * h.ey * h.ez;
         h.extk = h.next * 8;
-        return std::max(deposit_lds_bytes<Real>(h), push_move_lds_bytes<Real>(h));
+        set_slots(h);
+        return std::max(deposit_lds_bytes<Real>(h), push_lds<Real>(h, 256, 0).bytes);
     }
 
     void choose_tiles(const int32_t* req) {
@@ -446,7 +444,7 @@ public:
                 t[d] /= 2;
             }
             // enough tiles to fill the chip when the grid is small
-            while (ntiles() < 4096) {
+            while (ntiles() < 8192) {
                 int d = -1;
                 for (int q = 0; q < 3; ++q)
                     if (t[q] > 2 && (d < 0 || t[q] > t[d])) d = q;
@@ -470,10 +468,11 @@ public:
         g.ex = g.tx + 2; g.ey = g.ty + 2; g.ez = g.tz + 2;
         g.next = g.ex * g.ey * g.ez;
         g.extk = g.next * 8;
+        set_slots(g);
         if (g.extk > MAX_EXTK) throw ArgError("tile extended region too large");
         const uint64_t nk = (uint64_t)g.ntiles * g.tc * 8;
         if (nk >= 0xFFFFFFFFull) throw ArgError("grid too large for 32-bit subcell keys");
-        if ((uint64_t)g.ntiles * g.extk >= 0xFFFFFFFFull) throw ArgError("tiles too small for this grid (slot table)");
+        if ((uint64_t)g.ntiles * std::max(g.extk, g.kt) >= 0xFFFFFFFFull) throw ArgError("tiles too small for this grid (slot table)");
         g.nkeys = (uint32_t)nk;
     }
 
@@ -487,6 +486,44 @@ public:
         n_bc = (int)cells.size();
         bc_cells.alloc(std::max<size_t>(cells.size(), 1));
         if (n_bc) RH_HIP(hipMemcpy(bc_cells.p, cells.data(), cells.size() * sizeof(int), hipMemcpyHostToDevice));
+        // where each cell's particles may be
+        std::vector<uint16_t> dir(28), slot((size_t)g.next);
+        tile_slots(g, dir.data(), slot.data());
+        std::vector<int> beg(1, 0);
+        std::vector<CellRange> range;
+        for (int n : cells) {
+            int c[3], b[3], l[3], lo[3], hi[3];
+            cell_ijk(g, n, c[0], c[1], c[2]);
+            const int dims[3] = {g.nx, g.ny, g.nz}, lt[3] = {g.ltx, g.lty, g.ltz}, nt[3] = {g.ntx, g.nty, g.ntz},
+                      t[3] = {g.tx, g.ty, g.tz};
+            for (int d = 0; d < 3; ++d) {
+                b[d] = c[d] >> lt[d];
+                l[d] = c[d] - (b[d] << lt[d]);
+                lo[d] = l[d] == 0 && (b[d] > 0 || g.per[d]);
+                hi[d] = l[d] == tile_width(dims[d], lt[d], b[d]) - 1 && (b[d] < nt[d] - 1 || g.per[d]);
+            }
+            const int T = b[0] + g.ntx * (b[1] + g.nty * b[2]);
+            range.push_back({T, (uint32_t)T * (uint32_t)g.kt + 8u * (uint32_t)(l[0] + (l[1] << g.ltx) + (l[2] << (g.ltx + g.lty)))});
+            for (int z = -lo[2]; z <= hi[2]; ++z)
+                for (int y = -lo[1]; y <= hi[1]; ++y)
+                    for (int x = -lo[0]; x <= hi[0]; ++x) {
+                        if (!x && !y && !z) continue;
+                        const int o[3] = {x, y, z};
+                        int s[3], e[3];
+                        for (int d = 0; d < 3; ++d) {
+                            s[d] = (b[d] + o[d] + nt[d]) % nt[d];
+                            e[d] = o[d] < 0 ? t[d] + 1 : (o[d] > 0 ? 0 : l[d] + 1);
+                        }
+                        const int S = s[0] + g.ntx * (s[1] + g.nty * s[2]);
+                        range.push_back({S, (uint32_t)S * (uint32_t)g.kt + slot[e[0] + g.ex * (e[1] + g.ey * e[2])]});
+                    }
+            beg.push_back((int)range.size());
+        }
+        bc_beg.alloc(beg.size());
+        bc_range.alloc(std::max<size_t>(range.size(), 1));
+        RH_HIP(hipMemcpy(bc_beg.p, beg.data(), beg.size() * sizeof(int), hipMemcpyHostToDevice));
+        if (!range.empty())
+            RH_HIP(hipMemcpy(bc_range.p, range.data(), range.size() * sizeof(CellRange), hipMemcpyHostToDevice));
     }
 
     // ---- launch helpers -------------------------------------------------
@@ -507,23 +544,27 @@ public:
     // read where species differ in size.
     void resolve_timers() {
         RH_HIP(hipStreamSynchronize(stream));
-        std::map<std::string, Timer> per_species;
+        std::map<std::string, Timer> further;
         for (auto& kv : timers) {
             for (auto& pe : kv.second.pending) {
                 float ms = 0;
                 RH_HIP(hipEventElapsedTime(&ms, pe.e0, pe.e1));
                 kv.second.ms += ms;
-                if (pe.species >= 0) {
-                    Timer& t = per_species[kv.first + ":" + std::to_string(pe.species)];
+                auto add = [&](const std::string& name) {
+                    Timer& t = further[name];
                     t.ms += ms;
                     t.launches++;
-                }
+                };
+                const std::string of = ":" + std::to_string(pe.species);
+                if (pe.species >= 0) add(kv.first + of);
+                if (pe.also) add(pe.also);
+                if (pe.also && pe.species >= 0) add(pe.also + of);
                 event_pool.push_back(pe.e0);
                 event_pool.push_back(pe.e1);
             }
             kv.second.pending.clear();
         }
-        for (auto& kv : per_species) {
+        for (auto& kv : further) {
             Timer& t = timers[kv.first];
             t.ms += kv.second.ms;
             t.launches += kv.second.launches;
@@ -538,10 +579,15 @@ public:
         ~SpeciesScope() { slot = prev; }
     };
 
+    // The launch that pushes a species' particles and moves them is listed
+    // under both names, "push" and "move".
     template <typename K, typename... Args>
     void launch(const char* name, K kernel, dim3 grid, dim3 block, size_t shmem, Args... args) {
         if ((size_t)grid.x * grid.y * grid.z == 0) return;
         hipEvent_t e0 = nullptr, e1 = nullptr;
+        const char* also = std::strcmp(name, "move") == 0 ? "push" : nullptr;
+        if (also && timing_only == also) { name = also; also = nullptr; }
+        if (!timing_only.empty()) also = nullptr;
         const bool timed = timing && (timing_only.empty() || timing_only == name);
         if (timed) {
             e0 = get_event();
@@ -553,7 +599,7 @@ public:
         if (timed) {
             RH_HIP(hipEventRecord(e1, ls));
             Timer& t = timers[name];
-            t.pending.push_back({e0, e1, timing_species});
+            t.pending.push_back({e0, e1, timing_species, also});
             t.launches++;
             if (t.pending.size() > 4096) resolve_timers();
         }
@@ -577,6 +623,8 @@ public:
         return {p, p + g.nc, p + 2 * (size_t)g.nc};
     }
 
+    TileTables tables(const Species& S_) const { return {S_.tab.p, S_.live.p, slot_dir.p, slot_of.p, S_.lists ? 1 : 0}; }
+
     Species& S(int s) {
         if (s < 0 || s >= (int)sp.size()) throw ArgError("bad species id");
         return *sp[s];
@@ -587,20 +635,28 @@ public:
     int add_species(const rh_species_desc* d) override {
         auto s = std::make_unique<Species>();
         s->d = *d;
-        s->sub.alloc((size_t)g.nkeys + 1);
-        s->sub_new.alloc((size_t)g.nkeys + 1);
-        RH_HIP(hipMemsetAsync(s->sub.p, 0, sizeof(uint32_t) * ((size_t)g.nkeys + 1), stream));
-        s->cnt_tile.alloc((size_t)g.ntiles * g.extk);
+        s->tab.alloc((size_t)g.ntiles * g.kt);
+        s->tab_new.alloc((size_t)g.ntiles * g.kt);
+        s->live.alloc((size_t)g.ntiles);
+        s->live_new.alloc((size_t)g.ntiles);
+        fill(s->live.p, (uint8_t)0, s->live.n);
+        s->seg_loc.alloc((size_t)g.ntiles);
+        s->seg_blk.alloc(cdiv(g.ntiles, TILES_PER_LIST_BLOCK));
+        s->dtab.alloc((size_t)g.ntiles * DIR_WORDS);
+        s->tile_list.alloc((size_t)g.ntiles * LIST_WORDS);
+        fill(s->dtab.p, 0u, s->dtab.n);
+        fill(s->tile_list.p, 0u, s->tile_list.n);
+        fill(s->seg_loc.p, 0u, s->seg_loc.n);
+        fill(s->seg_blk.p, 0u, s->seg_blk.n);
+        s->scal.alloc(SC_N);
+        fill(s->scal.p, 0u, s->scal.n);
         s->partial.alloc((size_t)g.ntiles * g.next * 4);
-        s->live_src.alloc((size_t)g.ntiles);
-        fill(s->live_src.p, (uint8_t)0, s->live_src.n);
         s->pcount.alloc((size_t)C_N * COUNTER_SLOTS);
         RH_HIP(hipMemsetAsync(s->pcount.p, 0, sizeof(unsigned long long) * C_N * COUNTER_SLOTS, stream));
         s->bc_acc.alloc((size_t)std::max(n_bc, 1) * 4);
         fill(s->bc_acc.p, 0.0, s->bc_acc.n);
         ensure_capacity(*s, (size_t)std::max<int64_t>(d->capacity, 0));
         ensure_averages(*s);
-        alloc_scan_levels(s->scan_lv);
         sp.push_back(std::move(s));
         RH_HIP(hipStreamSynchronize(stream));
         return (int)sp.size() - 1;
@@ -610,10 +666,36 @@ public:
         if (cap <= s.cap && s.cap > 0) return;
         if (cap >= 0xFFFFFFFFull) throw CapError("particle capacity exceeds 32-bit indices");
         cap = std::max<size_t>(cap, 64);
-        for (int q = 0; q < 6; ++q) { s.a[q].alloc(cap); s.dst[q].alloc(cap); }
-        s.a_lc.alloc(cap);
-        s.dst_lc.alloc(cap);
+        // (room for the appendix of a usual injector: its walls' cells at up
+        // to eight places; a larger one reallocates)
+        if (s.app_cap == 0)
+            s.app_cap = 8 * (size_t)std::max(std::max(g.nx * g.ny, g.ny * g.nz), g.nx * g.nz);
+        s.app_cap = std::min(s.app_cap, (size_t)0xFFFFFFFFull - cap);
+        const size_t n = cap + s.app_cap;
+        for (int q = 0; q < 6; ++q) { s.a[q].alloc(n); s.dst[q].alloc(n); }
+        s.a_lc.alloc(n);
+        s.dst_lc.alloc(n);
         s.cap = cap;
+    }
+
+    // Room for `places` injected particles past the store's capacity; the
+    // stored particles stay.
+    void ensure_appendix(Species& s, size_t places) {
+        if (places <= s.app_cap) return;
+        if (s.cap + places > 0xFFFFFFFFull) throw CapError("particle capacity and injection places exceed 32-bit indices");
+        const size_t n = s.cap + places;
+        RH_HIP(hipStreamSynchronize(stream));
+        auto grow = [&](auto& b) {
+            typename std::remove_reference<decltype(b)>::type t;
+            t.alloc(n);
+            RH_HIP(hipMemcpyAsync(t.p, b.p, s.cap * sizeof(*t.p), hipMemcpyDeviceToDevice, stream));
+            RH_HIP(hipStreamSynchronize(stream));
+            b = std::move(t);
+        };
+        for (int q = 0; q < 6; ++q) { grow(s.a[q]); s.dst[q].alloc(n); }
+        grow(s.a_lc);
+        s.dst_lc.alloc(n);
+        s.app_cap = places;
     }
 
     void upload_field(int id, const double* data) override {
@@ -683,6 +765,20 @@ public:
         std::vector<uint32_t> sub((size_t)g.nkeys + 1, 0);
         for (int64_t p = 0; p < n; ++p) sub[key[p] + 1]++;
         for (size_t k2 = 0; k2 < g.nkeys; ++k2) sub[k2 + 1] += sub[k2];
+        // the tiles' tables: their subcells, and no particle in a halo slot
+        const size_t ns = (size_t)g.tc * 8;
+        std::vector<uint32_t> tab((size_t)g.ntiles * g.kt);
+        std::vector<uint8_t> live((size_t)g.ntiles);
+        std::vector<uint32_t> dtab((size_t)g.ntiles * DIR_WORDS);
+        for (size_t T = 0; T < (size_t)g.ntiles; ++T) {
+            uint32_t* t = tab.data() + T * g.kt;
+            std::copy(sub.begin() + T * ns, sub.begin() + (T + 1) * ns, t);
+            std::fill(t + ns, t + g.kt, sub[(T + 1) * ns]);
+            live[T] = sub[(T + 1) * ns] > sub[T * ns];
+            uint32_t* d = dtab.data() + T * DIR_WORDS;
+            std::fill(d, d + DIR_WORDS, sub[(T + 1) * ns]);
+            d[DIR_OWN] = sub[T * ns];
+        }
         std::vector<uint32_t> fillp(sub.begin(), sub.end() - 1);
         std::vector<Real> h[6];
         for (int q = 0; q < 6; ++q) h[q].resize((size_t)n);
@@ -699,10 +795,18 @@ public:
         for (int q = 0; q < 6; ++q)
             RH_HIP(hipMemcpyAsync(S_.a[q].p, h[q].data(), sizeof(Real) * n, hipMemcpyHostToDevice, stream));
         RH_HIP(hipMemcpyAsync(S_.a_lc.p, hl.data(), n, hipMemcpyHostToDevice, stream));
-        RH_HIP(hipMemcpyAsync(S_.sub.p, sub.data(), sizeof(uint32_t) * sub.size(), hipMemcpyHostToDevice, stream));
-        RH_HIP(hipStreamSynchronize(stream));
+        RH_HIP(hipMemcpyAsync(S_.tab.p, tab.data(), sizeof(uint32_t) * tab.size(), hipMemcpyHostToDevice, stream));
+        RH_HIP(hipMemcpyAsync(S_.live.p, live.data(), live.size(), hipMemcpyHostToDevice, stream));
+        uint32_t sc[SC_N] = {};
+        sc[SC_END] = (uint32_t)n;
+        RH_HIP(hipMemcpyAsync(S_.scal.p, sc, sizeof(sc), hipMemcpyHostToDevice, stream));
+        RH_HIP(hipMemcpyAsync(S_.dtab.p, dtab.data(), sizeof(uint32_t) * dtab.size(), hipMemcpyHostToDevice, stream));
+        tile_lists(S_, "sort_still");
+        look_at_fill(S_);
         S_.pushed = false;
         S_.inj_pending = false;
+        S_.lists = false;
+        S_.compact = true;
     }
 
     // live particles (those removed by the boundary conditions stay stored,
@@ -717,38 +821,39 @@ public:
     void download_particles(int s, int64_t capn, int64_t* cell, double* st) override {
         Species& S_ = S(s);
         if (S_.pushed) throw StateError("download between propagate and wait_particle_sends");
-        flush_injected(S_);
-        std::vector<uint32_t> sub((size_t)g.nkeys + 1);
-        RH_HIP(hipMemcpyAsync(sub.data(), S_.sub.p, sizeof(uint32_t) * sub.size(), hipMemcpyDeviceToHost, stream));
-        RH_HIP(hipStreamSynchronize(stream));
-        const uint32_t np = sub[g.nkeys];
+        if (S_.lists || S_.inj_pending) merge(S_);  // every particle in its own tile's segment
+        std::vector<uint32_t> tab((size_t)g.ntiles * g.kt);
+        std::vector<uint8_t> live((size_t)g.ntiles);
+        RH_HIP(hipMemcpyAsync(tab.data(), S_.tab.p, sizeof(uint32_t) * tab.size(), hipMemcpyDeviceToHost, stream));
+        RH_HIP(hipMemcpyAsync(live.data(), S_.live.p, live.size(), hipMemcpyDeviceToHost, stream));
+        const uint32_t end = scalar(S_, SC_END);
         std::vector<Real> h[6];
         for (int q = 0; q < 6; ++q) {
-            h[q].resize(np);
-            if (np) RH_HIP(hipMemcpy(h[q].data(), S_.a[q].p, sizeof(Real) * np, hipMemcpyDeviceToHost));
+            h[q].resize(end);
+            if (end) RH_HIP(hipMemcpy(h[q].data(), S_.a[q].p, sizeof(Real) * end, hipMemcpyDeviceToHost));
         }
-        // the cell of a particle follows from the subcell range holding it
-        std::vector<uint32_t> hc(np);
-        for (uint32_t key = 0; key < g.nkeys; ++key) {
-            if (sub[key] == sub[key + 1]) continue;
-            const int T = (int)(key / (uint32_t)(g.tc * 8)), lc = (int)((key % (uint32_t)(g.tc * 8)) >> 3);
+        // in slot order; the cell of a particle follows from the slots holding it
+        int64_t out = 0;
+        for (int T = 0; T < g.ntiles; ++T) {
+            if (!live[T]) continue;
             int ox, oy, oz;
             tile_origin(g, T, ox, oy, oz);
-            const uint32_t c = (uint32_t)cell_index(g, ox + lc % g.tx, oy + (lc / g.tx) % g.ty, oz + lc / (g.tx * g.ty));
-            for (uint32_t p = sub[key]; p < sub[key + 1]; ++p) hc[p] = c;
-        }
-        int64_t out = 0;
-        for (uint32_t p = 0; p < np; ++p) {
-            if (h[0][p] < Real(0)) continue;
-            if (out >= capn) throw CapError("download buffer too small");
-            if (cell) cell[out] = hc[p];
-            if (st) {
-                double* q = st + 7 * out;
-                q[0] = (double)h[0][p] * g.dx; q[1] = (double)h[1][p] * g.dx; q[2] = (double)h[2][p] * g.dx;
-                q[3] = (double)h[3][p]; q[4] = (double)h[4][p]; q[5] = (double)h[5][p];
-                q[6] = S_.d.w;
+            for (int lc = 0; lc < g.tc; ++lc) {
+                const uint32_t* t = tab.data() + (size_t)T * g.kt + 8 * lc;
+                const int c = cell_index(g, ox + lc % g.tx, oy + (lc / g.tx) % g.ty, oz + lc / (g.tx * g.ty));
+                for (uint32_t p = t[0]; p < t[8]; ++p) {
+                    if (h[0][p] < Real(0)) continue;
+                    if (out >= capn) throw CapError("download buffer too small");
+                    if (cell) cell[out] = c;
+                    if (st) {
+                        double* q = st + 7 * out;
+                        q[0] = (double)h[0][p] * g.dx; q[1] = (double)h[1][p] * g.dx; q[2] = (double)h[2][p] * g.dx;
+                        q[3] = (double)h[3][p]; q[4] = (double)h[4][p]; q[5] = (double)h[5][p];
+                        q[6] = S_.d.w;
+                    }
+                    ++out;
+                }
             }
-            ++out;
         }
     }
 
@@ -769,31 +874,133 @@ public:
         pp.use_gravity = P.use_gravity;
         pp.initial_flow_through = P.initial_flow_through;
         pp.still = 0;
-        pp.live = S_.live_src.p;
+        push(S_, pp, "move");
+    }
+
+    // The push's round (the particles that wait in LDS) and threads, from how
+    // full the tiles were when last looked at: the cheapest of every number of
+    // threads with the largest round that lets a CU's LDS hold so many
+    // workgroups.  A tile costs its passes over the threads, one more for what
+    // does not depend on the particles, and three times the passes if it does
+    // not fit the round; a CU works at its full rate with 24 waves or more, at
+    // (waves / 24)^0.65 of it below.  Measured per species: 128x96x96 with 32
+    // particles per cell (2,048 a tile) 456 us with 2 x 768 threads, 475 with
+    // 2 x 1,024, 511 with 2 x 512, 714 with 1 x 768; 128x64x64 with 8 (512 a
+    // tile) 76 us with 5 x 256, 93 with 4 x 512; 64x48x48 (1,090 a tile) 77 us
+    // with 3 x 512, 94 with 3 x 768.  The results do not depend on the choice.
+    struct PushShape { int round, threads, parts; };
+    PushShape choose_push(Species& S_) const {
+        const bool looked = S_.fill_np > 0 && S_.np_est < 1.5 * S_.fill_np;
+        const double mean = S_.np_est / g.ntiles;
+        std::array<uint32_t, FILL_CLASSES> one{};
+        one[fill_class((uint32_t)std::min(mean, 1e6))] = 5;
+        one[fill_class((uint32_t)std::min(mean + 3.0 * std::sqrt(mean), 1e6))] += 1;
+        const auto& fill = looked ? S_.tile_fill : one;
+        double tiles = 0, np = 0;
+        for (int c = 1; c < FILL_CLASSES; ++c) { tiles += fill[c]; np += fill[c] * (64.0 * c - 32.0); }
+        // parts of a slot with four to eight particles each
+        int lq = 0;
+        const double per_slot = tiles > 0 ? np / tiles / (8.0 * g.tc) : 0;
+        while ((g.nslot + 1) << (lq + 1) <= 1 << SLOT_BITS && per_slot >= (16 << lq)) ++lq;
+        PushShape best{256, 256, lq};
+        double best_cost = 1e300;
+        for (int k = 8; k >= 1; --k) {
+            const size_t lds = std::min(lds_limit, (size_t)PUSH_MAX_LDS) / k - 1024;
+            int round = 64 * (FILL_CLASSES - 2);
+            while (round > 256 && push_lds<Real>(g, round, lq).bytes > lds) round -= 64;
+            if (push_lds<Real>(g, round, lq).bytes > lds && k > 1) continue;
+            for (int threads : {256, 512, 768, 1024}) {
+                const double waves = std::min(24.0, k * threads / 64.0);
+                double cost = 0;
+                for (int c = 1; c < FILL_CLASSES; ++c) {
+                    const double passes = std::ceil((64.0 * c - 32.0) / threads);
+                    cost += fill[c] * (64 * c <= round && c < FILL_CLASSES - 1 ? passes + 1 : 3 * passes + 1);
+                }
+                cost *= threads * std::pow(24.0 / waves, 0.65);
+                if (cost < best_cost) { best_cost = cost; best = {round, threads, lq}; }
+            }
+        }
+        return best;
+    }
+
+    // The push of every particle into the other store.
+    void push(Species& S_, const PushParams& pp, const char* name) {
         prepare_push_fields();
-        launch("push", k_push_move<Real>, tile_grid(), PM_THREADS, push_move_lds_bytes<Real>(g), g, pp,
-               (const uint32_t*)pf_tile.p,
-               S_.A(), S_.Dst(), (const uint32_t*)S_.sub.p, S_.appendix(), S_.cnt_tile.p,
-               (const uint32_t*)S_.sub_new.p, S_.pcount.p, kbits, 0, (uint32_t)S_.cap);
-        S_.pp = pp;
+        const PushShape sh = choose_push(S_);
+        if (sh.threads == 256) push_shape<256>(S_, pp, name, sh.round, sh.parts);
+        else if (sh.threads == 512) push_shape<512>(S_, pp, name, sh.round, sh.parts);
+        else if (sh.threads == 768) push_shape<768>(S_, pp, name, sh.round, sh.parts);
+        else push_shape<1024>(S_, pp, name, sh.round, sh.parts);
         S_.pushed = true;
     }
 
-    // Merge injected particles that wait past the store's end into the
-    // sorted store without pushing anything (the same two passes, still).
-    void flush_injected(Species& S_) {
-        if (!S_.inj_pending) return;
+    // the default tile shapes are known to the compiler
+    template <int NT>
+    void push_shape(Species& S_, const PushParams& pp, const char* name, int round, int lq) {
+        const bool plain = pp.accelerate && !pp.use_gravity && !pp.initial_flow_through && !pp.still;
+        if (!plain) push_launch<NT, -1, -1, -1, false>(S_, pp, name, round, lq);
+        else if (g.tx == 4 && g.ty == 4 && g.tz == 4) push_launch<NT, 2, 2, 2, true>(S_, pp, name, round, lq);
+        else if (g.tx == 2 && g.ty == 2 && g.tz == 2) push_launch<NT, 1, 1, 1, true>(S_, pp, name, round, lq);
+        else push_launch<NT, -1, -1, -1, true>(S_, pp, name, round, lq);
+    }
+
+    static constexpr int PUSH_MAX_LDS = 156 * 1024;
+    template <int NT, int LX, int LY, int LZ, bool PLAIN>
+    void push_launch(Species& S_, const PushParams& pp, const char* name, int round, int lq) {
+        const size_t lds = push_lds<Real>(g, round, lq).bytes;
+        auto kernel = k_push_sort<Real, NT, LX, LY, LZ, PLAIN>;
+        if (lds > 65536)
+            RH_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        launch(name, kernel, tile_grid(), NT, lds, g, pp,
+               (const uint32_t*)pf_tile.p, S_.A(), S_.Dst(), (const uint16_t*)slot_dir.p, (const uint16_t*)slot_of.p,
+               (const uint32_t*)slot_code.p, S_.tab_new.p, S_.dtab.p, S_.live_new.p, (const uint32_t*)S_.tile_list.p, (const uint32_t*)S_.seg_loc.p,
+               (const uint32_t*)S_.seg_blk.p, S_.appendix(), S_.scal.p, S_.pcount.p, (uint32_t)S_.cap, round, lq);
+    }
+
+    // The tiles' lists of the store as it is now, and the next segments.
+    void tile_lists(Species& S_, const char* name) {
+        launch(name, k_tile_lists, cdiv(g.ntiles, TILES_PER_LIST_BLOCK), LIST_THREADS, 0, g, (const uint32_t*)S_.dtab.p,
+               S_.tile_list.p, S_.seg_loc.p, S_.seg_blk.p, S_.scal.p);
+    }
+
+    // Every particle into its own tile's segment, injected ones included,
+    // without pushing anything.
+    void merge(Species& S_) {
         if (S_.pushed) throw StateError("injected particles pending between propagate and wait_particle_sends");
         PushParams pp{};
         pp.still = 1;
-        pp.live = S_.live_src.p;
-        prepare_push_fields();
-        launch("sort_still", k_push_move<Real>, tile_grid(), PM_THREADS, push_move_lds_bytes<Real>(g), g, pp,
-               (const uint32_t*)pf_tile.p, S_.A(), S_.Dst(), (const uint32_t*)S_.sub.p, S_.appendix(), S_.cnt_tile.p,
-               (const uint32_t*)S_.sub_new.p, S_.pcount.p, kbits, 0, (uint32_t)S_.cap);
-        S_.pp = pp;
-        S_.pushed = true;
-        finish_sort(S_, "sort_still");
+        push(S_, pp, "sort_still");
+        swap_in(S_, "sort_still");
+        S_.lists = false;
+    }
+
+    void flush_injected(Species& S_) {
+        if (S_.inj_pending) merge(S_);
+    }
+
+    void swap_in(Species& S_, const char* name) {
+        tile_lists(S_, name);
+        S_.swap_stores();
+        S_.pushed = false;
+        S_.inj_pending = false;
+        S_.lists = true;
+        S_.compact = false;
+    }
+
+    void look_at_fill(Species& S_) {
+        uint32_t sc[SC_N];
+        launch("tile_fill", k_tile_fill, 1, FILL_THREADS, 0, g, (const uint32_t*)S_.tile_list.p, S_.scal.p);
+        RH_HIP(hipMemcpyAsync(sc, S_.scal.p, sizeof(sc), hipMemcpyDeviceToHost, stream));
+        RH_HIP(hipStreamSynchronize(stream));
+        std::copy(sc + SC_FILL, sc + SC_N, S_.tile_fill.begin());
+        S_.np_est = S_.fill_np = (double)sc[SC_NP];
+    }
+
+    uint32_t scalar(Species& S_, int id) {
+        uint32_t v = 0;
+        RH_HIP(hipMemcpyAsync(&v, S_.scal.p + id, sizeof(v), hipMemcpyDeviceToHost, stream));
+        RH_HIP(hipStreamSynchronize(stream));
+        return v;
     }
 
     void scan(const uint32_t* in, uint32_t n, uint32_t* out, std::vector<DevBuf<uint32_t>>& lv, size_t level) {
@@ -813,22 +1020,8 @@ public:
         SpeciesScope species_scope(timing_species, s);
         Species& S_ = S(s);
         if (!S_.pushed) throw StateError("wait_particle_sends without a preceding propagate");
-        finish_sort(S_, "move");
-    }
-
-    void finish_sort(Species& S_, const char* move_name) {
-        // totals and in-subcell offsets in one pass, then the scan of the totals
-        launch("sort_slots", k_slot_offsets,
-               N_XCD * cdiv(cdiv((uint32_t)g.ntiles * (uint32_t)g.tc, (uint32_t)SLOT_THREADS), (uint32_t)N_XCD),
-               SLOT_THREADS, 0, g, S_.cnt_tile.p, (const uint8_t*)S_.live_src.p, S_.sub_new.p, dcount.p);
-        scan(S_.sub_new.p, g.nkeys, S_.sub_new.p, S_.scan_lv, 0);
-        launch(move_name, k_push_move<Real>, tile_grid(), PM_THREADS, move_lds_bytes(&S_), g, S_.pp,
-               (const uint32_t*)pf_tile.p,
-               S_.A(), S_.Dst(), (const uint32_t*)S_.sub.p, S_.appendix(), S_.cnt_tile.p,
-               (const uint32_t*)S_.sub_new.p, S_.pcount.p, kbits, 1, (uint32_t)S_.cap);
-        S_.swap_stores();
-        S_.pushed = false;
-        S_.inj_pending = false;
+        // the push has written every particle where its new tile finds it
+        swap_in(S_, "sort_slots");
     }
 
     void clear_accumulation() override {
@@ -847,9 +1040,18 @@ public:
         // subcell the one-lane path is faster, at 16 three times slower)
         const uint32_t dense_min = 10u * (uint32_t)NS;
         launch("deposit", k_deposit<Real>, tile_grid(), NS, deposit_lds_bytes<Real>(g), g, S_.A(),
-               (const uint32_t*)S_.sub.p, (const uint16_t*)dep_list.p, (const uint8_t*)dep_count.p,
+               (const uint32_t*)S_.tab.p, (const uint32_t*)S_.tile_list.p, (const uint16_t*)dep_list.p, (const uint8_t*)dep_count.p,
                (const uint16_t*)dep_tlist.p, (const uint8_t*)dep_tcount.p, S_.partial.p, dense_min);
         S_.deposited = true;
+    }
+
+    // A cell has at most two candidate tiles per axis: tiles (also the last,
+    // partial one) of at least two cells, and no wrap onto the same tile.
+    bool fold_two_per_axis() const {
+        const int n[3] = {g.nx, g.ny, g.nz}, lt[3] = {g.ltx, g.lty, g.ltz}, nt[3] = {g.ntx, g.nty, g.ntz};
+        for (int d = 0; d < 3; ++d)
+            if (lt[d] == 0 || tile_width(n[d], lt[d], nt[d] - 1) < 2 || (g.per[d] && nt[d] < 3)) return false;
+        return true;
     }
 
     void add_remote_updates() override {
@@ -862,7 +1064,8 @@ public:
             src.wq[src.n] = s_->d.w * s_->d.q;
             src.n++;
         }
-        launch("fold", k_fold<Real>, cell_grid(), cell_block(), 0, g, src, 1.0 / (g.dx * g.dx * g.dx), P.min_rho,
+        auto fold = fold_two_per_axis() ? k_fold<Real, true> : k_fold<Real, false>;
+        launch("fold", fold, cell_grid(), cell_block(), 0, g, src, 1.0 / (g.dx * g.dx * g.dx), P.min_rho,
                fld[RH_CELL_RHOQ].p, ji.x, ji.y, ji.z, dcount.p);
         if (ave_on)
             for (auto& s_ : sp)
@@ -974,7 +1177,7 @@ public:
         if (S_.pushed) throw StateError("boundary conditions between propagate and wait_particle_sends");
         flush_injected(S_);
         launch("boundary", k_boundary<Real>, cdiv(n_bc, BC_CELLS_PER_BLOCK), 256, 0, g, (const int*)bc_cells.p, n_bc,
-               (const uint32_t*)S_.sub.p, S_.A(), S_.d.R2_obstacle, S_.bc_acc.p);
+               (const int*)bc_beg.p, (const CellRange*)bc_range.p, tables(S_), S_.A(), S_.d.R2_obstacle, S_.bc_acc.p);
     }
 
     void neumann_cell(int id, int dim) {
@@ -1139,14 +1342,9 @@ public:
             propagate_B_impl(it == n - 1);
         }
         check_overflow();
-        // each species' particle count (the sorted store's end; the stream has
-        // finished, check_overflow waited for it), for the next call's choice
-        // of the move's occupancy
+        // for the next call's choice of the push's workgroups
         for (auto& s_ : sp) {
-            uint32_t np = 0;
-            RH_HIP(hipMemcpyAsync(&np, s_->sub.p + g.nkeys, sizeof(np), hipMemcpyDeviceToHost, stream));
-            RH_HIP(hipStreamSynchronize(stream));
-            s_->dense = (double)np >= 4.0 * (double)g.nc;
+            look_at_fill(*s_);
         }
     }
 
@@ -1333,6 +1531,23 @@ public:
             for (size_t q = 0; q <= hc.size(); ++q) off[q] = (uint32_t)(q * (size_t)slots);
             RH_HIP(hipMemcpyAsync(S_.inj_off.p, off.data(), off.size() * sizeof(uint32_t), hipMemcpyHostToDevice, stream));
         }
+        if (ip.kind == INJ_SOLAR_WIND) {
+            ensure_appendix(S_, hc.size() * (size_t)slots);
+        } else if (ip.kind == INJ_EXOSPHERE) {
+            // a step's trial particles: sum(rate) and the deviation of one
+            // Bernoulli draw per cell; twelve of those are never exceeded
+            // (below 1e-30), and no cell draws more than ceil(rate)
+            double mean = 0, var = 0, most = 0;
+            for (double r : hr) {
+                const double f = r - std::floor(r);
+                mean += r;
+                var += f * (1.0 - f);
+                most += std::ceil(r);
+            }
+            const double places = std::min(most, std::ceil(mean + 12.0 * std::sqrt(var)) + 64.0);
+            if (places >= 2147483647.0) throw ArgError("injection rate too large for the appendix");
+            ensure_appendix(S_, (size_t)places);
+        }
         // inject energy accumulators: per block of places (fixed places), per listed cell (count and fill)
         S_.inj_acc.alloc(slots > 0 ? std::max<size_t>(cdiv(hc.size() * (size_t)slots, 256), 1) : nl);
         fill(S_.inj_acc.p, 0.0, S_.inj_acc.n);
@@ -1351,15 +1566,24 @@ public:
         if (S_.inj.kind == INJ_NONE || S_.inj_ncell == 0 || tstep <= 0) return;
         if (S_.inj.kind == INJ_UNIFORM && tstep != 1) return;  // src/particle_injector.cpp:181
         flush_injected(S_);  // a second injection before the next push
+        // the uniform fill goes to the store's end (its places would need a
+        // store of their own): the segments without empty places first (a
+        // merge drops the removed particles, a second one their places)
+        if (S_.inj.kind == INJ_UNIFORM && !S_.compact) {
+            merge(S_);
+            merge(S_);
+            S_.compact = true;
+        }
         InjParams ip = S_.inj;
         ip.step = (uint32_t)tstep;
         if (ip.kind == INJ_SOLAR_WIND || ip.kind == INJ_UNIFORM) {
             if (S_.inj_slots > 0)
                 launch("inject_slots", k_inject_slots<Real>, cdiv((size_t)S_.inj_ncell * S_.inj_slots, 256), 256, 0, g,
                        ip, S_.inj_ncell, S_.inj_slots, (const int*)S_.inj_cells.p,
-                       (const uint32_t*)(S_.sub.p + g.nkeys), S_.A(), (uint32_t)S_.cap, S_.inj_total.p, dcount.p,
-                       S_.inj_acc.p);
+                       (const uint32_t*)(S_.scal.p + SC_NP), ip.kind == INJ_UNIFORM ? 1 : 0, S_.A(), (uint32_t)S_.cap,
+                       S_.inj_total.p, dcount.p, S_.inj_acc.p);
             S_.inj_pending = S_.inj_slots > 0;
+            S_.np_est += (double)S_.inj_ncell * S_.inj.rate;
             return;
         }
         const unsigned nb = cdiv(S_.inj_ncell, 256);
@@ -1368,8 +1592,8 @@ public:
                rate, S_.inj_off.p);
         scan(S_.inj_off.p, (uint32_t)S_.inj_ncell, S_.inj_off.p, scan_lv, 0);
         launch("inject_fill", k_inject_fill<Real>, nb, 256, 0, g, ip, S_.inj_ncell, (const int*)S_.inj_cells.p, rate,
-               (const uint32_t*)S_.inj_off.p, (const uint32_t*)(S_.sub.p + g.nkeys), S_.A(), (uint32_t)S_.cap,
-               S_.inj_total.p, dcount.p, S_.inj_acc.p);
+               (const uint32_t*)S_.inj_off.p, (const uint32_t*)(S_.scal.p + SC_NP), S_.A(), (uint32_t)S_.cap,
+               (uint32_t)S_.app_cap, S_.inj_total.p, dcount.p, S_.inj_acc.p);
         S_.inj_pending = true;
     }
 
@@ -1453,7 +1677,7 @@ public:
             Species& S_ = *sp[s];
             double d[DIAG_Q];
             diag_raw((int)s, d);
-            launch("log_mass", k_cell_mass<Real>, cdiv(g.nc, 256), 256, 0, g, (const uint32_t*)S_.sub.p, S_.A(),
+            launch("log_mass", k_cell_mass<Real>, cdiv(g.nc, 256), 256, 0, g, tables(S_), S_.A(),
                    S_.d.m * S_.d.w, log_rhoM.p, s == 0 ? 1 : 0);
             double bc[4], v2inj = 0.0;
             sum_cols(S_.bc_acc.p, (size_t)n_bc, 4, bc);
@@ -1686,7 +1910,7 @@ public:
             // calcCellNPles (:355-373): macroparticles of all species per cell
             if (sp.empty()) fill(log_rhoM.p, 0.0, log_rhoM.n);
             for (size_t s = 0; s < sp.size(); ++s)
-                launch("vlsv_count", k_cell_mass<Real>, cdiv(g.nc, 256), 256, 0, g, (const uint32_t*)sp[s]->sub.p,
+                launch("vlsv_count", k_cell_mass<Real>, cdiv(g.nc, 256), 256, 0, g, tables(*sp[s]),
                        sp[s]->A(), 1.0, log_rhoM.p, s == 0 ? 1 : 0);
             h.assign(nc, 0.0);
             RH_HIP(hipMemcpyAsync(h.data(), log_rhoM.p, nc * sizeof(double), hipMemcpyDeviceToHost, stream));
@@ -1711,7 +1935,7 @@ public:
                 for (int pass = 0; pass < 2; ++pass)
                     for (size_t q = 0; q < members.size(); ++q) {
                         Species& S_ = *sp[members[q]];
-                        launch("vlsv_bulk", k_cell_bulk<Real>, cdiv(g.nc, 256), 256, 0, g, (const uint32_t*)S_.sub.p,
+                        launch("vlsv_bulk", k_cell_bulk<Real>, cdiv(g.nc, 256), 256, 0, g, tables(S_),
                                S_.A(), S_.d.w, pass, acc.p, tacc.p, q == 0 ? 1 : 0);
                     }
                 std::vector<double> ha(nc * 4), ht(nc);
@@ -1804,8 +2028,8 @@ public:
         Species& S_ = S(s);
         if (S_.pushed) throw StateError("diagnostics between propagate and wait_particle_sends");
         const uint32_t* extra = S_.inj_pending ? (const uint32_t*)(S_.inj_off.p + S_.inj_ncell) : nullptr;
-        launch("diag", k_diag<Real>, DIAG_BLOCKS, 256, 0, S_.A(), (const uint32_t*)(S_.sub.p + g.nkeys), extra,
-               (uint32_t)S_.cap, diag_partial.p);
+        launch("diag", k_diag<Real>, DIAG_BLOCKS, 256, 0, S_.A(), (const uint32_t*)S_.scal.p, extra,
+               S_.appendix().places, S_.inj.kind == INJ_UNIFORM ? 1 : 0, (uint32_t)S_.cap, diag_partial.p);
         std::vector<double> h(DIAG_BLOCKS * DIAG_Q);
         RH_HIP(hipMemcpyAsync(h.data(), diag_partial.p, sizeof(double) * h.size(), hipMemcpyDeviceToHost, stream));
         RH_HIP(hipStreamSynchronize(stream));

@@ -42,12 +42,19 @@ struct Geom {
     double x0, y0, z0;
     int tx, ty, tz, tc;        // tile shape (powers of two), cells per tile
     int ltx, lty, ltz;         // log2 of the tile shape
-    int ntx, nty, ntz, ntiles; // tiles per axis
+    int ntx, nty, ntz, ntiles; // tiles per axis (the last one of an axis may be partial)
     int ex, ey, ez, next;      // extended region shape and cell count
     int extk;                  // next * 8 subcell slots in the extended region
     uint32_t nkeys;            // ntiles * tc * 8
+    int nslot, kt;             // subcell and halo-cell slots of a tile; entries per tile of the slot tables
     int xpx, xpy, xpz, xchunk; // XCD bricks: parts per axis (product 8), most tiles in one brick
 };
+
+// slots of the tile shape: 8 subcells per cell of the tile, one per halo cell
+RH_HD void set_slots(Geom& g) {
+    g.nslot = 7 * g.tc + g.next;
+    g.kt = (g.nslot + 1 + 3) & ~3;
+}
 
 RH_HD void cell_ijk(const Geom& g, int n, int& i, int& j, int& k) {
     i = n % g.nx;
@@ -88,6 +95,12 @@ RH_HD bool has_neg(int i, int per) { return per || i > 0; }
 // the cell is missing a +x, +y or +z neighbour (node and face kernels skip it)
 RH_HD bool upper_missing(const Geom& g, int i, int j, int k) {
     return !has_pos(i, g.nx, g.per[0]) || !has_pos(j, g.ny, g.per[1]) || !has_pos(k, g.nz, g.per[2]);
+}
+
+// cells of tile b along an axis of n cells: the last tile ends with the grid
+RH_HD int tile_width(int n, int lt, int b) {
+    const int t = 1 << lt, left = n - (b << lt);
+    return left < t ? left : t;
 }
 
 RH_HD int tile_of(const Geom& g, int i, int j, int k) {

@@ -11,8 +11,9 @@
 //   sampleGaussian       :59-80 (polar method, second deviate kept per stream)
 //   sampleDerivGaussian  :97-114 (rejection from the unit Gaussian at the mode)
 //
-// New particles are written past the end of the sorted store in the order of
-// the listed cells.  The list is sorted by subcell key, so each tile's new
+// New particles are written to the species' appendix, past the store's
+// capacity (the uniform fill: past the store's end), in the order of the
+// listed cells.  The list is sorted by subcell key, so each tile's new
 // particles are one range; the next push/sort pass of the tile takes them
 // after the tile's own particles.  The solar wind gives every listed cell a
 // fixed number of places (at most ceil(rate) particles per step), filled in
@@ -165,8 +166,8 @@ __device__ __forceinline__ double store_particle(const InjParams& ip, PArrays<Re
 }
 
 // The new particles of listed cell n: their number (WRITE = false), or
-// their state written to A[at..] (WRITE = true; indices >= cap are not
-// written and set `overflow`).  Positions in cell units, velocities in m/s.
+// their state written to A[at..] (WRITE = true; at most `room` of them, more
+// set `overflow`).  Positions in cell units, velocities in m/s.
 //   solar wind (initParticleCrdVel{X,Y,Z}{Pos,Neg}, :464-535): on the wall
 //     face (local coordinate 0 on the +axis wall, 1 on the -axis wall),
 //     uniform across it, normal speed vth * sampleDerivGaussian(U/vth)
@@ -176,7 +177,7 @@ __device__ __forceinline__ double store_particle(const InjParams& ip, PArrays<Re
 //     per component.
 template <typename Real, bool WRITE>
 __device__ uint32_t inject_cell(const Geom& g, const InjParams& ip, int n, double rate, PArrays<Real> A,
-                                uint32_t at, uint32_t cap, uint8_t lc, bool& overflow, double& v2sum) {
+                                uint32_t at, uint32_t room, uint8_t lc, bool& overflow, double& v2sum) {
 #pragma clang fp contract(off)
     RngStream cs(ip.k0, ip.k1, (uint32_t)n, ip.step, 0xFFFFFFFFu);
     const int N = prob_round(rate, cs.uniform());
@@ -188,8 +189,7 @@ __device__ uint32_t inject_cell(const Geom& g, const InjParams& ip, int n, doubl
         double r[3], v[3];
         if (!gen_particle(g, ip, n, i, j, k, (uint32_t)m, WRITE, r, v)) continue;
         if (WRITE) {
-            const uint32_t p = at + q;
-            if (p < cap) v2sum += store_particle(ip, A, p, r, v, lc);
+            if (q < room) v2sum += store_particle(ip, A, at + q, r, v, lc);
             else overflow = true;
         }
         ++q;
@@ -197,8 +197,8 @@ __device__ uint32_t inject_cell(const Geom& g, const InjParams& ip, int n, doubl
     return q;
 }
 
-// Solar wind and uniform fill: every listed cell owns `slots` = ceil(rate) fixed places past
-// the store's end (cell c: slots c*slots ..), so no count and no scan are
+// Solar wind and uniform fill: every listed cell owns `slots` = ceil(rate) fixed places of
+// the appendix (cell c: slots c*slots ..), so no count and no scan are
 // needed; one thread per place writes particle m of its cell if m < the
 // cell's probRound draw, else marks the place removed (x = -1, skipped by
 // every later pass).  The step's total goes to *total; the block's sum of
@@ -206,7 +206,7 @@ __device__ uint32_t inject_cell(const Geom& g, const InjParams& ip, int n, doubl
 template <typename Real>
 __global__ __launch_bounds__(256) void k_inject_slots(Geom g, InjParams ip, int ncell, int slots,
                                                       const int* __restrict__ cells,
-                                                      const uint32_t* __restrict__ np_ptr, PArrays<Real> A,
+                                                      const uint32_t* __restrict__ np_ptr, int at_end, PArrays<Real> A,
                                                       uint32_t cap, unsigned long long* __restrict__ total,
                                                       unsigned long long* __restrict__ counters,
                                                       double* __restrict__ v2acc) {
@@ -218,8 +218,9 @@ __global__ __launch_bounds__(256) void k_inject_slots(Geom g, InjParams ip, int 
         const int n = cells[c];
         RngStream cs(ip.k0, ip.k1, (uint32_t)n, ip.step, 0xFFFFFFFFu);
         const int N = prob_round(ip.rate, cs.uniform());
-        const uint64_t p = (uint64_t)*np_ptr + (uint64_t)t;
-        if (p >= cap) {
+        const uint32_t np = *np_ptr;
+        const uint32_t p = (at_end ? np : cap) + (uint32_t)t;
+        if ((uint64_t)np + (uint64_t)t >= cap) {  // the store would be full
             overflow = m < N;
         } else if (m < N) {
             int i, j, k;
@@ -228,7 +229,7 @@ __global__ __launch_bounds__(256) void k_inject_slots(Geom g, InjParams ip, int 
                                          ((k & (g.tz - 1)) << (g.ltx + g.lty)));
             double r[3], v[3];
             gen_particle(g, ip, n, i, j, k, (uint32_t)m, true, r, v);
-            v2 = store_particle(ip, A, (uint32_t)p, r, v, lc);
+            v2 = store_particle(ip, A, p, r, v, lc);
             live = true;
         } else {
             A.x[p] = Real(-1);
@@ -258,15 +259,16 @@ __global__ __launch_bounds__(256) void k_inject_count(Geom g, InjParams ip, int 
     count[c] = inject_cell<Real, false>(g, ip, cells[c], rate ? rate[c] : ip.rate, none, 0, 0, 0, unused, unused_v2);
 }
 
-// The new particles of each listed cell at np + off[c] (np = the sorted
-// store's size); counts the step's total into *total (integer, so the sum is
+// The new particles of each listed cell at appendix place off[c] (room: the
+// places the store's capacity leaves beside its *np_ptr particles, at most
+// those of the appendix); counts the step's total into *total (integer, so the sum is
 // exact), overflows of the store into the sort's overflow counter, and adds
 // the cell's sum of v^2 to v2acc[c].
 template <typename Real>
 __global__ __launch_bounds__(256) void k_inject_fill(Geom g, InjParams ip, int ncell, const int* __restrict__ cells,
                                                      const double* __restrict__ rate, const uint32_t* __restrict__ off,
                                                      const uint32_t* __restrict__ np_ptr, PArrays<Real> A, uint32_t cap,
-                                                     unsigned long long* __restrict__ total,
+                                                     uint32_t places, unsigned long long* __restrict__ total,
                                                      unsigned long long* __restrict__ counters,
                                                      double* __restrict__ v2acc) {
     const int c = blockIdx.x * 256 + threadIdx.x;
@@ -277,10 +279,10 @@ __global__ __launch_bounds__(256) void k_inject_fill(Geom g, InjParams ip, int n
         cell_ijk(g, n, i, j, k);
         const uint8_t lc = (uint8_t)((i & (g.tx - 1)) + ((j & (g.ty - 1)) << g.ltx) +
                                      ((k & (g.tz - 1)) << (g.ltx + g.lty)));
-        const uint64_t at = (uint64_t)*np_ptr + off[c];
+        const uint32_t np = *np_ptr, room = min(cap > np ? cap - np : 0u, places);
         double v2 = 0.0;
-        inject_cell<Real, true>(g, ip, n, rate ? rate[c] : ip.rate, A, at > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)at,
-                                cap, lc, overflow, v2);
+        inject_cell<Real, true>(g, ip, n, rate ? rate[c] : ip.rate, A, cap + off[c], room > off[c] ? room - off[c] : 0u,
+                                lc, overflow, v2);
         v2acc[c] += v2;
         if (c == 0) atomicAdd(total, (unsigned long long)off[ncell]);
     }

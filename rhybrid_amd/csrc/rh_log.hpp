@@ -30,16 +30,16 @@ constexpr double LOG_KB = 1.3806505e-23;
 // rhoM[n] (+)= m*w * (live particles of the species in cell n); removed
 // particles (x < 0) are not counted.
 template <typename Real>
-__global__ __launch_bounds__(256) void k_cell_mass(Geom g, const uint32_t* __restrict__ sub, PArrays<Real> A, double mw,
+__global__ __launch_bounds__(256) void k_cell_mass(Geom g, TileTables tt, PArrays<Real> A, double mw,
                                                    double* __restrict__ rhoM, int first) {
     const int n = blockIdx.x * 256 + threadIdx.x;
     if (n >= g.nc) return;
     int i, j, k;
     cell_ijk(g, n, i, j, k);
-    const uint32_t kc = cell_key(g, i, j, k);
-    const uint32_t p0 = sub[(size_t)kc * 8], p1 = sub[(size_t)kc * 8 + 8];
     uint32_t c = 0;
-    for (uint32_t p = p0; p < p1; ++p) c += A.x[p] >= Real(0);
+    cell_ranges(g, tt, i, j, k, [&](uint32_t p0, uint32_t p1) {
+        for (uint32_t p = p0; p < p1; ++p) c += A.x[p] >= Real(0);
+    });
     rhoM[n] = (first ? 0.0 : rhoM[n]) + mw * (double)c;
 }
 
@@ -50,22 +50,22 @@ __global__ __launch_bounds__(256) void k_cell_mass(Geom g, const uint32_t* __res
 // sum w |v - U|^2 with U = the population's mean velocity in the cell (0
 // where the cell is empty).  Removed particles (x < 0) are skipped.
 template <typename Real>
-__global__ __launch_bounds__(256) void k_cell_bulk(Geom g, const uint32_t* __restrict__ sub, PArrays<Real> A, double w,
+__global__ __launch_bounds__(256) void k_cell_bulk(Geom g, TileTables tt, PArrays<Real> A, double w,
                                                    int pass, double* __restrict__ acc, double* __restrict__ tacc,
                                                    int first) {
     const int n = blockIdx.x * 256 + threadIdx.x;
     if (n >= g.nc) return;
     int i, j, k;
     cell_ijk(g, n, i, j, k);
-    const uint32_t kc = cell_key(g, i, j, k);
-    const uint32_t p0 = sub[(size_t)kc * 8], p1 = sub[(size_t)kc * 8 + 8];
     if (pass == 0) {
         double s0 = 0, sx = 0, sy = 0, sz = 0;
-        for (uint32_t p = p0; p < p1; ++p) {
-            if (A.x[p] < Real(0)) continue;
-            s0 += w;
-            sx += (double)A.vx[p] * w; sy += (double)A.vy[p] * w; sz += (double)A.vz[p] * w;
-        }
+        cell_ranges(g, tt, i, j, k, [&](uint32_t p0, uint32_t p1) {
+            for (uint32_t p = p0; p < p1; ++p) {
+                if (A.x[p] < Real(0)) continue;
+                s0 += w;
+                sx += (double)A.vx[p] * w; sy += (double)A.vy[p] * w; sz += (double)A.vz[p] * w;
+            }
+        });
         double* a = acc + (size_t)n * 4;
         if (first) { a[0] = s0; a[1] = sx; a[2] = sy; a[3] = sz; }
         else { a[0] += s0; a[1] += sx; a[2] += sy; a[3] += sz; }
@@ -74,11 +74,13 @@ __global__ __launch_bounds__(256) void k_cell_bulk(Geom g, const uint32_t* __res
         const double ux = a[0] > 0.0 ? a[1] / a[0] : 0.0, uy = a[0] > 0.0 ? a[2] / a[0] : 0.0,
                      uz = a[0] > 0.0 ? a[3] / a[0] : 0.0;
         double t = 0;
-        for (uint32_t p = p0; p < p1; ++p) {
-            if (A.x[p] < Real(0)) continue;
-            const double dx = (double)A.vx[p] - ux, dy = (double)A.vy[p] - uy, dz = (double)A.vz[p] - uz;
-            t += w * (dx * dx + dy * dy + dz * dz);
-        }
+        cell_ranges(g, tt, i, j, k, [&](uint32_t p0, uint32_t p1) {
+            for (uint32_t p = p0; p < p1; ++p) {
+                if (A.x[p] < Real(0)) continue;
+                const double dx = (double)A.vx[p] - ux, dy = (double)A.vy[p] - uy, dz = (double)A.vz[p] - uz;
+                t += w * (dx * dx + dy * dy + dz * dz);
+            }
+        });
         tacc[n] = first ? t : tacc[n] + t;
     }
 }

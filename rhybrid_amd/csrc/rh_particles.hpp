@@ -1,16 +1,17 @@
 // rh_particles.hpp -- device kernels of the particle half of the step:
-// Boris-Buneman push, the cell migration as a deterministic counting sort by
-// subcell, the cloud-in-cell deposit with fixed-order reductions, the FP64
+// Boris-Buneman push with the cell migration as a deterministic counting sort
+// by subcell inside each tile, the cloud-in-cell deposit with fixed-order reductions, the FP64
 // cross-tile ghost fold, particle boundary conditions and FP64 diagnostics.
 //
 // Storage (per species, structure of arrays, Real = float or double):
 //   x,y,z    cell-local position in units of dx, in [0,1); x = -1 marks a
-//            particle removed by the boundary conditions
+//            particle removed by the boundary conditions, or a place of a
+//            segment that holds none
 //   vx,vy,vz velocity in m/s
 //   lc       the particle's cell inside its tile (implied by the sort order,
 //            kept so that kernels need not search the subcell ranges)
-// sorted by subcell key (rh_geom.hpp); sub[k] .. sub[k+1] is the range of
-// subcell key k.
+// in one segment per tile, sorted inside it by slot; TileTables says where
+// each slot's particles are.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -18,6 +19,11 @@
 #include "rh_geom.hpp"
 
 namespace rh {
+
+template <typename Real>
+struct alignas(4 * sizeof(Real)) Real4 { Real v[4]; };
+template <typename Real>
+struct alignas(2 * sizeof(Real)) Real2 { Real v[2]; };
 
 template <typename Real>
 struct PArrays {
@@ -79,42 +85,30 @@ template <typename Real> __device__ __forceinline__ Real below_one();
 template <> __device__ __forceinline__ float below_one<float>() { return 0x1.fffffep-1f; }
 template <> __device__ __forceinline__ double below_one<double>() { return 0x1.fffffffffffffp-1; }
 
-// The push and the cell migration, one workgroup of four waves per old tile,
-// run twice with the same compiled body so that both passes compute bit-for-
-// bit the same pushed state, destination slot and rank:
-//   pass 0: BorisBuneman::propagate (src/particle_propagator_boris_buneman.h:
-//           64-194, fields by face2r/cell2r, src/hybrid_propagator.cpp:
-//           1740-1891), the move in FP64, and the destination slot in the
-//           tile's extended region; counts particles per slot;
-//   pass 1: the same, then writes each particle to (destination subcell's
-//           start + the slot's offset inside it + rank).
-// The tile's particles are taken 256 at a time.  Pass 0 counts slots with
-// integer LDS atomics.  In pass 1 the rank of a particle is its position among
-// the tile's particles with the same slot in memory order (the migration is a
-// stable counting sort): each wave ranks its lanes with ballots and publishes
-// its per-slot group sizes; a lane's destination is the slot's running
-// counter (started, once per tile, at the slot's first destination index)
-// plus its rank in the wave plus the group sizes of the earlier waves.
-// The tile's field block is copied to LDS; removed particles carry x < 0.
-constexpr int PM_THREADS = 256;
-constexpr int PM_WAVES = PM_THREADS / 64;
-
-RH_HD size_t pm_align8(size_t b) { return (b + 7) & ~size_t(7); }
+// The push and the cell migration, one workgroup per tile and one pass over
+// the particles (BorisBuneman::propagate, src/particle_propagator_boris_
+// buneman.h:64-194, fields by face2r/cell2r, src/hybrid_propagator.cpp:
+// 1740-1891, the move in FP64).  A tile owns one contiguous segment of the
+// store, as long as the particles it held before the push, and writes the
+// pushed particles into that segment of the other store in slot order: first
+// those that stay, by subcell, then those that leave, by the halo cell they
+// leave to.  A tile's particles are thus its own staying ones and, in up to
+// 26 neighbours' segments, the ones that left towards it; the next push, the
+// deposit and the boundary conditions read them there.  No tile needs
+// another's counts before it writes, so the particles are read once and
+// written once per step (a counting sort over the whole store needs a first
+// pass that only counts, and writes into its neighbours' cache lines).
+RH_HD size_t pm_align16(size_t b) { return (b + 15) & ~size_t(15); }
 
 // A tile's push fields as one contiguous block (32-bit words): faceB of the
 // (t+1)^3 cells -1..t-1 (halo on the low side), cellUe and cellEp of the
 // tile's cells, and the cells' neighbourhood masks.  Written once per field
-// update by k_push_fields and copied to LDS by both passes of k_push_move.
+// update by k_push_fields and copied to LDS by k_push_sort.
 template <typename Real>
 RH_HD size_t push_field_words(const Geom& g) {
     const size_t nh = (size_t)(g.tx + 1) * (g.ty + 1) * (g.tz + 1);
     const size_t words = (sizeof(Real) * (3 * nh + 6 * (size_t)g.tc) + 4 * (size_t)g.tc) / 4;
     return (words + 3) & ~size_t(3);  // 16-byte blocks keep every tile's block aligned
-}
-
-template <typename Real>
-RH_HD size_t push_move_lds_bytes(const Geom& g) {
-    return pm_align8(4 * (size_t)g.extk + (size_t)PM_WAVES * g.extk) + 4 * push_field_words<Real>(g);
 }
 
 // Neighbourhood mask of a cell: bit (a+1) + 3(b+1) + 9(c+1) is set when the
@@ -169,7 +163,9 @@ __device__ __forceinline__ void push_fields_store(const Geom& g, int i, int j, i
     // halo copies: the cell is local coordinate -1 of the tile above along
     // each axis where it is the tile's last cell (nowrap: the caller knows
     // that those tiles lie inside the grid without a wrap)
-    const int ux = li == g.tx - 1, uy = lj == g.ty - 1, uz = lk == g.tz - 1;
+    // (the grid's last cell ends its tile even where the tile is partial)
+    const int ux = li == g.tx - 1 || i == g.nx - 1, uy = lj == g.ty - 1 || j == g.ny - 1,
+              uz = lk == g.tz - 1 || k == g.nz - 1;
     for (int c = 0; c <= uz; ++c)
         for (int b = 0; b <= uy; ++b)
             for (int a = 0; a <= ux; ++a) {
@@ -203,350 +199,775 @@ __global__ __launch_bounds__(256) void k_push_fields(Geom g, PushFields<Real> f,
 
 // Injected particles waiting for their first push: per tile, the range of
 // listed injection cells (cbeg, ntiles + 1 entries, null when none wait) and
-// per listed cell the offset of its particles past the sorted store's end.
+// per listed cell the offset of its particles in the appendix, which has
+// `places` places from store index `cap`, or lies at the store's end for the
+// uniform fill (at_end).  slots > 0: fixed places per listed cell, whose
+// offsets need no table.
 struct InjAppendix {
     const uint32_t* cbeg;
     const uint32_t* off;
+    uint32_t places;
+    uint32_t slots;
+    int at_end;
 };
 
+__device__ __forceinline__ uint32_t appendix_offset(const InjAppendix& app, uint32_t cell) {
+    return app.slots ? cell * app.slots : app.off[cell];
+}
+
+// A species' scalars on the device.
+enum DevScalar {
+    SC_NP = 0,   // particles in the segments (removed ones included until the next push)
+    SC_END,      // store indices in use by the segments
+    SC_TICKET,   // blocks of k_tile_lists that are done
+    SC_FILL,     // k_tile_fill's FILL_CLASSES counts
+    SC_N = SC_FILL + 128
+};
+
+// Per tile DIR_WORDS store indices: where its halo slots of direction d begin
+// (entry d; entry 27: where they end), and where its own particles begin and
+// end.  Written by the push for every tile, also an empty one.
+constexpr int DIR_WORDS = 32, DIR_OWN = 28;
+// Per tile LIST_WORDS: where its particles are, as one sequence.  Its
+// arrivals from offset j (j%3-1, (j/3)%3-1, j/9-1) are arrivals LIST_PREF + j
+// to LIST_PREF + j + 1 of the sequence, arrival v at store index
+// (LIST_START + j) + v; LIST_OWN: its own particles' first index and count.
+constexpr int LIST_WORDS = 64, LIST_START = 0, LIST_PREF = 27, LIST_OWN = 55;
+
+// Where a tile's particles are (written by the push, read by everything
+// after it): per tile g.kt store indices, tab[T*kt + s] .. tab[T*kt + s + 1]
+// the range of slot s.  Slots 0 .. 8*tc-1 are the tile's subcells; then come
+// the halo cells of the tile's extended region, grouped by the direction
+// (a+1) + 3(b+1) + 9(c+1) they lie in; dir[d] is the first slot of direction
+// d, dir[27] the end.  slot[e] is the slot of extended cell e outside the
+// tile.  The tables of a tile that held nothing (live 0) are not written.
+// lists: particles may wait in halo slots (not after an upload or a merge).
+struct TileTables {
+    const uint32_t* tab;
+    const uint8_t* live;
+    const uint16_t* dir;
+    const uint16_t* slot;
+    int lists;
+};
+
+// Slots of a tile shape: dir (28 entries) and slot (g.next entries).
+inline void tile_slots(const Geom& g, uint16_t* dir, uint16_t* slot) {
+    int s = 8 * g.tc;
+    for (int d = 0; d < 27; ++d) {
+        dir[d] = (uint16_t)s;
+        if (d == 13) continue;
+        const int a[3] = {d % 3 - 1, (d / 3) % 3 - 1, d / 9 - 1}, t[3] = {g.tx, g.ty, g.tz};
+        int lo[3], hi[3];
+        for (int q = 0; q < 3; ++q) {
+            lo[q] = a[q] < 0 ? 0 : (a[q] > 0 ? t[q] + 1 : 1);
+            hi[q] = a[q] == 0 ? t[q] : lo[q];
+        }
+        for (int z = lo[2]; z <= hi[2]; ++z)
+            for (int y = lo[1]; y <= hi[1]; ++y)
+                for (int x = lo[0]; x <= hi[0]; ++x) slot[x + g.ex * (y + g.ey * z)] = (uint16_t)s++;
+    }
+    dir[27] = (uint16_t)s;
+    for (int e = 0; e < g.next; ++e) {
+        const int x = e % g.ex, y = (e / g.ex) % g.ey, z = e / (g.ex * g.ey);
+        if (x >= 1 && x <= g.tx && y >= 1 && y <= g.ty && z >= 1 && z <= g.tz) slot[e] = 0;  // the tile's own
+    }
+}
+
+// The source tile of the arrivals of tile (bx,by,bz) from offset (a,b,c);
+// -1 where there is none.
+__device__ __forceinline__ int neighbour_tile(const Geom& g, int bx, int by, int bz, int a, int b, int c) {
+    int x = bx + a, y = by + b, z = bz + c;
+    if (x < 0 || x >= g.ntx) { if (!g.per[0]) return -1; x += x < 0 ? g.ntx : -g.ntx; }
+    if (y < 0 || y >= g.nty) { if (!g.per[1]) return -1; y += y < 0 ? g.nty : -g.nty; }
+    if (z < 0 || z >= g.ntz) { if (!g.per[2]) return -1; z += z < 0 ? g.ntz : -g.ntz; }
+    return x + g.ntx * (y + g.nty * z);
+}
+
+// Store index of a tile's arrival v: in the last list that starts at or before v.
+__device__ __forceinline__ uint32_t arrival_index(const uint32_t* lists, uint32_t v) {
+    int j = 0;
+#pragma unroll
+    for (int s = 16; s > 0; s >>= 1)
+        if (j + s <= 26 && lists[LIST_PREF + j + s] <= v) j += s;
+    return lists[LIST_START + j] + v;
+}
+
+// f(first, end) for every store range that holds particles of cell (i,j,k):
+// its own subcells', then the halo cells of neighbouring tiles that it is.
+template <typename F>
+__device__ __forceinline__ void cell_ranges(const Geom& g, const TileTables& t, int i, int j, int k, F&& f) {
+    const int c[3] = {i, j, k}, n[3] = {g.nx, g.ny, g.nz}, lt[3] = {g.ltx, g.lty, g.ltz}, nt[3] = {g.ntx, g.nty, g.ntz};
+    int b[3], l[3], lo[3], hi[3];  // tile, local coordinate, whether a lower / upper neighbour's halo holds the cell
+    for (int d = 0; d < 3; ++d) {
+        b[d] = c[d] >> lt[d];
+        l[d] = c[d] - (b[d] << lt[d]);
+        lo[d] = l[d] == 0 && (b[d] > 0 || g.per[d]);
+        hi[d] = l[d] == tile_width(n[d], lt[d], b[d]) - 1 && (b[d] < nt[d] - 1 || g.per[d]);
+    }
+    const int T = b[0] + g.ntx * (b[1] + g.nty * b[2]);
+    if (t.live[T]) {
+        const uint32_t* tab = t.tab + (size_t)T * g.kt + 8 * (l[0] + (l[1] << g.ltx) + (l[2] << (g.ltx + g.lty)));
+        f(tab[0], tab[8]);
+    }
+    if (!t.lists) return;
+    for (int z = -lo[2]; z <= hi[2]; ++z)
+        for (int y = -lo[1]; y <= hi[1]; ++y)
+            for (int x = -lo[0]; x <= hi[0]; ++x) {
+                if (!x && !y && !z) continue;
+                const int S = neighbour_tile(g, b[0], b[1], b[2], x, y, z);
+                if (S < 0 || !t.live[S]) continue;
+                const int ex = x < 0 ? g.tx + 1 : (x > 0 ? 0 : l[0] + 1), ey = y < 0 ? g.ty + 1 : (y > 0 ? 0 : l[1] + 1),
+                          ez = z < 0 ? g.tz + 1 : (z > 0 ? 0 : l[2] + 1);
+                const uint32_t* tab = t.tab + (size_t)S * g.kt + t.slot[ex + g.ex * (ey + g.ey * ez)];
+                f(tab[0], tab[1]);
+            }
+}
+
+// inclusive sum over the lanes of a wave: DPP row shifts, then row broadcasts
+__device__ __forceinline__ uint32_t wave_inclusive(uint32_t v) {
+    int x = (int)v;
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr 1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr 2
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr 4
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // lane 15 of each row to the next one
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // lane 31 to the upper half
+    return (uint32_t)x;
+}
+
+// a value that is the same in every lane, in a scalar register
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+// exclusive prefix of v over the block (at most 16 waves; wsum: 16 words);
+// total in every thread
+template <int NT>
+__device__ __forceinline__ uint32_t block_prefix(uint32_t v, uint32_t* wsum, uint32_t& total) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint32_t inc = wave_inclusive(v);
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    const uint32_t sums = wave_inclusive(lane < NT / 64 ? wsum[lane] : 0u);
+    total = (uint32_t)__builtin_amdgcn_readlane((int)sums, NT / 64 - 1);
+    const int wu = __builtin_amdgcn_readfirstlane(w);
+    const uint32_t base = wu ? (uint32_t)__builtin_amdgcn_readlane((int)sums, wu - 1) : 0u;
+    return base + inc - v;
+}
+
+// After a push: every tile's lists (half a wave per tile, one lane per
+// neighbour), and its segment in the store the next push writes, as many
+// places as it has particles: loc[T] + blk[T / TILES_PER_LIST_BLOCK], plus the
+// injected particles of the tiles before it.  The last block to finish scans
+// the block sums, so one launch does both (18,432 tiles of the 128x96x96 box
+// are 576 sums; a second launch would cost more than the scan).
+constexpr int LIST_THREADS = 1024;
+constexpr int TILES_PER_LIST_BLOCK = LIST_THREADS / 32;
+
+__global__ __launch_bounds__(LIST_THREADS) void k_tile_lists(Geom g, const uint32_t* __restrict__ dtab,
+                                                             uint32_t* __restrict__ lists, uint32_t* __restrict__ loc,
+                                                             uint32_t* __restrict__ blk, uint32_t* __restrict__ scal) {
+    __shared__ uint32_t wsum[LIST_THREADS / 64], cnt[TILES_PER_LIST_BLOCK];
+    __shared__ uint32_t last;
+    const int tid = threadIdx.x, lane = tid & 31;
+    const int T = blockIdx.x * TILES_PER_LIST_BLOCK + (tid >> 5);
+    uint32_t s0 = 0, n = 0;
+    if (T < g.ntiles && lane < 27) {
+        int bx, by, bz;
+        tile_coords(g, T, bx, by, bz);
+        const int S = neighbour_tile(g, bx, by, bz, lane % 3 - 1, (lane / 3) % 3 - 1, lane / 9 - 1);
+        if (S >= 0) {
+            // the direction from the neighbour to the tile; the tile itself: its own particles
+            const uint32_t* d = dtab + (size_t)S * DIR_WORDS + (lane == 13 ? DIR_OWN : 26 - lane);
+            s0 = d[0];
+            n = d[1] - s0;
+        }
+    }
+    const uint32_t n0 = __shfl(n, 13, 32), p0 = __shfl(s0, 13, 32);
+    if (lane == 13) n = 0;
+    uint32_t inc = n;
+#pragma unroll
+    for (int off = 1; off < 32; off <<= 1) {
+        const uint32_t o = __shfl_up(inc, off, 32);
+        if (lane >= off) inc += o;
+    }
+    if (T < g.ntiles) {
+        uint32_t* L = lists + (size_t)T * LIST_WORDS;
+        if (lane < 27) {
+            L[LIST_START + lane] = s0 - (inc - n);
+            L[LIST_PREF + 1 + lane] = inc;
+        } else if (lane == 27) {
+            L[LIST_PREF] = 0;
+        } else if (lane == 28) {
+            L[LIST_OWN] = p0;
+            L[LIST_OWN + 1] = n0;
+        }
+    }
+    if (lane == 31) cnt[tid >> 5] = T < g.ntiles ? n0 + inc : 0u;
+    __syncthreads();
+    uint32_t total;
+    const uint32_t pre = block_prefix<LIST_THREADS>(tid < TILES_PER_LIST_BLOCK ? cnt[tid] : 0u, wsum, total);
+    const int Ts = blockIdx.x * TILES_PER_LIST_BLOCK + tid;
+    if (tid < TILES_PER_LIST_BLOCK && Ts < g.ntiles) loc[Ts] = pre;
+    if (tid == 0) {
+        // (the sums go around the caches, so the ticket need not write back
+        // and invalidate an L2 per block; only its order after the store
+        // matters: 27 -> 15 us per launch)
+        __hip_atomic_store(blk + blockIdx.x, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        last = __hip_atomic_fetch_add(scal + SC_TICKET, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    uint32_t run = 0;
+    for (uint32_t b0 = 0; b0 < gridDim.x; b0 += LIST_THREADS) {
+        const uint32_t b = b0 + tid;
+        const uint32_t v = b < gridDim.x ? __hip_atomic_load(blk + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+        uint32_t tot;
+        __syncthreads();  // the previous round's sums are read
+        const uint32_t p = block_prefix<LIST_THREADS>(v, wsum, tot);
+        if (b < gridDim.x) blk[b] = run + p;
+        run += tot;
+    }
+    if (tid == 0) {
+        scal[SC_NP] = run;  // all that the tiles hold
+        scal[SC_TICKET] = 0;
+    }
+}
+
+// How full the tiles are, for the choice of the push's workgroups: of about
+// FILL_SAMPLE tiles spread over the grid the number that hold
+// 64c-63 .. 64c particles, per class c (the last class also fuller ones;
+// empty tiles are not counted).  One block, once per run of steps.
+constexpr int FILL_CLASSES = SC_N - SC_FILL, FILL_SAMPLE = 4096, FILL_THREADS = 1024;
+RH_HD int fill_class(uint32_t n) { return n >= 64u * (FILL_CLASSES - 1) ? FILL_CLASSES - 1 : (int)((n + 63u) / 64u); }
+
+__global__ __launch_bounds__(FILL_THREADS) void k_tile_fill(Geom g, const uint32_t* __restrict__ lists,
+                                                            uint32_t* __restrict__ scal) {
+    __shared__ uint32_t h[FILL_CLASSES];
+    const int tid = threadIdx.x, stride = (g.ntiles + FILL_SAMPLE - 1) / FILL_SAMPLE;
+    if (tid < FILL_CLASSES) h[tid] = 0;
+    __syncthreads();
+    for (int T = tid * stride; T < g.ntiles; T += FILL_THREADS * stride) {
+        const uint32_t* L = lists + (size_t)T * LIST_WORDS;
+        const uint32_t n = L[LIST_PREF + 27] + L[LIST_OWN + 1];
+        if (n) atomicAdd(&h[fill_class(n)], 1u);
+    }
+    __syncthreads();
+    if (tid < FILL_CLASSES) scal[SC_FILL + tid] = h[tid];
+}
+
+// A Geom whose tile shape is known to the compiler: sides 2^LX, 2^LY, 2^LZ
+// (LX < 0: as g says).
+template <int LX, int LY, int LZ>
+__device__ __forceinline__ Geom with_shape(const Geom& g) {
+    Geom h = g;
+    if constexpr (LX >= 0) {
+        h.ltx = LX; h.lty = LY; h.ltz = LZ;
+        h.tx = 1 << LX; h.ty = 1 << LY; h.tz = 1 << LZ;
+        h.tc = h.tx * h.ty * h.tz;
+        h.ex = h.tx + 2; h.ey = h.ty + 2; h.ez = h.tz + 2;
+        h.next = h.ex * h.ey * h.ez;
+        h.extk = 8 * h.next;
+        set_slots(h);
+    }
+    return h;
+}
+
+// LDS of k_push_sort: one round's pushed particles (24 B in FP32) and their
+// codes, its list of particles by slot (each slot's part padded to an even
+// count), the slots' counts, list parts and places, the extended cells'
+// codes, the tile's field block.
 template <typename Real>
-__global__ __launch_bounds__(PM_THREADS) void k_push_move(Geom g, PushParams pp, const uint32_t* __restrict__ pfb,
-                                                         PArrays<Real> A, PArrays<Real> D,
-                                                         const uint32_t* __restrict__ sub, InjAppendix app,
-                                                         uint16_t* __restrict__ cnt_tile,
-                                                         const uint32_t* __restrict__ key_base,
-                                                         unsigned long long* __restrict__ counters, int kbits,
-                                                         int pass, uint32_t cap) {
-    extern __shared__ __align__(16) unsigned char pm_smem[];
-    const int NS = g.tc * 8;
+struct PushLds {
+    size_t s2, code, list, cnt, loff, goff, codes, field, bytes;
+};
+template <typename Real>
+RH_HD PushLds<Real> push_lds(const Geom& g, int round, int lq) {
+    const size_t kq = (size_t)g.kt << lq;
+    PushLds<Real> o;
+    o.s2 = 4 * sizeof(Real) * (size_t)round;
+    o.code = o.s2 + 2 * sizeof(Real) * (size_t)round;
+    o.list = o.code + 4 * (size_t)round;
+    o.cnt = o.list + pm_align16(2 * ((size_t)round + kq));
+    o.loff = o.cnt + pm_align16(4 * kq);
+    o.goff = o.loff + pm_align16(2 * kq);
+    o.codes = o.goff + pm_align16(4 * kq);
+    o.field = o.codes + pm_align16(4 * ((size_t)g.next + 1));
+    o.bytes = o.field + 4 * push_field_words<Real>(g);
+    return o;
+}
+
+// A particle's code in the push: its slot (g.nslot: removed), in CODE_OCT the
+// octant bits that the slot still lacks (7 for a cell of the tile), then its
+// rank in the round and the destination's local cell.
+constexpr uint32_t SLOT_BITS = 10, SLOT_MASK = (1u << SLOT_BITS) - 1u;
+constexpr uint32_t CODE_OCT_SHIFT = SLOT_BITS;
+constexpr uint32_t RANK_SHIFT = SLOT_BITS, RANK_ROUND_BITS = 13, RANK_MASK_ROUND = (1u << RANK_ROUND_BITS) - 1u;
+constexpr uint32_t CELL_SHIFT = RANK_SHIFT + RANK_ROUND_BITS;
+
+// Host: the codes of the extended cells of a tile with full neighbours on
+// all sides, and per extended cell in which directions it leaves the tile
+// (bit 0 -x, 1 +x, 2 -y, 3 +y, 4 -z, 5 +z).
+inline void tile_codes(const Geom& g, const uint16_t* slots, uint32_t* code, uint32_t* side) {
+    for (int e = 0; e < g.next; ++e) {
+        const int t[3] = {g.tx, g.ty, g.tz};
+        int l[3] = {e % g.ex - 1, (e / g.ex) % g.ey - 1, e / (g.ex * g.ey) - 1};
+        side[e] = 0;
+        for (int d = 0; d < 3; ++d) {
+            if (l[d] < 0) { side[e] |= 1u << (2 * d); l[d] = t[d] - 1; }
+            else if (l[d] >= t[d]) { side[e] |= 2u << (2 * d); l[d] = 0; }
+        }
+        const uint32_t nlc = (uint32_t)(l[0] + (l[1] << g.ltx) + (l[2] << (g.ltx + g.lty)));
+        code[e] = side[e] ? (uint32_t)slots[e] | nlc << CELL_SHIFT : 8u * nlc | 7u << CODE_OCT_SHIFT | nlc << CELL_SHIFT;
+    }
+}
+
+// The code of extended cell e of tile (bx,by,bz): a cell of the tile, of a
+// neighbouring tile (with that tile's local cell), or none (outside a
+// non-periodic grid, or beyond the halo of a partial tile).
+__device__ __forceinline__ uint32_t cell_code(const Geom& g, int bx, int by, int bz, int e, const uint16_t* slots) {
+    const int b[3] = {bx, by, bz}, n[3] = {g.nx, g.ny, g.nz}, lt[3] = {g.ltx, g.lty, g.ltz}, nt[3] = {g.ntx, g.nty, g.ntz},
+              t[3] = {g.tx, g.ty, g.tz};
+    const int l[3] = {e % g.ex - 1, (e / g.ex) % g.ey - 1, e / (g.ex * g.ey) - 1};
+    bool own = true, exists = true;
+    int c[3], x[3];  // destination's local coordinate; extended coordinate in a full tile
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const int w = tile_width(n[d], lt[d], b[d]);
+        c[d] = l[d];
+        x[d] = l[d] + 1;
+        if (l[d] < 0) {
+            own = false;
+            exists = exists && (b[d] > 0 || g.per[d]);
+            c[d] = tile_width(n[d], lt[d], b[d] > 0 ? b[d] - 1 : nt[d] - 1) - 1;
+        } else if (l[d] >= w) {
+            own = false;
+            exists = exists && l[d] == w && (b[d] < nt[d] - 1 || g.per[d]);
+            c[d] = 0;
+            x[d] = t[d] + 1;
+        }
+    }
+    const uint32_t nlc = (uint32_t)(c[0] + (c[1] << g.ltx) + (c[2] << (g.ltx + g.lty)));
+    if (own) return 8u * nlc | 7u << CODE_OCT_SHIFT | nlc << CELL_SHIFT;
+    if (!exists) return (uint32_t)g.nslot;
+    return (uint32_t)slots[x[0] + g.ex * (x[1] + g.ey * x[2])] | nlc << CELL_SHIFT;
+}
+
+template <typename Real>
+struct Particle {
+    Real X, Y, Z, vx, vy, vz;
+};
+
+// One particle: push, move, code.  fl is the tile's field block, codes its
+// extended cells' codes; edge: the tile holds cells without all neighbours.
+// PLAIN: accelerated, without gravity, and moved (the parameters of most
+// runs; the others are tested for).  Without branches except for the speed
+// limit, so that several particles' LDS reads are in flight.
+template <typename Real, bool PLAIN>
+__device__ __forceinline__ uint32_t push_particle(const Geom& g, const PushParams& pp, const int (&org)[3], bool edge,
+                                                  const Real* fl, const uint32_t* codes, Particle<Real>& q, int lc,
+                                                  uint32_t& n_clamped, uint32_t& n_dropped) {
+    const bool act = q.X >= Real(0);
     const int hx = g.tx + 1, hy = g.ty + 1, nh = (g.tx + 1) * (g.ty + 1) * (g.tz + 1);
-    uint32_t* cnt = reinterpret_cast<uint32_t*>(pm_smem);     // extk running slot counts
-    uint8_t* grp = reinterpret_cast<uint8_t*>(cnt + g.extk);   // PM_WAVES x extk group sizes
-    Real* fl = reinterpret_cast<Real*>(pm_smem + pm_align8(4 * (size_t)g.extk + (size_t)PM_WAVES * g.extk));
-    Real* sbx = fl;            // faceB of local cells -1..t-1 (halo on the low side)
-    Real* sby = fl + nh;
-    Real* sbz = fl + 2 * nh;
-    Real* sue = fl + 3 * nh;   // cellUe, cellEp of the tile's cells
-    Real* sep = sue + 3 * g.tc;
-    uint32_t* nmask = reinterpret_cast<uint32_t*>(sep + 3 * g.tc);  // neighbourhood of each tile cell
-    const int T = pass == 1 ? xcd_brick_tile(g, (int)blockIdx.x) : xcd_tile(g, (int)blockIdx.x);
+    const Real* sbx = fl;  // faceB of local cells -1..t-1 (halo on the low side)
+    const Real* sby = fl + nh;
+    const Real* sbz = fl + 2 * nh;
+    const Real* sue = fl + 3 * nh;  // cellUe, cellEp of the tile's cells
+    const Real* sep = sue + 3 * g.tc;
+    Real X = q.X, Y = q.Y, Z = q.Z, vx = q.vx, vy = q.vy, vz = q.vz;
+    int li, lj, lk;
+    local_ijk(g, lc, li, lj, lk);
+    bool accel = PLAIN || (pp.accelerate && !pp.initial_flow_through);
+    // (the neighbourhood mask of the cell)
+    if (edge) accel = accel && ((reinterpret_cast<const uint32_t*>(sep + 3 * g.tc)[lc] >> NMASK_ALL) & 1u);
+    if (PLAIN || (pp.accelerate && !pp.initial_flow_through)) {
+        const int h = (li + 1) + hx * ((lj + 1) + hy * (lk + 1));
+        // face2r: each component linear along its own axis only
+        const Real Bx = X * sbx[h] + (Real(1) - X) * sbx[h - 1];
+        const Real By = Y * sby[h] + (Real(1) - Y) * sby[h - hx];
+        const Real Bz = Z * sbz[h] + (Real(1) - Z) * sbz[h - hx * hy];
+        // cell2r: nearest grid point; E = B x Ue (= -Ue x B) (+ Ep)
+        const Real Ux = sue[lc], Uy = sue[g.tc + lc], Uz = sue[2 * g.tc + lc];
+        Real Ex = By * Uz - Bz * Uy;
+        Real Ey = Bz * Ux - Bx * Uz;
+        Real Ez = Bx * Uy - By * Ux;
+        Ex += sep[lc]; Ey += sep[g.tc + lc]; Ez += sep[2 * g.tc + lc];
+        const Real qm = (Real)pp.qmdt2;
+        const Real dvx = qm * Ex, dvy = qm * Ey, dvz = qm * Ez;
+        const Real tx = qm * Bx, ty = qm * By, tz = qm * Bz;
+        const Real t2 = tx * tx + ty * ty + tz * tz;
+        const Real b2 = boris_s_factor(t2);
+        const Real sx = b2 * tx, sy = b2 * ty, sz = b2 * tz;
+        const Real vmx = vx + dvx, vmy = vy + dvy, vmz = vz + dvz;
+        const Real v0x = vmx + vmy * tz - vmz * ty;
+        const Real v0y = vmy + vmz * tx - vmx * tz;
+        const Real v0z = vmz + vmx * ty - vmy * tx;
+        vx = vmx + v0y * sz - v0z * sy + dvx;
+        vy = vmy + v0z * sx - v0x * sz + dvy;
+        vz = vmz + v0x * sy - v0y * sx + dvz;
+        if (!PLAIN && pp.use_gravity) {
+            const double rx = g.x0 + (org[0] + li + (double)X) * g.dx;
+            const double ry = g.y0 + (org[1] + lj + (double)Y) * g.dx;
+            const double rz = g.z0 + (org[2] + lk + (double)Z) * g.dx;
+            const double r = sqrt(rx * rx + ry * ry + rz * rz);
+            const double r3 = r * r * r;
+            if (r3 > 0) {
+                const double s = -pp.GMdt / r3;
+                vx += (Real)(s * rx); vy += (Real)(s * ry); vz += (Real)(s * rz);
+            }
+        }
+        const Real v2 = vx * vx + vy * vy + vz * vz;
+        if (act && accel && v2 > (Real)pp.max_vi2) {
+            const Real norm = sqrt((Real)pp.max_vi2 / v2);
+            vx *= norm; vy *= norm; vz *= norm;
+            ++n_clamped;
+        }
+        if (edge) {  // particles of cells without all neighbours keep their velocity
+            vx = accel ? vx : q.vx; vy = accel ? vy : q.vy; vz = accel ? vz : q.vz;
+        }
+    }
+    // move in FP64; the integer part is the cell crossing (a still pass keeps
+    // every particle where it is)
+    int sx = 0, sy = 0, sz = 0;
+    if (PLAIN || !pp.still) {
+        const double Xd = (double)X + (double)vx * pp.dt_dx;
+        const double Yd = (double)Y + (double)vy * pp.dt_dx;
+        const double Zd = (double)Z + (double)vz * pp.dt_dx;
+        sx = (int)floor(Xd); sy = (int)floor(Yd); sz = (int)floor(Zd);
+        // (a tiny negative Xd has the fraction next below one, as the
+        // difference from its floor, which rounds to one, has after the limit)
+        X = (Real)__builtin_amdgcn_fract(Xd); Y = (Real)__builtin_amdgcn_fract(Yd); Z = (Real)__builtin_amdgcn_fract(Zd);
+    }
+    // at most one cell along each axis, and nothing that is not a number
+    const bool ok = (unsigned)(sx + 1) <= 2u && (unsigned)(sy + 1) <= 2u && (unsigned)(sz + 1) <= 2u && X + Y + Z >= Real(0);
+    if (PLAIN || !pp.still) {
+        X = X < Real(1) ? X : below_one<Real>();
+        Y = Y < Real(1) ? Y : below_one<Real>();
+        Z = Z < Real(1) ? Z : below_one<Real>();
+    }
+    const uint32_t code = codes[act && ok ? (li + sx + 1) + g.ex * ((lj + sy + 1) + g.ey * (lk + sz + 1)) : g.next];
+    const uint32_t o = (X >= Real(0.5)) + 2 * (Y >= Real(0.5)) + 4 * (Z >= Real(0.5));
+    n_dropped += act && (code & SLOT_MASK) == (uint32_t)g.nslot;
+    q.X = X; q.Y = Y; q.Z = Z; q.vx = vx; q.vy = vy; q.vz = vz;
+    return (code & ~(7u << CODE_OCT_SHIFT)) + (o & (code >> CODE_OCT_SHIFT & 7u));
+}
+
+// How many of the slot's list entries (from `part`, c of them, padded with
+// 0xFFFF to an even count) are below `me`: two at a time.
+__device__ __forceinline__ uint32_t list_rank(const uint16_t* part, uint32_t c, uint32_t me) {
+    const uint32_t m = me | me << 16;
+    uint32_t r = 0;
+#pragma clang loop unroll(disable)
+    for (uint32_t e = 0; e < c; e += 2) {
+        uint32_t a;  // (me - entry, limited to 0 and 1, in each half)
+        asm("v_pk_sub_u16 %0, %1, %2 clamp" : "=v"(a) : "v"(m), "v"(*reinterpret_cast<const uint32_t*>(part + e)));
+        asm("v_pk_min_u16 %0, %1, 1 op_sel_hi:[1,0]" : "=v"(a) : "v"(a));
+        r += a;
+    }
+    return (r & 0xFFFFu) + (r >> 16);
+}
+
+// A tile whose particles fit one round (`round` of them, as the LDS was sized
+// for) is read once: each pushed particle waits in LDS while the slots are
+// counted (integer LDS atomics) and scanned, and is then written to its
+// place, a wave writing 64 places in a row (written by the particles' own
+// order instead, a wave's places lie in up to twice as many cache lines and
+// the address units bound the kernel).  A fuller tile is pushed three times:
+// to count, then round by round for the codes and to write.  A particle's
+// rank in its slot is the number of the round's particles of that slot that
+// come before it: the atomics hand out places of a list by slot in any order,
+// and each particle then counts the smaller entries of its slot's few, so the
+// sort is stable and every run writes the same order.
+template <typename Real, int NT, int LX, int LY, int LZ, bool PLAIN>
+__global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
+    Geom g_, PushParams pp, const uint32_t* __restrict__ pfb, PArrays<Real> A, PArrays<Real> D,
+    const uint16_t* __restrict__ dirs,
+    const uint16_t* __restrict__ slots, const uint32_t* __restrict__ full_codes, uint32_t* __restrict__ tab_out,
+    uint32_t* __restrict__ dtab_out, uint8_t* __restrict__ live_out, const uint32_t* __restrict__ lists,
+    const uint32_t* __restrict__ seg_loc, const uint32_t* __restrict__ seg_blk, InjAppendix app,
+    uint32_t* __restrict__ scal, unsigned long long* __restrict__ counters, uint32_t cap, int round, int lq) {
+    const Geom g = with_shape<LX, LY, LZ>(g_);
+    extern __shared__ __align__(16) unsigned char pm_smem[];
+    __shared__ uint32_t wsum[16], L[LIST_WORDS];
+    const int NS = 8 * g.tc, K = g.nslot;
+    const int KQ = K << lq, KT = g.kt << lq;  // the parts of the slots
+    const PushLds<Real> o = push_lds<Real>(g, round, lq);
+    Real4<Real>* S4 = reinterpret_cast<Real4<Real>*>(pm_smem);         // x, y, z, vx
+    Real2<Real>* S2 = reinterpret_cast<Real2<Real>*>(pm_smem + o.s2);  // vy, vz
+    uint32_t* scode = reinterpret_cast<uint32_t*>(pm_smem + o.code);
+    uint16_t* list = reinterpret_cast<uint16_t*>(pm_smem + o.list);
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(pm_smem + o.cnt);    // this round's particles per slot (entry K: the removed)
+    uint16_t* loff = reinterpret_cast<uint16_t*>(pm_smem + o.loff);  // where the slot's part of the list starts
+    uint32_t* goff = reinterpret_cast<uint32_t*>(pm_smem + o.goff);  // the slot's next place in the slot order
+    uint32_t* codes = reinterpret_cast<uint32_t*>(pm_smem + o.codes);
+    Real* fl = reinterpret_cast<Real*>(pm_smem + o.field);
+    const int T = xcd_tile(g, (int)blockIdx.x);
     if (T >= g.ntiles) return;
+    const int tid = threadIdx.x, lane = tid & 63;
+    // the tile's lists, one word per lane, and everything else that does not
+    // depend on them: one round of latency, then the particles' own
+    const uint32_t lw = lists[(size_t)T * LIST_WORDS + lane];
+    const uint32_t np = scal[SC_NP], sloc = seg_loc[T], sblk = seg_blk[T / TILES_PER_LIST_BLOCK];
+    const int mydir = tid < 28 ? (int)dirs[tid] : 0;
+    uint32_t c0 = 0, c1 = 0;
+    if (app.cbeg) { c0 = app.cbeg[T]; c1 = app.cbeg[T + 1]; }
     int bx, by, bz;
     tile_coords(g, T, bx, by, bz);
-    const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-    const int ox = bx << g.ltx, oy = by << g.lty, oz = bz << g.ltz;
-    // the tile's particle range first: its loads overlap the set-up below
-    const uint32_t p0 = sub[(size_t)T * NS], p1 = sub[(size_t)(T + 1) * NS];
-    // the tile's injected particles (past the store's end) follow its own
-    uint32_t a0 = 0, na = 0;
-    if (app.cbeg) {
-        const uint32_t c0 = app.cbeg[T], c1 = app.cbeg[T + 1];
-        if (c1 > c0) { a0 = sub[g.nkeys] + app.off[c0]; na = app.off[c1] - app.off[c0]; }
-    }
-    const uint32_t n0 = p1 - p0, ntot = n0 + na;
-    if (pass == 0 && tid == 0) pp.live[T] = ntot > 0 ? 1 : 0;
-    // an empty tile (common for a species confined to part of the grid):
-    // nothing to push or move, and its slot table is not written (the slot
-    // kernel reads the tables of live tiles only)
-    if (ntot == 0) return;
-    const uint32_t deadkey = (uint32_t)MAX_EXTK;
-    // prefetch of the first chunk; an injected particle beyond the store's
-    // capacity was never written (the injection counted the overflow)
-    // (the tile's particles in chunks of PM_THREADS, prefetched two chunks
-    // ahead into two register buffers used in turn: no copies between them,
-    // so a buffer's loads are waited for only where its chunk is used)
-    struct PBuf { Real X, Y, Z, vx, vy, vz; int lc; };
-    auto load_chunk = [&](PBuf& b, uint32_t u) {
-        const uint32_t p = u < n0 ? p0 + u : a0 + (u - n0);
-        if (u < ntot) {
-            if (p < cap) { b.X = A.x[p]; b.Y = A.y[p]; b.Z = A.z[p]; b.vx = A.vx[p]; b.vy = A.vy[p]; b.vz = A.vz[p]; b.lc = A.lc[p]; }
-            else b.X = Real(-1);
-        }
+    const int org[3] = {bx << g.ltx, by << g.lty, bz << g.ltz};
+    const bool edge = (!g.per[0] && (org[0] < 1 || org[0] + g.tx > g.nx - 1)) ||
+                      (!g.per[1] && (org[1] < 1 || org[1] + g.ty > g.ny - 1)) ||
+                      (!g.per[2] && (org[2] < 1 || org[2] + g.tz > g.nz - 1));
+    const uint32_t p0 = (uint32_t)__builtin_amdgcn_readlane((int)lw, LIST_OWN),
+                   n0 = (uint32_t)__builtin_amdgcn_readlane((int)lw, LIST_OWN + 1),
+                   na = (uint32_t)__builtin_amdgcn_readlane((int)lw, LIST_PREF + 27);
+    // (uniform base pointers and 32-bit offsets for the tile's own places)
+    auto own = [&](uint32_t u, Particle<Real>& q, int& lc) {
+        q.X = (A.x + p0)[u]; q.Y = (A.y + p0)[u]; q.Z = (A.z + p0)[u];
+        q.vx = (A.vx + p0)[u]; q.vy = (A.vy + p0)[u]; q.vz = (A.vz + p0)[u];
+        lc = (A.lc + p0)[u];
     };
-    PBuf bufA{Real(0), Real(0), Real(0), Real(0), Real(0), Real(0), 0};
-    PBuf bufB = bufA;
-    load_chunk(bufA, tid);
-    load_chunk(bufB, tid + PM_THREADS);
-    // slot counters: the 8 octant slots of an extended cell are 8 consecutive
-    // entries (16-byte vectors of counts, 32-byte vectors of subcell starts)
-    uint4* cnt4 = reinterpret_cast<uint4*>(cnt);
-    if (pass == 0) {
-        for (int e = tid; e < g.extk / 4; e += PM_THREADS) cnt4[e] = make_uint4(0u, 0u, 0u, 0u);
-    } else {
-        // each slot's first destination index: the destination subcell's
-        // start (key_base) plus the slot's offset inside it (cnt_tile); the
-        // running counter then grows by the slot's particles in order
-        for (int ec = tid; ec < g.next; ec += PM_THREADS) {
-            const int lx = ec % g.ex - 1, ly = (ec / g.ex) % g.ey - 1, lz = ec / (g.ex * g.ey) - 1;
-            int tX = bx + (lx < 0 ? -1 : (lx >= g.tx ? 1 : 0));
-            int tY = by + (ly < 0 ? -1 : (ly >= g.ty ? 1 : 0));
-            int tZ = bz + (lz < 0 ? -1 : (lz >= g.tz ? 1 : 0));
-            // (outside a non-periodic grid the slot is never used; the wrap
-            // keeps the index in range)
-            tX += tX < 0 ? g.ntx : (tX >= g.ntx ? -g.ntx : 0);
-            tY += tY < 0 ? g.nty : (tY >= g.nty ? -g.nty : 0);
-            tZ += tZ < 0 ? g.ntz : (tZ >= g.ntz ? -g.ntz : 0);
-            const uint32_t nl = (uint32_t)((lx & (g.tx - 1)) + ((ly & (g.ty - 1)) << g.ltx) +
-                                           ((lz & (g.tz - 1)) << (g.ltx + g.lty)));
-            const uint32_t gk = ((uint32_t)(tX + g.ntx * (tY + g.nty * tZ)) * (uint32_t)g.tc + nl) * 8u;
-            const uint4 b0 = *reinterpret_cast<const uint4*>(key_base + gk);
-            const uint4 b1 = *reinterpret_cast<const uint4*>(key_base + gk + 4);
-            const uint4 c = *reinterpret_cast<const uint4*>(cnt_tile + ((size_t)T * g.next + ec) * 8);
-            cnt4[2 * ec] = make_uint4(b0.x + (c.x & 0xFFFFu), b0.y + (c.x >> 16), b0.z + (c.y & 0xFFFFu), b0.w + (c.y >> 16));
-            cnt4[2 * ec + 1] = make_uint4(b1.x + (c.z & 0xFFFFu), b1.y + (c.z >> 16), b1.z + (c.w & 0xFFFFu), b1.w + (c.w >> 16));
-        }
+    Particle<Real> nq{Real(-1), Real(0), Real(0), Real(0), Real(0), Real(0)};  // the thread's next particle
+    int nlc = 0;
+    if ((uint32_t)tid < n0) own((uint32_t)tid, nq, nlc);
+    const uint32_t room = min(cap > np ? cap - np : 0u, app.places);
+    uint32_t a0 = 0, a1 = 0, before = 0;  // injected particles: the tile's, those of the tiles before it
+    if (app.cbeg) {
+        before = min(appendix_offset(app, c0), room);
+        a0 = before;
+        a1 = min(appendix_offset(app, c1), room);
     }
-    for (int e = tid; e < PM_WAVES * g.extk / 16; e += PM_THREADS) reinterpret_cast<uint4*>(grp)[e] = make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t n1 = n0 + na, N = uniform(n1 + (a1 - a0));
+    a0 += app.at_end ? np : cap;
+    // the segment: the places of the tiles before it
+    const uint32_t seg = uniform(sloc + sblk + before);
+    if (tid == 0) {
+        live_out[T] = N > 0;
+        if (T == 0) scal[SC_END] = np + (app.cbeg ? min(appendix_offset(app, app.cbeg[g.ntiles]), room) : 0u);
+    }
+    if (N == 0) {  // the slot tables of an empty tile are not read
+        if (tid < DIR_WORDS) dtab_out[(size_t)T * DIR_WORDS + tid] = seg;
+        return;
+    }
+    if (tid < LIST_WORDS) L[tid] = lw;
+    // the others: arrivals, then injected particles
+    auto other = [&](uint32_t v, Particle<Real>& q, int& lc) {
+        const uint32_t p = v < na ? arrival_index(L, v) : a0 + (v - na);
+        q.X = A.x[p]; q.Y = A.y[p]; q.Z = A.z[p];
+        q.vx = A.vx[p]; q.vy = A.vy[p]; q.vz = A.vz[p];
+        lc = A.lc[p];
+    };
+    const uint32_t places = cap > seg ? cap - seg : 0u;
+    const bool one = N <= (uint32_t)round;
+    for (int e = tid; e < KT; e += NT) cnt[e] = 0u;
+    for (int e = tid; e < (round + KT) / 2; e += NT) reinterpret_cast<uint32_t*>(list)[e] = ~0u;
     {
         const int nw4 = (int)push_field_words<Real>(g) / 4;
         const uint4* src = reinterpret_cast<const uint4*>(pfb) + (size_t)T * nw4;
         uint4* dst = reinterpret_cast<uint4*>(fl);
-        for (int q = tid; q < nw4; q += PM_THREADS) dst[q] = src[q];
+        for (int e = tid; e < nw4; e += NT) dst[e] = src[e];
+        // the extended cells' codes: those of a tile amid full ones, less the
+        // cells that do not exist; beside a partial tile (also across a wrap)
+        // they differ
+        const int b[3] = {bx, by, bz}, n[3] = {g.nx, g.ny, g.nz}, lt[3] = {g.ltx, g.lty, g.ltz}, nt[3] = {g.ntx, g.nty, g.ntz};
+        uint32_t missing = 0;
+        bool full = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            if (!g.per[d] && b[d] == 0) missing |= 1u << (2 * d);
+            if (!g.per[d] && b[d] == nt[d] - 1) missing |= 2u << (2 * d);
+            const bool whole = (n[d] & ((1 << lt[d]) - 1)) == 0;
+            full = full && (whole || (b[d] < nt[d] - 1 && !(g.per[d] && b[d] == 0)));
+        }
+        for (int e = tid; e <= g.next; e += NT) {
+            uint32_t c = (uint32_t)K;
+            if (e < g.next) {
+                if (!full) c = cell_code(g, bx, by, bz, e, slots);
+                else if (!(full_codes[g.next + e] & missing)) c = full_codes[e];
+            }
+            codes[e] = c;
+        }
     }
     __syncthreads();
-    uint32_t n_clamped = 0, n_dropped = 0;  // this lane's events (pass 0)
-    auto chunk = [&](uint32_t ub, PBuf& buf) {
-        const uint32_t u = ub + tid;
-        const bool act = u < ntot;
-        Real X = buf.X, Y = buf.Y, Z = buf.Z, vx = buf.vx, vy = buf.vy, vz = buf.vz;
-        const int lc = buf.lc;
-        load_chunk(buf, u + 2 * PM_THREADS);
-        uint32_t key = deadkey;
-        bool clamped = false, dropped = false;
-        int di = 0, dj = 0, dk = 0;  // destination cell, local coordinates of the source tile
-        if (act && X >= Real(0)) {
-            int li, lj, lk;
-            local_ijk(g, lc, li, lj, lk);
-            const uint32_t nm = nmask[lc];
-            const bool accel = pp.accelerate && ((nm >> NMASK_ALL) & 1u) && !pp.initial_flow_through;
-            if (accel) {
-                const int h = (li + 1) + hx * ((lj + 1) + hy * (lk + 1));
-                // face2r: each component linear along its own axis only
-                const Real Bx = X * sbx[h] + (Real(1) - X) * sbx[h - 1];
-                const Real By = Y * sby[h] + (Real(1) - Y) * sby[h - hx];
-                const Real Bz = Z * sbz[h] + (Real(1) - Z) * sbz[h - hx * hy];
-                // cell2r: nearest grid point; E = B x Ue (= -Ue x B) (+ Ep)
-                const Real Ux = sue[lc], Uy = sue[g.tc + lc], Uz = sue[2 * g.tc + lc];
-                Real Ex = By * Uz - Bz * Uy;
-                Real Ey = Bz * Ux - Bx * Uz;
-                Real Ez = Bx * Uy - By * Ux;
-                Ex += sep[lc]; Ey += sep[g.tc + lc]; Ez += sep[2 * g.tc + lc];
-                const Real qm = (Real)pp.qmdt2;
-                const Real dvx = qm * Ex, dvy = qm * Ey, dvz = qm * Ez;
-                const Real tx = qm * Bx, ty = qm * By, tz = qm * Bz;
-                const Real t2 = tx * tx + ty * ty + tz * tz;
-                const Real b2 = boris_s_factor(t2);
-                const Real sx = b2 * tx, sy = b2 * ty, sz = b2 * tz;
-                const Real vmx = vx + dvx, vmy = vy + dvy, vmz = vz + dvz;
-                const Real v0x = vmx + vmy * tz - vmz * ty;
-                const Real v0y = vmy + vmz * tx - vmx * tz;
-                const Real v0z = vmz + vmx * ty - vmy * tx;
-                vx = vmx + v0y * sz - v0z * sy + dvx;
-                vy = vmy + v0z * sx - v0x * sz + dvy;
-                vz = vmz + v0x * sy - v0y * sx + dvz;
-                if (pp.use_gravity) {
-                    const double rx = g.x0 + (ox + li + (double)X) * g.dx;
-                    const double ry = g.y0 + (oy + lj + (double)Y) * g.dx;
-                    const double rz = g.z0 + (oz + lk + (double)Z) * g.dx;
-                    const double r = sqrt(rx * rx + ry * ry + rz * rz);
-                    const double r3 = r * r * r;
-                    if (r3 > 0) {
-                        const double s = -pp.GMdt / r3;
-                        vx += (Real)(s * rx); vy += (Real)(s * ry); vz += (Real)(s * rz);
-                    }
-                }
-                const Real v2 = vx * vx + vy * vy + vz * vz;
-                if (v2 > (Real)pp.max_vi2) {
-                    const Real norm = sqrt((Real)pp.max_vi2 / v2);
-                    vx *= norm; vy *= norm; vz *= norm;
-                    clamped = true;
+    uint32_t n_clamped = 0, n_dropped = 0;
+    // the code with the slot's part of the round's particle i
+    auto part_code = [&](uint32_t c, int i) {
+        const uint32_t s = c & SLOT_MASK;
+        return c + (s << lq) - s + ((uint32_t)i & ((1u << lq) - 1u));
+    };
+    // The slots' places in the slot order (goff) and parts of the list (loff,
+    // even) from the counts; the sum in every thread.
+    auto scan_slots = [&](bool whole) {
+        const int E = (KQ + NT - 1) / NT, e0 = tid * E;
+        uint32_t s = 0, sp = 0;
+        for (int e = e0; e < e0 + E; ++e)
+            if (e < KQ) { s += cnt[e]; sp += (cnt[e] + 1u) & ~1u; }
+        // (both sums in one scan, 16 bits each, unless the counts are the
+        // whole tile's, whose list parts are not used)
+        uint32_t total;
+        uint32_t run = block_prefix<NT>(whole ? s : s | sp << 16, wsum, total);
+        for (int e = e0; e < e0 + E; ++e)
+            if (e < KQ) {
+                const uint32_t c = cnt[e];
+                if (whole) {
+                    goff[e] = run;
+                    run += c;
+                } else {
+                    if (one) goff[e] = run & 0xFFFFu;
+                    loff[e] = (uint16_t)(run >> 16);
+                    run += c | ((c + 1u) & ~1u) << 16;
                 }
             }
-            // move in FP64; the integer part is the cell crossing (a still
-            // pass keeps every particle where it is)
-            int sx = 0, sy = 0, sz = 0;
-            bool ok = true;
-            if (!pp.still) {
-                const double Xd = (double)X + (double)vx * pp.dt_dx;
-                const double Yd = (double)Y + (double)vy * pp.dt_dx;
-                const double Zd = (double)Z + (double)vz * pp.dt_dx;
-                const double fx = floor(Xd), fy = floor(Yd), fz = floor(Zd);
-                ok = (fx >= -1.0 && fx <= 1.0 && fy >= -1.0 && fy <= 1.0 && fz >= -1.0 && fz <= 1.0);
-                sx = (int)fx; sy = (int)fy; sz = (int)fz;
-                X = (Real)(Xd - fx); Y = (Real)(Yd - fy); Z = (Real)(Zd - fz);
-                if (X >= Real(1)) X = below_one<Real>();
-                if (Y >= Real(1)) Y = below_one<Real>();
-                if (Z >= Real(1)) Z = below_one<Real>();
-            }
-            if (ok && ((nm >> ((sx + 1) + 3 * (sy + 1) + 9 * (sz + 1))) & 1u)) {
-                const int o = (X >= Real(0.5)) + 2 * (Y >= Real(0.5)) + 4 * (Z >= Real(0.5));
-                di = li + sx; dj = lj + sy; dk = lk + sz;
-                key = (uint32_t)(((di + 1) + g.ex * ((dj + 1) + g.ey * (dk + 1))) * 8 + o);
-            } else {
-                dropped = true;
-            }
+        total = whole ? total : total & 0xFFFFu;
+        if ((whole || one) && tid == 0) goff[KQ] = total;
+        return total;
+    };
+    // the tile's tables, from the slots' places
+    auto write_tables = [&](uint32_t total) {
+        __syncthreads();  // goff is written
+        for (int e = tid; e < K; e += NT) {
+            const uint32_t f = goff[e << lq];
+            tab_out[(size_t)T * g.kt + e] = seg + f;
+            if (e < NS && goff[(e + 1) << lq] - f > 0xFFFFu) atomicAdd(counters + C_RANK_OVERFLOW, 1ull);  // slot 0
         }
-        if (pass == 0) {
-            // counts only: integer LDS atomics, so the order does not matter;
-            // the events are counted once per tile
-            if (key != deadkey) atomicAdd(&cnt[key], 1u);
-            n_clamped += clamped;
-            n_dropped += dropped;
-            return;
+        if (tid < 28) {
+            dtab_out[(size_t)T * DIR_WORDS + tid] = seg + goff[mydir << lq];
+        } else if (tid < 30) {
+            dtab_out[(size_t)T * DIR_WORDS + tid] = seg + (tid == DIR_OWN ? 0u : goff[NS << lq]);
+        } else if (tid == 30) {
+            tab_out[(size_t)T * g.kt + K] = seg + total;
         }
-        // tiles divide the grid, so a periodic wrap keeps the local index
-        const uint8_t nlcell = (uint8_t)((di & (g.tx - 1)) + ((dj & (g.ty - 1)) << g.ltx) +
-                                         ((dk & (g.tz - 1)) << (g.ltx + g.lty)));
-        // rank among this wave's lanes holding the same slot
-        unsigned long long match = __ballot(key != deadkey);
-        for (int b = 0; b < kbits; ++b) {
-            const bool bit = (key >> b) & 1u;
-            const unsigned long long bal = __ballot(bit);
-            match &= bit ? bal : ~bal;
+        // places of the segment whose particles are removed
+        for (uint32_t u = total + tid; u < N; u += NT)
+            if (u < places) (D.x + seg)[u] = Real(-1);
+    };
+    auto store = [&](uint32_t dst, const Particle<Real>& q, uint32_t c) {
+        (D.x + seg)[dst] = q.X; (D.y + seg)[dst] = q.Y; (D.z + seg)[dst] = q.Z;
+        (D.vx + seg)[dst] = q.vx; (D.vy + seg)[dst] = q.vy; (D.vz + seg)[dst] = q.vz;
+        (D.lc + seg)[dst] = (uint8_t)(c >> CELL_SHIFT);
+    };
+    if (one) {
+        for (int i = tid; i < (int)N; i += NT) {
+            if (i >= (int)n0) other((uint32_t)i - n0, nq, nlc);
+            Particle<Real> q = nq;
+            const int lc = nlc;
+            const uint32_t u = (uint32_t)(i + NT);
+            if (u < n0) own(u, nq, nlc);  // the next own one is loaded ahead
+            uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, n_clamped, n_dropped);
+            S4[i] = Real4<Real>{{q.X, q.Y, q.Z, q.vx}};
+            S2[i] = Real2<Real>{{q.vy, q.vz}};
+            c = part_code(c, i);
+            c |= atomicAdd(&cnt[c & SLOT_MASK], 1u) << RANK_SHIFT;
+            scode[i] = c;
         }
-        const unsigned long long below = (lane == 0) ? 0ull : (match & ((~0ull) >> (64 - lane)));
-        const uint32_t rin = (uint32_t)__popcll(below);
-        const uint32_t gsz = (uint32_t)__popcll(match);
-        const bool leader = key != deadkey && rin == gsz - 1;
-        if (leader) grp[w * g.extk + key] = (uint8_t)gsz;
         __syncthreads();
-        if (key != deadkey) {
-            uint32_t dst = cnt[key] + rin;  // the slot's next destination index
-            for (int v = 0; v < w; ++v) dst += grp[v * g.extk + key];
-            if (dst < cap) {
-                D.x[dst] = X; D.y[dst] = Y; D.z[dst] = Z;
-                D.vx[dst] = vx; D.vy[dst] = vy; D.vz[dst] = vz;
-                D.lc[dst] = nlcell;
+        const uint32_t total = scan_slots(false);
+        write_tables(total);
+        for (int i = tid; i < (int)N; i += NT) {
+            const uint32_t c = scode[i], s = c & SLOT_MASK;
+            if (s < (uint32_t)KQ) list[loff[s] + (c >> RANK_SHIFT & RANK_MASK_ROUND)] = (uint16_t)i;
+        }
+        __syncthreads();
+        for (int i = tid; i < (int)N; i += NT) {
+            const uint32_t c = scode[i], s = c & SLOT_MASK;
+            uint32_t dst = 0xFFFFu;
+            if (s < (uint32_t)KQ) dst = goff[s] + list_rank(list + loff[s], cnt[s], (uint32_t)i);
+            scode[i] = dst | c >> CELL_SHIFT << 16;
+        }
+        __syncthreads();
+        for (int i = tid; i < (int)N; i += NT) {
+            const uint32_t dst = scode[i] & 0xFFFFu;
+            if (dst != 0xFFFFu) list[dst] = (uint16_t)i;
+        }
+        __syncthreads();
+        for (uint32_t d = tid; d < total; d += NT) {
+            const uint32_t i = list[d];
+            const Real4<Real> a = S4[i];
+            const Real2<Real> b = S2[i];
+            const uint32_t cell = scode[i] >> 16;
+            if (d < places) {
+                (D.x + seg)[d] = a.v[0]; (D.y + seg)[d] = a.v[1]; (D.z + seg)[d] = a.v[2];
+                (D.vx + seg)[d] = a.v[3]; (D.vy + seg)[d] = b.v[0]; (D.vz + seg)[d] = b.v[1];
+                (D.lc + seg)[d] = (uint8_t)cell;
             } else {
                 atomicAdd(counters + C_RANK_OVERFLOW, 1ull);  // slot 0
             }
         }
-        __syncthreads();
-        if (leader) {
-            atomicAdd(&cnt[key], gsz);  // integer: the order of the four waves does not matter
-            grp[w * g.extk + key] = 0;
+    } else {
+        auto any = [&](uint32_t u, Particle<Real>& q, int& lc) {
+            if (u < n0) own(u, q, lc);
+            else other(u - n0, q, lc);
+        };
+        for (uint32_t u = tid; u < N; u += NT) {
+            Particle<Real> q;
+            int lc;
+            any(u, q, lc);
+            const uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, n_clamped, n_dropped);
+            atomicAdd(&cnt[part_code(c, (int)u) & SLOT_MASK], 1u);
         }
         __syncthreads();
-    };
-    for (uint32_t ub = 0; ub < ntot; ub += 2 * PM_THREADS) {
-        chunk(ub, bufA);
-        if (ub + PM_THREADS < ntot) chunk(ub + PM_THREADS, bufB);  // the same for the whole workgroup
-    }
-    __syncthreads();
-    if (pass == 0) {
-        count_events(counters, C_MAX_VI, n_clamped);
-        count_events(counters, C_DROPPED, n_dropped);
-    }
-    if (pass == 0)
-        for (int ec = tid; ec < g.next; ec += PM_THREADS) {
-            const uint4 a = cnt4[2 * ec], b = cnt4[2 * ec + 1];
-            const uint32_t hi = (a.x | a.y | a.z | a.w | b.x | b.y | b.z | b.w) >> 16;
-            if (hi) atomicAdd(counters + C_RANK_OVERFLOW, 1ull);  // slot 0
-            *reinterpret_cast<uint4*>(cnt_tile + ((size_t)T * g.next + ec) * 8) =
-                make_uint4((a.x & 0xFFFFu) | (a.y << 16), (a.z & 0xFFFFu) | (a.w << 16),
-                           (b.x & 0xFFFFu) | (b.y << 16), (b.z & 0xFFFFu) | (b.w << 16));
+        const uint32_t total = scan_slots(true);
+        write_tables(total);
+        __syncthreads();
+        for (int e = tid; e < KT; e += NT) cnt[e] = 0u;
+        __syncthreads();
+        // each round's particles are pushed for their codes, and again to be
+        // written at their places (their input is still in the caches)
+        for (uint32_t ub = 0; ub < N; ub += round) {
+            const int n = (int)min((uint32_t)round, N - ub);
+            uint32_t unused0 = 0, unused1 = 0;
+            for (int i = tid; i < n; i += NT) {
+                Particle<Real> q;
+                int lc;
+                any(ub + i, q, lc);
+                uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, unused0, unused1);
+                c = part_code(c, i);
+                c |= atomicAdd(&cnt[c & SLOT_MASK], 1u) << RANK_SHIFT;
+                scode[i] = c;
+            }
+            __syncthreads();
+            scan_slots(false);
+            __syncthreads();
+            for (int i = tid; i < n; i += NT) {
+                const uint32_t c = scode[i], s = c & SLOT_MASK;
+                if (s < (uint32_t)KQ) list[loff[s] + (c >> RANK_SHIFT & RANK_MASK_ROUND)] = (uint16_t)i;
+            }
+            __syncthreads();
+            for (int i = tid; i < n; i += NT) {
+                const uint32_t s = scode[i] & SLOT_MASK;
+                if (s >= (uint32_t)KQ) continue;
+                Particle<Real> q;
+                int lc;
+                any(ub + i, q, lc);
+                const uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, unused0, unused1);
+                const uint32_t dst = goff[s] + list_rank(list + loff[s], cnt[s], (uint32_t)i);
+                if (dst < places) {
+                    store(dst, q, c);
+                } else {
+                    atomicAdd(counters + C_RANK_OVERFLOW, 1ull);  // slot 0
+                }
+            }
+            __syncthreads();
+            for (int e = tid; e < KT; e += NT) {
+                if (e < KQ) goff[e] += cnt[e];
+                cnt[e] = 0u;
+            }
+            for (int e = tid; e < (round + KT) / 2; e += NT) reinterpret_cast<uint32_t*>(list)[e] = ~0u;
+            __syncthreads();
         }
+    }
+    count_events(counters, C_MAX_VI, n_clamped);
+    count_events(counters, C_DROPPED, n_dropped);
 }
 
-// Number of particles arriving in each subcell: the slot counts of every tile
-// whose extended region holds the cell, in a fixed order (out = totals, to be
-// scanned into the subcells' first destination index); the slot counts are
-// replaced by each slot's offset inside its subcell's range.  One thread per
-// cell: a cell's eight octant slots are eight consecutive 16-bit entries of
-// every candidate tile's table, read and written as one 16-byte vector.
 // axis_candidates for an axis with at least three tiles or without wrap: the
 // previous tile (cell on the tile's low face), the own tile, the next tile
 // (cell on the high face), in that order.
-__device__ __forceinline__ int axis_candidates_fast(int i, int lt, int nt, int per, int* tl, int* el) {
-    const int t = 1 << lt, t0 = i >> lt, l = i & (t - 1);
+__device__ __forceinline__ int axis_candidates_fast(int i, int n, int lt, int nt, int per, int* tl, int* el) {
+    const int t0 = i >> lt, l = i - (t0 << lt);
     int m = 0;
-    if (l == 0 && (t0 > 0 || per)) { tl[m] = t0 > 0 ? t0 - 1 : nt - 1; el[m++] = t + 1; }
+    if (l == 0 && (t0 > 0 || per)) { tl[m] = t0 > 0 ? t0 - 1 : nt - 1; el[m] = tile_width(n, lt, tl[m]) + 1; ++m; }
     tl[m] = t0; el[m++] = l + 1;
-    if (l == t - 1 && (t0 < nt - 1 || per)) { tl[m] = t0 < nt - 1 ? t0 + 1 : 0; el[m++] = 0; }
+    if (l == tile_width(n, lt, t0) - 1 && (t0 < nt - 1 || per)) { tl[m] = t0 < nt - 1 ? t0 + 1 : 0; el[m++] = 0; }
     return m;
-}
-
-// The slot offsets of one candidate (eight packed 16-bit counts) before its
-// counts are added to the running totals.
-__device__ __forceinline__ uint4 slot_offsets8(uint32_t (&run)[8], uint4 v) {
-    const uint4 off = make_uint4((run[0] & 0xFFFFu) | (run[1] << 16), (run[2] & 0xFFFFu) | (run[3] << 16),
-                                 (run[4] & 0xFFFFu) | (run[5] << 16), (run[6] & 0xFFFFu) | (run[7] << 16));
-    run[0] += v.x & 0xFFFFu; run[1] += v.x >> 16; run[2] += v.y & 0xFFFFu; run[3] += v.y >> 16;
-    run[4] += v.z & 0xFFFFu; run[5] += v.z >> 16; run[6] += v.w & 0xFFFFu; run[7] += v.w >> 16;
-    return off;
-}
-
-constexpr int SLOT_THREADS = 256;
-
-__global__ __launch_bounds__(SLOT_THREADS) void k_slot_offsets(Geom g, uint16_t* __restrict__ cnt_tile,
-                                                              const uint8_t* __restrict__ live,
-                                                              uint32_t* __restrict__ out,
-                                                              unsigned long long* __restrict__ counters) {
-    // blocks dealt to the XCDs in contiguous ranges (slab order): a tile's
-    // slot table is read by its own cells and its neighbours' face cells
-    const uint32_t nb = ((uint32_t)g.ntiles * (uint32_t)g.tc + SLOT_THREADS - 1) / SLOT_THREADS;
-    const uint32_t blk = (uint32_t)xcd_index((int)nb, (int)blockIdx.x);
-    if (blk >= nb) return;
-    const uint32_t id = blk * (uint32_t)SLOT_THREADS + threadIdx.x;  // = tile * tc + local cell
-    if (id >= (uint32_t)g.ntiles * (uint32_t)g.tc) return;
-    const int T = (int)(id >> (g.ltx + g.lty + g.ltz)), lc = (int)(id & (uint32_t)(g.tc - 1));
-    int li, lj, lk;
-    local_ijk(g, lc, li, lj, lk);
-    const int i = ((T % g.ntx) << g.ltx) + li, j = (((T / g.ntx) % g.nty) << g.lty) + lj,
-              k = ((T / (g.ntx * g.nty)) << g.ltz) + lk;
-    int tx[6], ex[6], ty[6], ey[6], tz[6], ez[6];
-    const bool fx = !g.per[0] || g.ntx >= 3, fy = !g.per[1] || g.nty >= 3, fz = !g.per[2] || g.ntz >= 3;
-    uint4* tab = reinterpret_cast<uint4*>(cnt_tile);  // [tile][extended cell]: eight octant slots
-    uint32_t run[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-    if (fx && fy && fz && g.tx >= 2 && g.ty >= 2 && g.tz >= 2) {
-        // tile sides >= 2: a cell is on at most one face of its tile per
-        // axis, so at most two candidates per axis; all eight loads are
-        // issued before the ordered accumulation (32-bit slot offsets: the
-        // context rejects tilings whose slot table has 2^32 entries or more)
-        const int mx = axis_candidates_fast(i, g.ltx, g.ntx, g.per[0], tx, ex);
-        const int my = axis_candidates_fast(j, g.lty, g.nty, g.per[1], ty, ey);
-        const int mz = axis_candidates_fast(k, g.ltz, g.ntz, g.per[2], tz, ez);
-        // (an empty candidate tile has no slot table: it adds nothing)
-        uint32_t slot[8];
-        uint4 v[8];
-        bool use[8];
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-            for (int b = 0; b < 2; ++b)
-#pragma unroll
-                for (int a = 0; a < 2; ++a) {
-                    const int q = a + 2 * b + 4 * c;
-                    const bool inb = a < mx && b < my && c < mz;
-                    const int TT = inb ? tx[a] + g.ntx * (ty[b] + g.nty * tz[c]) : T;
-                    use[q] = inb && live[TT];
-                    slot[q] = (uint32_t)TT * (uint32_t)g.next + (uint32_t)(inb ? ex[a] + g.ex * (ey[b] + g.ey * ez[c]) : 0);
-                    v[q] = use[q] ? tab[slot[q]] : make_uint4(0u, 0u, 0u, 0u);
-                }
-#pragma unroll
-        for (int q = 0; q < 8; ++q)
-            if (use[q]) tab[slot[q]] = slot_offsets8(run, v[q]);  // offsets inside the subcells' ranges
-    } else {
-        const int mx = fx ? axis_candidates_fast(i, g.ltx, g.ntx, g.per[0], tx, ex)
-                          : axis_candidates(i, g.nx, g.ltx, g.ntx, g.per[0], tx, ex);
-        const int my = fy ? axis_candidates_fast(j, g.lty, g.nty, g.per[1], ty, ey)
-                          : axis_candidates(j, g.ny, g.lty, g.nty, g.per[1], ty, ey);
-        const int mz = fz ? axis_candidates_fast(k, g.ltz, g.ntz, g.per[2], tz, ez)
-                          : axis_candidates(k, g.nz, g.ltz, g.ntz, g.per[2], tz, ez);
-        for (int c = 0; c < mz; ++c)
-            for (int b = 0; b < my; ++b)
-                for (int a = 0; a < mx; ++a) {
-                    const int TT = tx[a] + g.ntx * (ty[b] + g.nty * tz[c]);
-                    if (!live[TT]) continue;
-                    const size_t slot = (size_t)TT * g.next + (size_t)(ex[a] + g.ex * (ey[b] + g.ey * ez[c]));
-                    tab[slot] = slot_offsets8(run, tab[slot]);
-                }
-    }
-    uint4* o4 = reinterpret_cast<uint4*>(out + (size_t)id * 8);
-    o4[0] = make_uint4(run[0], run[1], run[2], run[3]);
-    o4[1] = make_uint4(run[4], run[5], run[6], run[7]);
-    if ((run[0] | run[1] | run[2] | run[3] | run[4] | run[5] | run[6] | run[7]) > 0xFFFFu)
-        atomicAdd(counters + C_RANK_OVERFLOW, 1ull);  // offsets are 16-bit
 }
 
 // Exclusive scan of uint32 counts (three passes: block sums, scan of the block
@@ -679,10 +1100,11 @@ __device__ __forceinline__ void cic_accumulate2(Real (&acc)[2][8], bool hx, bool
 
 // LDS of the deposit: half of the subcell sums (2 quantities x 8 corners) as
 // [quantity*8+corner][octant][cell] (octant blocks of deposit_octant_block
-// words); the first half's results.
+// words); per extended cell four sums, the arrivals' and, on the crowded
+// path, the first half's results.
 template <typename Real>
 RH_HD size_t deposit_lds_bytes(const Geom& g) {
-    return sizeof(Real) * (16 * 8 * (size_t)deposit_octant_block(g) + 2 * (size_t)g.next);
+    return sizeof(Real) * (16 * 8 * (size_t)deposit_octant_block(g) + 4 * (size_t)g.next);
 }
 
 // For every cell of the extended region, the LDS offsets (corner plane,
@@ -806,10 +1228,6 @@ RH_HD int deposit_chunk(const Geom& g) {
     return ((16 * 8 * deposit_octant_block(g)) / 6) & ~63;
 }
 
-template <typename Real>
-struct alignas(4 * sizeof(Real)) Real4 { Real v[4]; };
-template <typename Real>
-struct alignas(2 * sizeof(Real)) Real2 { Real v[2]; };
 
 // The deposit of a crowded tile (k_deposit sends tiles with at least
 // dense_min particles here): eight lanes share a subcell and read eight
@@ -818,9 +1236,9 @@ struct alignas(2 * sizeof(Real)) Real2 { Real v[2]; };
 // subcells per round.  Within the same LDS as the sparse path, the two
 // halves (charge and vx, then vy and vz) each read the particles once.
 template <typename Real>
-__device__ void deposit_dense_tile(const Geom& g, const PArrays<Real>& A, const uint32_t* __restrict__ sub,
+__device__ void deposit_dense_tile(const Geom& g, const PArrays<Real>& A, const uint32_t* __restrict__ tab,
                                    const uint16_t* __restrict__ glist, const uint8_t* __restrict__ gcount,
-                                   Real* __restrict__ partial, int T, Real* S, Real* R) {
+                                   Real* __restrict__ partial, int T, Real* S, Real4<Real>* R) {
     const int NS = g.tc * 8;
     const int OB = deposit_octant_block(g);
     const int QS = 8 * OB;
@@ -831,8 +1249,7 @@ __device__ void deposit_dense_tile(const Geom& g, const PArrays<Real>& A, const 
         for (int base = 0; base < NS; base += ngrp) {
             const int ls = base + grp;
             const bool valid = ls < NS;
-            const uint32_t key = (uint32_t)(T * NS + (valid ? ls : 0));
-            const uint32_t p0 = valid ? sub[key] : 0u, p1 = valid ? sub[key + 1] : 0u;
+            const uint32_t p0 = valid ? tab[ls] : 0u, p1 = valid ? tab[ls + 1] : 0u;
             const int o = ls & 7, cell = ls >> 3;
             const bool hx = o & 1, hy = (o >> 1) & 1, hz = (o >> 2) & 1;
             Real acc[2][8];
@@ -873,35 +1290,97 @@ __device__ void deposit_dense_tile(const Geom& g, const PArrays<Real>& A, const 
                     res[1] += S[8 * QS + off];
                 }
             }
-            if (half == 0) {
-                R[2 * e] = res[0];
-                R[2 * e + 1] = res[1];
-            } else {
-                Real4<Real> r;
-                r.v[0] = R[2 * e]; r.v[1] = R[2 * e + 1]; r.v[2] = res[0]; r.v[3] = res[1];
-                out[e] = r;
-            }
+            R[e].v[2 * half] += res[0];
+            R[e].v[2 * half + 1] += res[1];
+            if (half) out[e] = R[e];
         }
     }
 }
 
+// The arrivals of a crowded tile, which wait in its neighbours' segments: every wave
+// takes a contiguous part of the sequence and adds each particle's weights
+// times (1, vx, vy, vz) to sums of its own over the extended region (in LDS,
+// where the particle staging comes later): lane = corner + 8 * quantity, so
+// the 32 targets of one particle are distinct words and need no atomics.  The
+// waves' sums are then added in order into R.
 template <typename Real>
-__global__ __launch_bounds__(512) void k_deposit(Geom g, PArrays<Real> A, const uint32_t* __restrict__ sub,
+__device__ void deposit_arrivals(const Geom& g, const PArrays<Real>& A, const uint32_t* lists,
+                                 Real* S, Real4<Real>* R) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const uint32_t na = lists[LIST_PREF + 27];
+    const int nwaves = ((int)blockDim.x + 63) >> 6;
+    const int room = 16 * 8 * deposit_octant_block(g) / (4 * g.next);  // copies of the region that fit
+    const int nw = nwaves < room ? nwaves : room;
+    for (int e = tid; e < nw * 4 * g.next; e += blockDim.x) S[e] = Real(0);
+    __syncthreads();
+    const int nl = blockDim.x < 64 ? (int)blockDim.x : 64;  // lanes of this wave (8 to 64)
+    if (w < nw) {
+        Real* mine = S + (size_t)w * 4 * g.next;
+        const uint32_t v0 = (uint32_t)((uint64_t)na * w / nw), v1 = (uint32_t)((uint64_t)na * (w + 1) / nw);
+        for (uint32_t vb = v0; vb < v1; vb += nl) {
+            Real X = Real(-1), Y = Real(0), Z = Real(0), vx = Real(0), vy = Real(0), vz = Real(0);
+            int lc = 0;
+            if (vb + lane < v1) {
+                const uint32_t p = arrival_index(lists, vb + lane);
+                X = A.x[p]; Y = A.y[p]; Z = A.z[p];
+                vx = A.vx[p]; vy = A.vy[p]; vz = A.vz[p];
+                lc = A.lc[p];
+            }
+            const int n = (int)min((uint32_t)nl, v1 - vb);
+            for (int i = 0; i < n; ++i) {
+                const Real x = __shfl(X, i), y = __shfl(Y, i), z = __shfl(Z, i);
+                const Real f[4] = {Real(1), __shfl(vx, i), __shfl(vy, i), __shfl(vz, i)};
+                const int l = __shfl(lc, i);
+                if (x < Real(0)) continue;  // removed (the same for the whole wave)
+                int li, lj, lk;
+                local_ijk(g, l, li, lj, lk);
+                const int hx = x >= Real(0.5), hy = y >= Real(0.5), hz = z >= Real(0.5);
+                const Real wx1 = hx ? x - Real(0.5) : x + Real(0.5);
+                const Real wy1 = hy ? y - Real(0.5) : y + Real(0.5);
+                const Real wz1 = hz ? z - Real(0.5) : z + Real(0.5);
+                for (int t = lane; t < 32; t += nl) {
+                    const int kx = t & 1, ky = (t >> 1) & 1, kz = (t >> 2) & 1, qt = t >> 3;
+                    const Real wt = (kx ? wx1 : Real(1) - wx1) * (ky ? wy1 : Real(1) - wy1) * (kz ? wz1 : Real(1) - wz1);
+                    const int e = (li + kx + hx) + g.ex * ((lj + ky + hy) + g.ey * (lk + kz + hz));
+                    mine[4 * e + qt] += wt * (qt == 0 ? f[0] : (qt == 1 ? f[1] : (qt == 2 ? f[2] : f[3])));
+                }
+            }
+        }
+    }
+    __syncthreads();
+    Real* Rw = reinterpret_cast<Real*>(R);
+    for (int e = tid; e < 4 * g.next; e += blockDim.x) {
+        Real s = Real(0);
+        for (int q = 0; q < nw; ++q) s += S[(size_t)q * 4 * g.next + e];
+        Rw[e] = s;
+    }
+    __syncthreads();
+}
+
+template <typename Real>
+__global__ __launch_bounds__(512) void k_deposit(Geom g, PArrays<Real> A, const uint32_t* __restrict__ tabs,
+                                                 const uint32_t* __restrict__ lists,
                                                  const uint16_t* __restrict__ glist,
                                                  const uint8_t* __restrict__ gcount,
                                                  const uint16_t* __restrict__ tlist,
                                                  const uint8_t* __restrict__ tcount, Real* __restrict__ partial,
                                                  uint32_t dense_min) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ uint32_t L[LIST_WORDS];
     const int NS = g.tc * 8;
     const int OB = deposit_octant_block(g);  // octant block (padded)
     const int QS = 8 * OB;            // one (quantity, corner) plane
     Real* S = reinterpret_cast<Real*>(smem_raw);
-    Real* R = S + 16 * QS;  // first-half results, next x 2
+    // per extended cell four words: the crowded path's arrivals' sums, or
+    // this path's arrivals by subcell (below)
+    Real4<Real>* R = reinterpret_cast<Real4<Real>*>(S + 16 * QS);
     const int T = xcd_tile(g, (int)blockIdx.x);
     if (T >= g.ntiles) return;
-    const uint32_t t0 = sub[(size_t)T * NS], t1 = sub[(size_t)(T + 1) * NS];
-    if (t1 == t0) {
+    const uint32_t* tab = tabs + (size_t)T * g.kt;
+    const int ls = threadIdx.x;
+    const uint32_t t0 = lists[(size_t)T * LIST_WORDS + LIST_OWN], n0 = lists[(size_t)T * LIST_WORDS + LIST_OWN + 1];
+    const uint32_t na = lists[(size_t)T * LIST_WORDS + LIST_PREF + 27], t1 = t0 + n0;
+    if (n0 == 0 && na == 0) {
         // an empty tile: zero ghost partials (the fold reads every tile's;
         // a per-tile flag that let the fold skip them cost it more, 35 -> 45
         // us on the dense box, than the zero stores cost here)
@@ -911,13 +1390,20 @@ __global__ __launch_bounds__(512) void k_deposit(Geom g, PArrays<Real> A, const 
         for (int e = threadIdx.x; e < g.next; e += blockDim.x) out[e] = z;
         return;
     }
-    if (t1 - t0 >= dense_min) {
-        deposit_dense_tile(g, A, sub, glist, gcount, partial, T, S, R);
+    uint32_t p0 = 0, p1 = 0;
+    if (n0) { p0 = tab[ls]; p1 = tab[ls + 1]; }
+    for (int e = ls; e < LIST_WORDS; e += blockDim.x) L[e] = lists[(size_t)T * LIST_WORDS + e];
+    if (n0 >= dense_min) {
+        if (na) {
+            __syncthreads();
+            deposit_arrivals(g, A, L, S, R);
+        } else {
+            Real* Rw = reinterpret_cast<Real*>(R);
+            for (int e = ls; e < 4 * g.next; e += blockDim.x) Rw[e] = Real(0);
+        }
+        deposit_dense_tile(g, A, tab, glist, gcount, partial, T, S, R);
         return;
     }
-    const int ls = threadIdx.x;
-    const uint32_t key = (uint32_t)(T * NS + ls);
-    const uint32_t p0 = sub[key], p1 = sub[key + 1];
     const int o = ls & 7, cell = ls >> 3;
     const bool hx = o & 1, hy = (o >> 1) & 1, hz = (o >> 2) & 1;
     Real acc[4][8];
@@ -925,29 +1411,56 @@ __global__ __launch_bounds__(512) void k_deposit(Geom g, PArrays<Real> A, const 
     for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int c = 0; c < 8; ++c) acc[q][c] = Real(0);
-    // The tile's particles go through LDS in chunks read with coalesced
-    // loads; each thread then takes its subcell's particles of the chunk, in
-    // particle order (the same sums as reading them directly).  A particle is
+    // The tile's particles, its own and then its arrivals, go through LDS in
+    // chunks (its own read with coalesced loads); each thread then takes its
+    // subcell's particles of the chunk, in particle order.  A particle is
     // staged as (x, y, z, vx) and (vy, vz): two LDS reads instead of six.
+    // The arrivals, about 2 % of the particles, are linked by subcell as they
+    // are staged; a thread takes the few of its list in ascending order, in
+    // the same loop as its own particles, so that a wave runs hardly longer.
+    // The first of a thread's arrivals is loaded ahead.
     const int CH = deposit_chunk<Real>(g);
     Real4<Real>* L4 = reinterpret_cast<Real4<Real>*>(S);          // x, y, z, vx
     Real2<Real>* L2 = reinterpret_cast<Real2<Real>*>(S + 4 * CH);  // vy, vz
-    for (uint32_t cs = t0; cs < t1; cs += (uint32_t)CH) {
-        const int n = (int)min((uint32_t)CH, t1 - cs);
+    constexpr uint32_t NONE = 0xFFFFu;
+    uint32_t* head = reinterpret_cast<uint32_t*>(R);               // per subcell its list's first entry
+    uint16_t* next = reinterpret_cast<uint16_t*>(head + NS);       // per arrival of the chunk the next one
+    const uint32_t AR = (uint32_t)((4 * sizeof(Real) * g.next - 4 * (size_t)NS) / 2);  // arrivals of one chunk
+    head[ls] = NONE;
+    uint32_t n = 0;
+    for (uint32_t cs = 0; cs < n0 + na; cs += n) {
+        const uint32_t qa = n0 > cs ? n0 - cs : 0u;  // the chunk's first arrival
+        n = min(min((uint32_t)CH, n0 + na - cs), qa + AR);
         __syncthreads();  // the previous chunk is consumed
-        for (int q = ls; q < n; q += blockDim.x) {
-            const uint32_t p = cs + (uint32_t)q;
+        for (uint32_t q = ls; q < n; q += blockDim.x) {
+            const uint32_t p = q < qa ? t0 + cs + q : arrival_index(L, cs + q - n0);
             Real4<Real> r;
             r.v[0] = A.x[p]; r.v[1] = A.y[p]; r.v[2] = A.z[p]; r.v[3] = A.vx[p];
             Real2<Real> t;
             t.v[0] = A.vy[p]; t.v[1] = A.vz[p];
             L4[q] = r;
             L2[q] = t;
+            if (q >= qa) {
+                const int oct = (r.v[0] >= Real(0.5)) + 2 * (r.v[1] >= Real(0.5)) + 4 * (r.v[2] >= Real(0.5));
+                next[q - qa] = (uint16_t)atomicExch(&head[A.lc[p] * 8 + oct], q);
+            }
         }
         __syncthreads();
-        const uint32_t a = max(p0, cs), b = min(p1, cs + (uint32_t)n);
-        for (uint32_t p = a; p < b; ++p) {
-            const int q = (int)(p - cs);
+        const uint32_t a = max(p0, t0 + cs) - t0 - cs, b = min(p1, t0 + cs + n) - t0 - cs;
+        const int own = p1 > t0 + cs && p0 < t0 + cs + n && p1 > p0 ? (int)(b - a) : 0;
+        int m = own;
+        const uint32_t first = head[ls];
+        for (uint32_t h = first; h != NONE; h = next[h - qa]) ++m;
+        head[ls] = NONE;
+        int last = -1;
+        for (int it = 0; it < m; ++it) {
+            int q = (int)a + it;
+            if (it >= own) {
+                int best = 0x7FFFFFFF;
+                for (uint32_t h = first; h != NONE; h = next[h - qa])
+                    if ((int)h > last && (int)h < best) best = (int)h;
+                q = last = best;
+            }
             const Real4<Real> r = L4[q];
             const Real2<Real> t = L2[q];
             cic_accumulate(acc, hx, hy, hz, r.v[0], r.v[1], r.v[2], r.v[3], t.v[0], t.v[1]);
@@ -1012,7 +1525,8 @@ struct FoldSources {
     int n;
 };
 
-template <typename Real>
+// TWO: no cell has more than two candidate tiles along an axis.
+template <typename Real, bool TWO>
 __global__ __launch_bounds__(256) void k_fold(Geom g, FoldSources<Real> src, double inv_dV, double min_rho,
                                              Real* __restrict__ rho, Real* __restrict__ jx, Real* __restrict__ jy,
                                              Real* __restrict__ jz, unsigned long long* __restrict__ counters) {
@@ -1021,14 +1535,13 @@ __global__ __launch_bounds__(256) void k_fold(Geom g, FoldSources<Real> src, dou
     if (i < g.nx && j < g.ny) {
         const int n = cell_index(g, i, j, k);
         int tx[6], ex[6], ty[6], ey[6], tz[6], ez[6];
-        const bool fx = !g.per[0] || g.ntx >= 3, fy = !g.per[1] || g.nty >= 3, fz = !g.per[2] || g.ntz >= 3;
         double s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-        if (fx && fy && fz && g.tx >= 2 && g.ty >= 2 && g.tz >= 2) {
+        if constexpr (TWO) {
             // at most two candidate tiles per axis: all eight loads of a
             // species issued before its sum (the same order as below)
-            const int mx = axis_candidates_fast(i, g.ltx, g.ntx, g.per[0], tx, ex);
-            const int my = axis_candidates_fast(j, g.lty, g.nty, g.per[1], ty, ey);
-            const int mz = axis_candidates_fast(k, g.ltz, g.ntz, g.per[2], tz, ez);
+            const int mx = axis_candidates_fast(i, g.nx, g.ltx, g.ntx, g.per[0], tx, ex);
+            const int my = axis_candidates_fast(j, g.ny, g.lty, g.nty, g.per[1], ty, ey);
+            const int mz = axis_candidates_fast(k, g.nz, g.ltz, g.ntz, g.per[2], tz, ez);
             for (int s = 0; s < src.n; ++s) {
                 const Real4<Real>* part = reinterpret_cast<const Real4<Real>*>(src.partial[s]);
                 Real4<Real> v[8];
@@ -1133,35 +1646,58 @@ constexpr int BC_CELLS_PER_BLOCK = 256 / BC_LANES;
 // / Impact and their kinetic energies, :121-122,153-154): per listed cell,
 // acc[4q..4q+3] += (escapes, sum v^2 of escapes, impacts, sum v^2 of
 // impacts), summed over the cell's lanes in a fixed butterfly.
+// rng[beg[q] .. beg[q+1]-1]: where the cell's particles may be, its own
+// subcells' range first, then the halo slots of neighbouring tiles that it
+// is: the tile and the table entry, which are the same in every step.
+struct CellRange {
+    int tile;
+    uint32_t entry;
+};
 template <typename Real>
 __global__ __launch_bounds__(256) void k_boundary(Geom g, const int* __restrict__ cells, int ncells,
-                                                 const uint32_t* __restrict__ sub, PArrays<Real> A,
+                                                 const int* __restrict__ beg, const CellRange* __restrict__ rng,
+                                                 TileTables tt, PArrays<Real> A,
                                                  double R2, double* __restrict__ acc) {
     const int q = blockIdx.x * BC_CELLS_PER_BLOCK + (int)(threadIdx.x / BC_LANES);
     const int lane = threadIdx.x & (BC_LANES - 1);
     const bool valid = q < ncells;
     double c[4] = {0, 0, 0, 0};
     if (valid) {
+        const int b0 = beg[q], nr = tt.lists ? beg[q + 1] - b0 : 1;
+        // up to 16 ranges at a time, one lane each
+        uint32_t r0 = 0, r1 = 0;
+        if (lane < nr) {
+            const CellRange cr = rng[b0 + lane];
+            if (tt.live[cr.tile]) { r0 = tt.tab[cr.entry]; r1 = tt.tab[cr.entry + (lane == 0 ? 8 : 1)]; }
+        }
         const int n = cells[q];
         int i, j, k;
         cell_ijk(g, n, i, j, k);
-        const uint32_t kc = cell_key(g, i, j, k);
-        const uint32_t p0 = sub[(size_t)kc * 8], p1 = sub[(size_t)kc * 8 + 8];
         const bool exterior = !all_nbrs(g, i, j, k);
         const double xb = g.x0 + i * g.dx, yb = g.y0 + j * g.dx, zb = g.z0 + k * g.dx;
-        for (uint32_t p = p0 + lane; p < p1; p += BC_LANES) {
-            if (A.x[p] < Real(0)) continue;
-            const double vx = A.vx[p], vy = A.vy[p], vz = A.vz[p];
-            const double v2 = vx * vx + vy * vy + vz * vz;
-            if (exterior) {
-                A.x[p] = Real(-1);
-                c[0] += 1.0; c[1] += v2;
-                continue;
+        for (int t = 0; t < nr; ++t) {
+            if (t > 0 && (t & (BC_LANES - 1)) == 0) {  // (only cells of tiles one cell wide have more)
+                r0 = r1 = 0;
+                if (t + lane < nr) {
+                    const CellRange cr = rng[b0 + t + lane];
+                    if (tt.live[cr.tile]) { r0 = tt.tab[cr.entry]; r1 = tt.tab[cr.entry + 1]; }
+                }
             }
-            const double x = xb + (double)A.x[p] * g.dx, y = yb + (double)A.y[p] * g.dx, z = zb + (double)A.z[p] * g.dx;
-            if (x * x + y * y + z * z < R2) {
-                A.x[p] = Real(-1);
-                c[2] += 1.0; c[3] += v2;
+            const uint32_t p0 = __shfl(r0, t & (BC_LANES - 1), BC_LANES), p1 = __shfl(r1, t & (BC_LANES - 1), BC_LANES);
+            for (uint32_t p = p0 + lane; p < p1; p += BC_LANES) {
+                if (A.x[p] < Real(0)) continue;
+                const double vx = A.vx[p], vy = A.vy[p], vz = A.vz[p];
+                const double v2 = vx * vx + vy * vy + vz * vz;
+                if (exterior) {
+                    A.x[p] = Real(-1);
+                    c[0] += 1.0; c[1] += v2;
+                    continue;
+                }
+                const double x = xb + (double)A.x[p] * g.dx, y = yb + (double)A.y[p] * g.dx, z = zb + (double)A.z[p] * g.dx;
+                if (x * x + y * y + z * z < R2) {
+                    A.x[p] = Real(-1);
+                    c[2] += 1.0; c[3] += v2;
+                }
             }
         }
     }
@@ -1178,17 +1714,20 @@ __global__ __launch_bounds__(256) void k_boundary(Geom g, const int* __restrict_
 // vz, sum |v|, sum v^2 (unweighted; one weight per species) and max |v|.
 constexpr int DIAG_BLOCKS = 1024;
 constexpr int DIAG_Q = 7;
-// Injected particles waiting past the store's end (*extra of them, extra may
-// be null) are included.
+// Every place of the segments (*end of them; those without a particle are
+// marked), and the injected particles waiting in the appendix (*extra of
+// them, extra may be null, up to the store's capacity) from store index
+// `base`, or from the store's end.
 template <typename Real>
-__global__ __launch_bounds__(256) void k_diag(PArrays<Real> A, const uint32_t* __restrict__ np_ptr,
-                                             const uint32_t* __restrict__ extra, uint32_t cap,
-                                             double* __restrict__ partial) {
+__global__ __launch_bounds__(256) void k_diag(PArrays<Real> A, const uint32_t* __restrict__ scal,
+                                             const uint32_t* __restrict__ extra, uint32_t places, int at_end,
+                                             uint32_t cap, double* __restrict__ partial) {
     __shared__ double red[DIAG_Q][256];
-    uint32_t np = *np_ptr;
-    if (extra) np = (uint64_t)np + *extra > cap ? cap : np + *extra;
+    const uint32_t np = scal[SC_NP], end = scal[SC_END], room = min(cap > np ? cap - np : 0u, places);
+    const uint32_t nx = extra ? min(*extra, room) : 0u, base = at_end ? np : cap;
     double s[DIAG_Q] = {0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t p = blockIdx.x * 256u + threadIdx.x; p < np; p += 256u * gridDim.x) {
+    for (uint32_t u = blockIdx.x * 256u + threadIdx.x; u < end + nx; u += 256u * gridDim.x) {
+        const uint32_t p = u < end ? u : base + (u - end);
         if (A.x[p] < Real(0)) continue;
         const double vx = A.vx[p], vy = A.vy[p], vz = A.vz[p];
         const double v2 = vx * vx + vy * vy + vz * vz, v = sqrt(v2);

@@ -1,0 +1,71 @@
+"""The push that sorts a tile's particles into its own segment, against the
+FP64 oracle, where its dispatch and its lists change:
+  * tiles that fit their round and tiles that do not (one crowded cell among
+    almost empty ones: the tile is pushed in rounds);
+  * slots split in parts (many particles in a tile of few cells);
+  * wraps: one to four tiles along a periodic axis, where a tile is its
+    own neighbour or the same neighbour on both sides;
+  * a store that is uploaded, stepped, downloaded and uploaded again: its
+    particles are then in their own tiles' segments and stay the same ones.
+FP64 fields are compared with the oracle's to 1e-9 of the global L2 norm (a
+step's operations round in another order: a few hundred units of 1e-16 per
+step), FP32 fields to 1e-5, counts exactly."""
+import numpy as np
+import pytest
+
+from rhybrid_amd import problem as P
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300)
+
+
+def crowded_box(dims, ppc, share, seed):
+    """The periodic box of config_periodic at other sides, with a share of the
+    particles moved into one cell."""
+    base = P.config_periodic(n=max(dims), ppc=ppc, seed=seed)
+    n = max(dims)
+    c = base.particles[0].cell
+    i, j, k = c % n, (c // n) % n, c // (n * n)
+    keep = (i < dims[0]) & (j < dims[1]) & (k < dims[2])
+    cell = (i + dims[0] * (j + dims[1] * k))[keep]
+    pick = np.random.default_rng(seed + 1).random(cell.size) < share
+    cell[pick] = dims[0] * dims[1] * dims[2] // 2
+    base.particles[0] = P.Particles(cell, base.particles[0].state[keep].copy())
+    g = base.grid
+    base.grid = P.Grid(dims[0], dims[1], dims[2], g.periodic, g.dx, g.x0, g.y0, g.z0)
+    base.fields = P.make_fields(base.grid, base.params.imf)
+    base.flags = P.make_flags(base.grid)
+    return base
+
+
+BOXES = [  # cells, tile, particles per cell, share moved into one cell
+    ((8, 4, 4), (2, 2, 2), 200, 0.0),
+    ((8, 8, 8), (4, 4, 4), 24, 0.3),
+    ((4, 4, 4), (1, 1, 1), 40, 0.5),
+    ((4, 8, 12), (4, 4, 4), 16, 0.0),
+    ((6, 4, 4), (2, 2, 2), 300, 0.4),
+]
+
+
+@pytest.mark.parametrize("prec", [1, 0])
+@pytest.mark.parametrize("dims,tile,ppc,share", BOXES)
+def test_push_sort_vs_oracle(gpu_mod, oracle_mod, prec, dims, tile, ppc, share):
+    print("case %s tile %s ppc %d share %g precision %d" % (dims, tile, ppc, share, prec), flush=True)
+    pr = crowded_box(dims, ppc, share, 51)
+    ora = oracle_mod.Oracle(pr)
+    ora.step(3)
+    ctx = gpu_mod.Context(pr, precision=prec, tile=tile)
+    ctx.step(1)
+    for s in range(len(pr.species)):  # the same store by way of the host
+        ctx.upload_particles(s, *ctx.particles(s))
+    ctx.step(2)
+    n = [ctx.num_particles(s) for s in range(len(pr.species))]
+    assert n == [ora.num_particles(s) for s in range(len(pr.species))]
+    for name in ("cellRhoQi", "cellJi", "faceB"):
+        r = rel(ctx.field(name), ora.field(name))
+        print("%s rel L2 %.3e" % (name, r), flush=True)
+        assert r < (1e-9 if prec else 1e-5), (name, r)
+    ctx.close()
