@@ -40,8 +40,8 @@ typedef enum rh_precision { RH_FP32 = 0, RH_FP64 = 1 } rh_precision;
 /* Grid of nx*ny*nz cells including the exterior layer of non-periodic
  * dimensions (the LogicallyCartesian grids of the reference's example
  * configs); cubic cells of edge dx; (x0,y0,z0) is the lower corner of cell
- * (0,0,0).  tile[] is the cell tile of the sort and deposit (0 = choose);
- * each must divide its dimension. */
+ * (0,0,0).  tile[] is the cell tile of the sort and deposit (0 = choose; a
+ * given one must divide its dimension, a chosen one may leave partial tiles). */
 typedef struct rh_grid_desc {
     int32_t nx, ny, nz;
     int32_t periodic[3];

@@ -432,19 +432,32 @@ public:
         // the deposit runs one thread per subcell (at most 512) and both
         // per-tile kernels keep their tile in LDS
         const int max_cells = 64;
-        if (t[0] <= 0 || t[1] <= 0 || t[2] <= 0) {
+        const bool chosen = t[0] <= 0 || t[1] <= 0 || t[2] <= 0;
+        if (chosen) {
+            // The last tile of an axis may be partial, with cells that do not
+            // exist up to a quarter of the axis: tiles of one or two cells
+            // send most of their particles to neighbours, and have many more
+            // halo cells (75x54x49 with 24 particles per cell: 458 us a step
+            // in 2x4x4 tiles, 480 in 2x2x4, 1,520 in the 1x2x1 that divide it).
+            auto padded = [&](int d) { return (dims[d] + t[d] - 1) / t[d] * t[d]; };
             for (int d = 0; d < 3; ++d) {
                 t[d] = 4;
-                while (t[d] > 1 && dims[d] % t[d]) t[d] /= 2;
+                while (t[d] > 1 && 4 * padded(d) > 5 * dims[d]) t[d] /= 2;
             }
-            auto ntiles = [&]() { return (dims[0] / t[0]) * (dims[1] / t[1]) * (dims[2] / t[2]); };
+            auto ntiles = [&]() {
+                return (dims[0] + t[0] - 1) / t[0] * ((dims[1] + t[1] - 1) / t[1]) * ((dims[2] + t[2] - 1) / t[2]);
+            };
             while (t[0] * t[1] * t[2] > max_cells || (t[0] * t[1] * t[2] > 1 && tile_lds_bytes(t) > lds_limit)) {
                 int d = 0;
                 for (int q = 1; q < 3; ++q) if (t[q] > t[d]) d = q;
                 t[d] /= 2;
             }
-            // enough tiles to fill the chip when the grid is small
-            while (ntiles() < 8192) {
+            // Enough tiles for eight turns of two workgroups a CU when the
+            // grid is small (64x32x32 with 256 particles per cell and species:
+            // 1,025 us a step with 8,192 tiles of 2x2x2 cells, 1,125 with 4,096
+            // of 2x2x4; the other way round with more tiles than that:
+            // 64x48x48 491 us with 4,608 of 2x4x4, 503 with 9,216 of 2x2x4).
+            while (ntiles() <= 4096) {
                 int d = -1;
                 for (int q = 0; q < 3; ++q)
                     if (t[q] > 2 && (d < 0 || t[q] > t[d])) d = q;
@@ -453,7 +466,7 @@ public:
             }
         }
         for (int d = 0; d < 3; ++d)
-            if (t[d] < 1 || (t[d] & (t[d] - 1)) || dims[d] % t[d])
+            if (t[d] < 1 || (t[d] & (t[d] - 1)) || (!chosen && dims[d] % t[d]))
                 throw ArgError("tile sides must be powers of two that divide the grid");
         if (t[0] * t[1] * t[2] > max_cells) throw ArgError("tile has more than 64 cells");
         if (tile_lds_bytes(t) > lds_limit)
@@ -462,7 +475,7 @@ public:
         g.tx = t[0]; g.ty = t[1]; g.tz = t[2];
         g.ltx = __builtin_ctz(g.tx); g.lty = __builtin_ctz(g.ty); g.ltz = __builtin_ctz(g.tz);
         g.tc = g.tx * g.ty * g.tz;
-        g.ntx = g.nx / g.tx; g.nty = g.ny / g.ty; g.ntz = g.nz / g.tz;
+        g.ntx = (g.nx + g.tx - 1) / g.tx; g.nty = (g.ny + g.ty - 1) / g.ty; g.ntz = (g.nz + g.tz - 1) / g.tz;
         g.ntiles = g.ntx * g.nty * g.ntz;
         xcd_bricks(g);
         g.ex = g.tx + 2; g.ey = g.ty + 2; g.ez = g.tz + 2;

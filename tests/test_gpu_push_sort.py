@@ -5,6 +5,8 @@ FP64 oracle, where its dispatch and its lists change:
   * slots split in parts (many particles in a tile of few cells);
   * wraps: one to four tiles along a periodic axis, where a tile is its
     own neighbour or the same neighbour on both sides;
+  * tiles of which only a part lies in the grid (sides that no power of two
+    divides, the context's own choice of tiles), periodic and with walls;
   * a store that is uploaded, stepped, downloaded and uploaded again: its
     particles are then in their own tiles' segments and stay the same ones.
 FP64 fields are compared with the oracle's to 1e-9 of the global L2 norm (a
@@ -47,6 +49,8 @@ BOXES = [  # cells, tile, particles per cell, share moved into one cell
     ((4, 4, 4), (1, 1, 1), 40, 0.5),
     ((4, 8, 12), (4, 4, 4), 16, 0.0),
     ((6, 4, 4), (2, 2, 2), 300, 0.4),
+    ((7, 11, 13), (0, 0, 0), 12, 0.0),
+    ((13, 9, 7), (0, 0, 0), 12, 0.2),
 ]
 
 
@@ -64,6 +68,31 @@ def test_push_sort_vs_oracle(gpu_mod, oracle_mod, prec, dims, tile, ppc, share):
     ctx.step(2)
     n = [ctx.num_particles(s) for s in range(len(pr.species))]
     assert n == [ora.num_particles(s) for s in range(len(pr.species))]
+    for name in ("cellRhoQi", "cellJi", "faceB"):
+        r = rel(ctx.field(name), ora.field(name))
+        print("%s rel L2 %.3e" % (name, r), flush=True)
+        assert r < (1e-9 if prec else 1e-5), (name, r)
+    ctx.close()
+
+
+@pytest.mark.parametrize("prec", [1, 0])
+@pytest.mark.parametrize("dims", [(19, 14, 11), (15, 23, 9), (31, 13, 25)])
+def test_partial_tiles_obstacle_inflow(gpu_mod, oracle_mod, prec, dims):
+    print("case %s precision %d" % (dims, prec), flush=True)
+    pr = P.config_obstacle(nx=dims[0], ny=dims[1], nz=dims[2], ppc=8, R_cells=2.2, seed=53, inflow=True)
+    for sp in pr.species:
+        sp.capacity = 2 * pr.particles[0].n
+    ora = oracle_mod.Oracle(pr)
+    ora.step(6)
+    ctx = gpu_mod.Context(pr, precision=prec)
+    lay = ctx.layout()
+    assert any(n % t for n, t in zip(dims, (lay["tx"], lay["ty"], lay["tz"])))
+    ctx.step(3)
+    ctx.step(3)
+    for s in range(len(pr.species)):
+        assert abs(ctx.num_particles(s) - ora.num_particles(s)) <= (0 if prec else 1)
+        cell, _ = ctx.particles(s)
+        assert len(cell) == ctx.num_particles(s)
     for name in ("cellRhoQi", "cellJi", "faceB"):
         r = rel(ctx.field(name), ora.field(name))
         print("%s rel L2 %.3e" % (name, r), flush=True)
