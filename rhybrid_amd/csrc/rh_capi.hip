@@ -24,6 +24,7 @@
 #include "rh_geom.hpp"
 #include "rh_inject.hpp"
 #include "rh_log.hpp"
+#include "rh_readback.hpp"
 #include "rh_vlsv.hpp"
 #include "rh_particles.hpp"
 
@@ -325,6 +326,8 @@ public:
         RH_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         ls = stream;
         RH_HIP(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming));
+        RH_HIP(hipHostMalloc(&staging, READBACK_SLOTS * READBACK_SLOT_BYTES, hipHostMallocDefault));
+        for (auto& e : staging_ev) RH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         for (int f = 0; f < RH_N_FIELDS; ++f) {
             fld[f].alloc((size_t)g.nc * FIELD_DIM[f]);
             fill(fld[f].p, Real(0), fld[f].n);
@@ -408,6 +411,8 @@ public:
             for (auto& pe : t.second.pending) { (void)hipEventDestroy(pe.e0); (void)hipEventDestroy(pe.e1); }
         for (auto e : event_pool) (void)hipEventDestroy(e);
         if (fork_ev) (void)hipEventDestroy(fork_ev);
+        for (auto e : staging_ev) if (e) (void)hipEventDestroy(e);
+        if (staging) (void)hipHostFree(staging);
         sp.clear();
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -725,11 +730,23 @@ public:
     void download_field(int id, double* data) override {
         if (id < 0 || id >= RH_N_FIELDS || !data) throw ArgError("bad field id or null data");
         const int dim = FIELD_DIM[id];
-        std::vector<Real> h((size_t)g.nc * dim);
-        RH_HIP(hipMemcpyAsync(h.data(), fld[id].p, h.size() * sizeof(Real), hipMemcpyDeviceToHost, stream));
-        RH_HIP(hipStreamSynchronize(stream));
-        for (int l = 0; l < dim; ++l)
-            for (int n = 0; n < g.nc; ++n) data[(size_t)n * dim + l] = (double)h[(size_t)l * g.nc + n];
+        const size_t chunk = std::min((size_t)g.nc, READBACK_SLOT_BYTES / (dim * sizeof(Real)));
+        Real* slot[READBACK_SLOTS];
+        for (int q = 0; q < READBACK_SLOTS; ++q)
+            slot[q] = reinterpret_cast<Real*>(static_cast<char*>(staging) + q * READBACK_SLOT_BYTES);
+        readback<Real>(
+            (size_t)g.nc, dim, data, slot, chunk,
+            [&](size_t c, size_t first, size_t n) {
+                Real* to = slot[c % READBACK_SLOTS];
+                if (n == (size_t)g.nc)  // the planes follow each other
+                    RH_HIP(hipMemcpyAsync(to, fld[id].p, dim * n * sizeof(Real), hipMemcpyDeviceToHost, stream));
+                else
+                    for (int l = 0; l < dim; ++l)
+                        RH_HIP(hipMemcpyAsync(to + l * chunk, fld[id].p + (size_t)l * g.nc + first, n * sizeof(Real),
+                                              hipMemcpyDeviceToHost, stream));
+                RH_HIP(hipEventRecord(staging_ev[c % READBACK_SLOTS], stream));
+            },
+            [&](size_t c) { RH_HIP(hipEventSynchronize(staging_ev[c % READBACK_SLOTS])); });
     }
 
     void upload_flags(int id, const uint8_t* data) override {
@@ -1117,6 +1134,8 @@ public:
         fill(S_.ave_v.p, 0.0, S_.ave_v.n);
     }
 
+    void* staging = nullptr;  // download_field's pinned ring
+    hipEvent_t staging_ev[READBACK_SLOTS] = {};
     DevBuf<float> dn_in, dn_out, dn_filt;  // denoiser volumes, filtered density (allocated on first use)
     DevBuf<uint32_t> pf_tile;     // push fields, one block per tile (k_push_fields)
     bool pf_dirty = true;         // fields changed since the blocks were written
