@@ -20,11 +20,11 @@
 //    FP32 residual (last layer).
 //  * backward-weights (k_wgrad): dW[tap][ci][co] = sum over voxels of
 //    in[v + tap][ci] * G[v][co]: M = 16 input channels, N = 16 output
-//    channels, K = 32 voxels.  The workgroups are persistent; each stages a
-//    16x4x2 voxel tile transposed into LDS (channel-major, three copies of
-//    the input shifted by dx = -1, 0, +1 so that every 8-voxel K run is one
-//    aligned 16-byte read) and keeps its taps' partial sums in registers;
-//    k_wgrad_reduce adds the per-workgroup partials in a fixed order.
+//    channels, K = 32 voxels.  The workgroups are persistent; each stages
+//    16x4x4 voxel tiles into LDS as they lie in memory (channels last), reads
+//    the fragments' voxel runs with LDS transpose reads, and keeps its taps'
+//    partial sums in registers; k_wgrad_reduce adds the per-workgroup
+//    partials in a fixed order.
 //
 // Fragment lane layouts (checked on the device): for 16x16x32, lane l holds
 // A[l%16][8*(l/16) .. +7], B[8*(l/16) .. +7][l%16] and D[4*(l/16) + i][l%16].
@@ -48,9 +48,7 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
-constexpr int TX = 16, TY = 4, TZ = 4;             // forward output tile
-constexpr int HX = TX + 2, HY = TY + 2, HZ = TZ + 2;
-constexpr int HV = HX * HY * HZ;
+constexpr int TX = 16, HX = TX + 2;  // x extent of a convolution's output tile, and with its halo
 constexpr int NTAP = 27;
 
 struct Layer {
@@ -78,10 +76,10 @@ __device__ __forceinline__ floatx4 mfma(bf16x8 a, bf16x8 b, floatx4 c) {
 // Convolution over zero-padded volumes; CIN in {8, 32}, NT output tiles of 16.
 // A workgroup computes a 16x4xTZ_ tile, one wave per z plane (TZ_ = 4 or 8:
 // the taller tile stages 10 halo planes for 8 output planes instead of 6 for 4).
-template <int CIN, int NT, int EP, int TZ_>
+template <int CIN, int NT, int EP, int TY, int TZ_>
 __global__ __launch_bounds__(64 * TZ_) void k_conv(ConvArgs a) {
     constexpr int CH = CIN / 8;  // 16-byte chunks per voxel
-    constexpr int HZ_ = TZ_ + 2, HV_ = HX * HY * HZ_, NTH = 64 * TZ_;
+    constexpr int HY = TY + 2, HZ_ = TZ_ + 2, HV_ = HX * HY * HZ_, NTH = 64 * TZ_;
     __shared__ bf16x8 tile[HV_ * CH];
     // the first weight group of the 32-channel path, loaded while the halo is staged
     bf16x8 bnx[3][NT];
@@ -214,22 +212,49 @@ __global__ __launch_bounds__(64 * TZ_) void k_conv(ConvArgs a) {
 }
 
 // Backward-weights.  CIN, COUT = channels of the layer input and of G
-// (8 or 32); tiles of 16x4x2 output voxels; each wave owns the taps
-// w, w+4, ... and all (ci, co) tiles of them.
-constexpr int WX = 16, WY = 4, WZ = 2, WK = WX * WY * WZ;  // 128 voxels = 4 K steps
-constexpr int WHY = WY + 2, WHZ = WZ + 2;
-constexpr int WTAPS = 7;  // taps per wave (27 = 7+7+7+6)
+// (8 or 32); tiles of 16x4x4 output voxels, eight waves: wave w owns the taps
+// w%4, w%4+4, ... with all their (ci, co) tiles, over the planes 2*(w/4) and
+// 2*(w/4)+1.
+//
+// Both operands are needed with voxels along K and lie in memory with
+// channels along it; ds_read_b64_tr_b16 turns 4 voxels x 16 channels while
+// reading, so a tile is staged as it is (one 16-byte LDS write per 8 channels,
+// the next tile's loads in flight meanwhile) and the taps are offsets.  The
+// 16-channel halves lie apart and a row is WPX = 20 voxels long: then a read
+// of two rows meets each bank twice, the least that 512 bytes can.  Bound by
+// LDS reads and MFMA alike (about 2,000 cycles each per tile and CU).
+// 8 volumes of 32^3, 32 -> 32 channels: 26 us; 59 to 67 with a tile transposed by
+// 2-byte LDS writes into three shifted copies, two workgroups of four waves a CU.
+constexpr int WX = 16, WY = 4, WZ = 4, WK = WX * WY * WZ;
+constexpr int WHY = WY + 2, WHZ = WZ + 2, WPX = 20;
+constexpr int WHV = (WX + 2) * WHY * WHZ, WPV = WPX * WHY * WHZ;  // the halo's voxels, with the row padding
+constexpr int WTAPS = 7;       // taps per wave (27 = 7+7+7+6)
+constexpr int WG_THREADS = 512;
+constexpr int WGRAD_BLOCKS = 256;  // persistent workgroups, one per CU
+
+typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
+
+// a fragment's 8 voxels of one channel: the lane addresses voxel (l%16)/4 and
+// channels 4*(l%4).. of the run, and gets channel l%16 of voxels 0-3 and 4-7
+__device__ __forceinline__ bf16x8 read_run(const unsigned char* p, int voxel_bytes) {
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 4 * voxel_bytes));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
 
 template <int CIN, int COUT>
-__global__ __launch_bounds__(256) void k_wgrad(const bf16* __restrict__ in, const bf16* __restrict__ G, int X,
-                                               int Y, int Z, int nvol, float* __restrict__ part) {
-    constexpr int CI = CIN < 16 ? 16 : CIN;   // M extent (padded to a tile)
+__global__ __launch_bounds__(WG_THREADS, 2) void k_wgrad(const bf16* __restrict__ in, const bf16* __restrict__ G, int X,
+                                                         int Y, int Z, int nvol, float* __restrict__ part) {
+    constexpr int CI = CIN < 16 ? 16 : CIN;   // M extent (rows past CIN repeat its channels and are not used)
     constexpr int CO = COUT < 16 ? 16 : COUT; // N extent
     constexpr int MT = CI / 16, NT = CO / 16;
-    // 16-byte fragment reads: both arrays aligned to 16 bytes
-    __shared__ __attribute__((aligned(16))) bf16 Xs[3 * CI * WHZ * WHY * WX];  // [dx][ci][z][y][x]
-    __shared__ __attribute__((aligned(16))) bf16 Gt[CO * WK];                  // [co][voxel]
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    constexpr int BI = CIN < 16 ? 16 : 32, BO = COUT < 16 ? 16 : 32;  // bytes of a voxel's 8 or 16 channels
+    constexpr int CHI = CIN / 8, CHG = COUT / 8;
+    constexpr int X_BYTES = MT * WPV * BI, BUF = X_BYTES + NT * WK * BO;
+    constexpr int ACC_BYTES = 4 * WTAPS * MT * NT * 64 * 16;
+    constexpr int LDS = 2 * BUF > ACC_BYTES ? 2 * BUF : ACC_BYTES;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[LDS];
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), wt = w & 3, wh = w >> 2;
     const int m = lane & 15, kg = lane >> 4;
     const int ntx = X / WX, nty = Y / WY, ntz = Z / WZ;
     const int ntiles = ntx * nty * ntz * nvol;
@@ -241,113 +266,153 @@ __global__ __launch_bounds__(256) void k_wgrad(const bf16* __restrict__ in, cons
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) acc[t][mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // zero the padding channels once (never written by the staging below)
-    for (int idx = threadIdx.x; idx < 3 * CI * WHZ * WHY * WX; idx += blockDim.x) Xs[idx] = (bf16)0.0f;
-    for (int idx = threadIdx.x; idx < CO * WK; idx += blockDim.x) Gt[idx] = (bf16)0.0f;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+    // the thread's 16-byte pieces of a tile
+    constexpr int NI = (WHV * CHI + WG_THREADS - 1) / WG_THREADS, NG = (WK * CHG + WG_THREADS - 1) / WG_THREADS;
+    bf16x8 si[NI], sg[NG];
+    auto load = [&](int tile) {
         int r = tile;
-        const int tx = r % ntx; r /= ntx;
-        const int ty = r % nty; r /= nty;
-        const int tz = r % ntz; r /= ntz;
-        const int p = r;
-        const int bx = tx * WX, by = ty * WY, bz = tz * WZ;
-        __syncthreads();  // the previous tile's reads are done
-        // input halo: 18 x 6 x 4 voxels, each written to the three shifted copies
-        constexpr int CHI = CIN / 8;
-        for (int idx = threadIdx.x; idx < (WX + 2) * WHY * WHZ * CHI; idx += blockDim.x) {
-            const int c8 = idx % CHI;
-            const int v = idx / CHI;
-            const int hx = v % (WX + 2), hy = (v / (WX + 2)) % WHY, hz = v / ((WX + 2) * WHY);
-            const int gx = bx + hx - 1, gy = by + hy - 1, gz = bz + hz - 1;
-            bf16x8 val;
+        const int bx = r % ntx * WX; r /= ntx;
+        const int by = r % nty * WY; r /= nty;
+        const int bz = r % ntz * WZ; r /= ntz;
+        const bf16* inp = in + (size_t)r * vol * CIN;
+        const bf16* gp = G + (size_t)r * vol * COUT;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) val[j] = (bf16)0.0f;
-            if (gx >= 0 && gx < X && gy >= 0 && gy < Y && gz >= 0 && gz < Z)
-                val = *reinterpret_cast<const bf16x8*>(in + ((size_t)p * vol + ((size_t)gz * Y + gy) * X + gx) * CIN +
-                                                       c8 * 8);
-            // copy dx holds in[x + dx - 1] at column x: column = hx - dx
+        for (int q = 0; q < NI; ++q) {
+            const int idx = tid + WG_THREADS * q, c8 = idx % CHI, v = idx / CHI;
+            const int gx = bx + v % (WX + 2) - 1, gy = by + v / (WX + 2) % WHY - 1, gz = bz + v / ((WX + 2) * WHY) - 1;
 #pragma unroll
-            for (int dx = 0; dx < 3; ++dx) {
-                const int col = hx - dx;
-                if (col < 0 || col >= WX) continue;
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    Xs[(((dx * CI + c8 * 8 + j) * WHZ + hz) * WHY + hy) * WX + col] = val[j];
-            }
+            for (int j = 0; j < 8; ++j) si[q][j] = (bf16)0.0f;
+            if (idx < WHV * CHI && gx >= 0 && gx < X && gy >= 0 && gy < Y && gz >= 0 && gz < Z)
+                si[q] = *reinterpret_cast<const bf16x8*>(inp + (((size_t)gz * Y + gy) * X + gx) * CIN + c8 * 8);
         }
-        constexpr int CHG = COUT / 8;
-        for (int idx = threadIdx.x; idx < WK * CHG; idx += blockDim.x) {
-            const int c8 = idx % CHG, k = idx / CHG;
-            const int x = k % WX, y = (k / WX) % WY, zz = k / (WX * WY);
-            const bf16x8 val = *reinterpret_cast<const bf16x8*>(
-                G + ((size_t)p * vol + ((size_t)(bz + zz) * Y + by + y) * X + bx + x) * COUT + c8 * 8);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) Gt[(c8 * 8 + j) * WK + k] = val[j];
+        for (int q = 0; q < NG; ++q) {
+            const int idx = tid + WG_THREADS * q, c8 = idx % CHG, k = idx / CHG;
+            if (idx < WK * CHG)
+                sg[q] = *reinterpret_cast<const bf16x8*>(
+                    gp + (((size_t)(bz + k / (WX * WY)) * Y + by + k / WX % WY) * X + bx + k % WX) * COUT + c8 * 8);
         }
-        __syncthreads();
+    };
+    auto store = [&](unsigned char* buf) {
 #pragma unroll
-        for (int ks = 0; ks < WK / 32; ++ks) {
-            // this lane's 8 voxels: row r = 2*ks + kg/2 of the tile, columns xo..xo+7
-            const int row = 2 * ks + (kg >> 1), xo = (kg & 1) * 8;
-            const int yy = row % WY, zz = row / WY;
+        for (int q = 0; q < NI; ++q) {
+            const int idx = tid + WG_THREADS * q, c8 = idx % CHI, v = idx / CHI;
+            const int at = (c8 >> 1) * WPV * BI + (v / (WX + 2) * WPX + v % (WX + 2)) * BI + (c8 & 1) * 16;
+            if (idx < WHV * CHI) *reinterpret_cast<bf16x8*>(buf + at) = si[q];
+        }
+#pragma unroll
+        for (int q = 0; q < NG; ++q) {
+            const int idx = tid + WG_THREADS * q, c8 = idx % CHG, k = idx / CHG;
+            if (idx < WK * CHG)
+                *reinterpret_cast<bf16x8*>(buf + X_BYTES + (c8 >> 1) * WK * BO + k * BO + (c8 & 1) * 16) = sg[q];
+        }
+    };
+    // the lane's voxel in a run, and its channels; K step ks of the wave's
+    // planes takes rows 2*ks and 2*ks+1 of their eight, 8 voxels per kg
+    const int run = m >> 2;
+    const int base_i = ((2 * wh * WHY + (kg >> 1)) * WPX + (kg & 1) * 8 + run) * BI + (BI == 32 ? m & 3 : m & 1) * 8;
+    const int base_g = X_BYTES + (2 * wh * WX * WY + kg * 8 + run) * BO + (BO == 32 ? m & 3 : m & 1) * 8;
+    int cur = 0;
+    int tile = blockIdx.x;
+    if (tile < ntiles) {
+        load(tile);
+        store(lds);
+    }
+    __syncthreads();
+    for (; tile < ntiles; tile += gridDim.x) {
+        const bool more = tile + (int)gridDim.x < ntiles;
+        if (more) load(tile + gridDim.x);
+        const unsigned char* buf = lds + cur * BUF;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
             bf16x8 b[NT];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                b[nt] = *reinterpret_cast<const bf16x8*>(&Gt[(nt * 16 + m) * WK + ks * 32 + kg * 8]);
+            for (int nt = 0; nt < NT; ++nt) b[nt] = read_run(buf + base_g + nt * WK * BO + ks * 32 * BO, BO);
 #pragma unroll
             for (int t = 0; t < WTAPS; ++t) {
-                const int tap = w + 4 * t;
+                const int tap = wt + 4 * t;
                 if (tap >= NTAP) break;
                 const int dx = tap % 3, dy = (tap / 3) % 3, dz = tap / 9;
+                const unsigned char* row = buf + base_i + ((dz * WHY + dy) * WPX + dx) * BI;
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    const bf16x8 av = *reinterpret_cast<const bf16x8*>(
-                        &Xs[(((dx * CI + mt * 16 + m) * WHZ + zz + dz) * WHY + yy + dy) * WX + xo]);
+                    const bf16x8 av = read_run(row + mt * WPV * BI + ((ks >> 1) * WHY + (ks & 1) * 2) * WPX * BI, BI);
 #pragma unroll
                     for (int nt = 0; nt < NT; ++nt) acc[t][mt][nt] = mfma(av, b[nt], acc[t][mt][nt]);
                 }
             }
         }
+        cur ^= 1;
+        if (more) store(lds + cur * BUF);
+        __syncthreads();  // the next tile is there, and this one's buffer is free
     }
-    // partial[block][tap][ci][co]; lane holds D[ci = 4*kg + i][co = m] of each tile
-    float* out = part + (size_t)blockIdx.x * NTAP * CI * CO;
+    // the two halves of the planes added through LDS
+    floatx4* sum = reinterpret_cast<floatx4*>(lds);
 #pragma unroll
-    for (int t = 0; t < WTAPS; ++t) {
-        const int tap = w + 4 * t;
-        if (tap >= NTAP) break;
+    for (int t = 0; t < WTAPS; ++t)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
+                if (wh == 1) sum[(((wt * WTAPS + t) * MT + mt) * NT + nt) * 64 + lane] = acc[t][mt][nt];
+    __syncthreads();
+    if (wh == 1) return;
+    // partial[block][tap][ci][co]; lane holds D[ci = 4*kg + i][co = m] of each tile
+    float* out = part + (size_t)blockIdx.x * NTAP * CI * CO;
+#pragma unroll
+    for (int t = 0; t < WTAPS; ++t) {
+        const int tap = wt + 4 * t;
+        if (tap >= NTAP) break;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const floatx4 o = sum[(((wt * WTAPS + t) * MT + mt) * NT + nt) * 64 + lane];
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    out[((size_t)tap * CI + mt * 16 + 4 * kg + i) * CO + nt * 16 + m] = acc[t][mt][nt][i];
+                    out[((size_t)tap * CI + mt * 16 + 4 * kg + i) * CO + nt * 16 + m] = acc[t][mt][nt][i] + o[i];
+            }
     }
 }
 
 // grad[offset + (co*cin + ci)*27 + tap] = sum over workgroups in a fixed
-// order: a block of 256 threads takes 8 consecutive weights (co fastest, the
-// partials' memory order) x 32 groups of workgroups; group g sums workgroups
-// g, g+32, ... and the 32 group sums are added in order of g.
-constexpr int RED_W = 8, RED_G = 32;
-__global__ __launch_bounds__(RED_W * RED_G) void k_wgrad_reduce(const float* __restrict__ part, int nblk, int CI,
-                                                                int CO, int cin, int cout, float* __restrict__ grad) {
+// order, all layers in one launch: a block takes 64 consecutive entries of a
+// layer's partials (256 bytes of each workgroup's) x RED_G groups of
+// workgroups; group g sums workgroups g, g+RED_G, ... and the group sums are
+// added in order of g.  Entries of padding channels are not read.  Bound by
+// the partials' 85 MB, which are still in the last-level cache: 23 us for 256
+// workgroups; 100 in four launches that read 32 bytes at a time of 512.
+constexpr int RED_W = 64, RED_G = 16;
+struct WgradLayer {
+    int ci, co, cin, cout, offset, block0;  // padded and real channels, first weight, first block
+    const float* part;
+};
+struct WgradLayers {
+    WgradLayer l[4];
+};
+constexpr int wgrad_words(int l) {  // of one workgroup's partials
+    return NTAP * (LAYERS[l].cin < 16 ? 16 : LAYERS[l].cin) * (LAYERS[l].cout < 16 ? 16 : LAYERS[l].cout);
+}
+
+__global__ __launch_bounds__(RED_W * RED_G) void k_wgrad_reduce(WgradLayers a, int nblk, float* __restrict__ grad) {
     __shared__ double red[RED_G][RED_W];
+    int q = 0;
+    while (q < 3 && (int)blockIdx.x >= a.l[q + 1].block0) ++q;
+    const WgradLayer L = a.l[q];
     const int wl = threadIdx.x % RED_W, gi = threadIdx.x / RED_W;
-    const int e = blockIdx.x * RED_W + wl;
-    const int ne = cout * cin * NTAP;
-    const int co = e % cout, ci = (e / cout) % cin, tap = e / (cout * cin);
-    const size_t stride = (size_t)NTAP * CI * CO;
-    const size_t off = ((size_t)tap * CI + ci) * CO + co;
+    const int e = ((int)blockIdx.x - L.block0) * RED_W + wl;
+    const int co = e % L.co, ci = e / L.co % L.ci, tap = e / (L.co * L.ci);
+    const size_t stride = (size_t)NTAP * L.ci * L.co;
+    const bool real = co < L.cout && ci < L.cin && tap < NTAP;
     double s = 0.0;
-    if (e < ne)
-        for (int b = gi; b < nblk; b += RED_G) s += part[b * stride + off];
+    if (real)
+        for (int b = gi; b < nblk; b += RED_G) s += L.part[b * stride + e];
     red[gi][wl] = s;
     __syncthreads();
-    if (gi == 0 && e < ne) {
+    if (gi == 0 && real) {
         double t = 0.0;
         for (int g = 0; g < RED_G; ++g) t += red[g][wl];
-        grad[((size_t)co * cin + ci) * NTAP + tap] = (float)t;
+        grad[L.offset + ((size_t)co * L.cin + ci) * NTAP + tap] = (float)t;
     }
 }
 
@@ -540,7 +605,6 @@ struct rh_denoiser {
     Buf<float> part;
     Buf<double> lpart;
     int adam_step = 0;
-    int wgrad_blocks = 512;  // persistent workgroups (two rounds of one per CU)
     int device = 0;                  // the device current at creation (own_stream's)
     unsigned char* static_scratch = nullptr;  // that device's copy of `scratch`
     // timing
@@ -607,7 +671,7 @@ struct rh_denoiser {
         g2.alloc(V * 32);
         g1.alloc(V * 32);
         y.alloc(V * 4);
-        part.alloc((size_t)wgrad_blocks * NTAP * 32 * 32);
+        part.alloc((size_t)WGRAD_BLOCKS * (wgrad_words(0) + wgrad_words(1) + wgrad_words(2) + wgrad_words(3)));
         lpart.alloc(1024);
         DN_HIP(hipMemsetAsync(w.p, 0, RH_DN_N_WEIGHTS * sizeof(float), stream));
         reset_adam();
@@ -657,13 +721,14 @@ struct rh_denoiser {
         a.yout = yo;
         a.xres = xres;
         for (int c = 0; c < 4; ++c) a.s[c] = scale[c];
-        if (Z % 8 == 0) {
-            a.nzb = Z / 8;
-            launch(name, k_conv<CIN, NT, EP, 8>, dim3(X / TX, Y / TY, P * a.nzb), dim3(512), a);
-        } else {
-            a.nzb = Z / 4;
-            launch(name, k_conv<CIN, NT, EP, 4>, dim3(X / TX, Y / TY, P * a.nzb), dim3(256), a);
-        }
+        if (Z % 8 == 0) conv_launch<CIN, NT, EP, 4, 8>(name, a, P);
+        else conv_launch<CIN, NT, EP, 4, 4>(name, a, P);
+    }
+
+    template <int CIN, int NT, int EP, int TY, int TZ>
+    void conv_launch(const char* name, ConvArgs& a, int P) {
+        a.nzb = a.Z / TZ;
+        launch(name, k_conv<CIN, NT, EP, TY, TZ>, dim3(a.X / TX, a.Y / TY, P * a.nzb), dim3(64 * TZ), a);
     }
 
     // The forward pass with the packed input in bx8 and the activations of
@@ -685,15 +750,29 @@ struct rh_denoiser {
         forward_with(x, yo, P, X, Y, Z, x8.p, a1.p, a2.p, a3.p);
     }
 
+    float* wgrad_part(int layer) {
+        size_t at = 0;
+        for (int l = 0; l < layer; ++l) at += (size_t)WGRAD_BLOCKS * wgrad_words(l);
+        return part.p + at;
+    }
+    static int wgrad_blocks(int P, int X, int Y, int Z) {
+        const size_t ntiles = (size_t)(X / WX) * (Y / WY) * (Z / WZ) * P;
+        return (int)std::min<size_t>(ntiles, WGRAD_BLOCKS);
+    }
     template <int CIN, int COUT>
     void wgrad(const char* name, const bf16* in, const bf16* G, int P, int X, int Y, int Z, int layer) {
-        constexpr int CI = CIN < 16 ? 16 : CIN, CO = COUT < 16 ? 16 : COUT;
-        const int ntiles = (X / WX) * (Y / WY) * (Z / WZ) * P;
-        const int nblk = ntiles < wgrad_blocks ? ntiles : wgrad_blocks;
-        launch(name, k_wgrad<CIN, COUT>, dim3(nblk), dim3(256), in, G, X, Y, Z, P, part.p);
-        const Layer& L = LAYERS[layer];
-        launch("wgrad_reduce", k_wgrad_reduce, dim3(cdiv((size_t)L.cin * L.cout * NTAP, RED_W)), dim3(RED_W * RED_G),
-               (const float*)part.p, nblk, CI, CO, L.cin, L.cout, g.p + L.offset);
+        launch(name, k_wgrad<CIN, COUT>, dim3(wgrad_blocks(P, X, Y, Z)), dim3(WG_THREADS), in, G, X, Y, Z, P,
+               wgrad_part(layer));
+    }
+    void wgrad_reduce(int P, int X, int Y, int Z) {
+        WgradLayers a;
+        int blocks = 0;
+        for (int l = 0; l < 4; ++l) {
+            const Layer& L = LAYERS[l];
+            a.l[l] = {L.cin < 16 ? 16 : L.cin, L.cout < 16 ? 16 : L.cout, L.cin, L.cout, L.offset, blocks, wgrad_part(l)};
+            blocks += (int)cdiv(wgrad_words(l), RED_W);
+        }
+        launch("wgrad_reduce", k_wgrad_reduce, dim3(blocks), dim3(RED_W * RED_G), a, wgrad_blocks(P, X, Y, Z), g.p);
     }
 
     // forward + loss + backward into g; loss left in `loss`
@@ -714,6 +793,7 @@ struct rh_denoiser {
         wgrad<32, 32>("wgrad3", a2.p, g3.p, P, X, Y, Z, 2);
         wgrad<32, 32>("wgrad2", a1.p, g2.p, P, X, Y, Z, 1);
         wgrad<8, 32>("wgrad1", x8.p, g1.p, P, X, Y, Z, 0);
+        wgrad_reduce(P, X, Y, Z);
     }
 
     void adam(float lr) {
