@@ -1,9 +1,10 @@
 // readback() against a plain loop: array sizes about the chunk's multiples, one
-// to more chunks than slots, with and without helper threads, and an error
-// thrown by a copy or a wait, which must end the threads and reach the caller.
+// to more chunks than slots, and an error thrown by a copy or a wait, which must
+// reach the caller.
 #include <cstdio>
 #include <cstring>
 #include <stdexcept>
+#include <vector>
 
 #include "../rhybrid_amd/csrc/rh_readback.hpp"
 
@@ -48,7 +49,7 @@ int main() {
             bad += !run<double>(nc, dim, 1000, -1, -1);
             bad += !run<float>(nc, dim, nc, -1, -1);
         }
-    // helper threads: several times READBACK_VALUES_PER_THREAD
+    // the sizes of production arrays
     for (size_t nc : {size_t(1) << 18, (size_t(1) << 20) + 77}) {
         bad += !run<float>(nc, 3, 87381, -1, -1);
         bad += !run<double>(nc, 1, 100000, -1, -1);
