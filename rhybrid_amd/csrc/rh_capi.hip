@@ -203,6 +203,7 @@ public:
     // the destination of the next push (dst, tab_new, live_new), swapped after
     // it.  `cap` places hold the segments; app_cap more, after them, the
     // appendix of injected particles that wait for their first push.
+    static constexpr int NEVER = 1 << 20, LOOK_EVERY = 8;  // steps
     struct Species {
         rh_species_desc d;
         size_t cap = 0;
@@ -218,6 +219,9 @@ public:
         double np_est = 0;     // about how many particles there are
         std::array<uint32_t, FILL_CLASSES> tile_fill{};  // of the store as last looked at (k_tile_fill)
         double fill_np = 0;    // np_est then
+        uint32_t fill_max = 0; // the most particles in a tile then, 0 if the classes tell
+        int since_look = NEVER;  // steps since then
+        bool has_lists = false;  // k_tile_lists has run
         DevBuf<Real> partial;  // deposit: per-tile ghost partials (ntiles x next x 4)
         DevBuf<double> ave_n, ave_v;  // temporal averages: running charge and current sums (FP64)
         bool deposited = false;
@@ -385,6 +389,14 @@ public:
             tile_codes(g, slot.data(), code.data(), code.data() + g.next);
             slot_code.alloc(code.size());
             RH_HIP(hipMemcpy(slot_code.p, code.data(), code.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+        }
+        // the staging ring's pages and the stream's copy queue, ready for the
+        // first read-back (1 ms otherwise)
+        memset(staging, 0, READBACK_SLOTS * READBACK_SLOT_BYTES);
+        for (auto& e : staging_ev) {
+            RH_HIP(hipMemcpyAsync(staging, fld[RH_FACE_B].p, std::min(READBACK_SLOT_BYTES, fld[RH_FACE_B].n * sizeof(Real)),
+                                  hipMemcpyDeviceToHost, stream));
+            RH_HIP(hipEventRecord(e, stream));
         }
         RH_HIP(hipStreamSynchronize(stream));
     }
@@ -910,14 +922,18 @@ public:
     // The push's round (the particles that wait in LDS) and threads, from how
     // full the tiles were when last looked at: the cheapest of every number of
     // threads with the largest round that lets a CU's LDS hold so many
-    // workgroups.  A tile costs its passes over the threads, one more for what
-    // does not depend on the particles, and three times the passes if it does
-    // not fit the round; a CU works at its full rate with 24 waves or more, at
-    // (waves / 24)^0.65 of it below.  Measured per species: 128x96x96 with 32
-    // particles per cell (2,048 a tile) 456 us with 2 x 768 threads, 475 with
-    // 2 x 1,024, 511 with 2 x 512, 714 with 1 x 768; 128x64x64 with 8 (512 a
-    // tile) 76 us with 5 x 256, 93 with 4 x 512; 64x48x48 (1,090 a tile) 77 us
-    // with 3 x 512, 94 with 3 x 768.  The results do not depend on the choice.
+    // workgroups.  A tile costs its passes over the threads and one more for
+    // what does not depend on the particles; nearly two times the passes and
+    // two more per round if it does not fit the round.  A CU works at its full
+    // rate with 24 waves or more, at (waves / 24)^0.65 of it below, and starts
+    // an empty tile's workgroup in 1.5 us.  The fullest tile takes about 2 us
+    // a pass however many others there are.  Measured per species: 128x96x96
+    // with 32 particles per cell (2,048 a tile) 456 us with 2 x 768 threads,
+    // 475 with 2 x 1,024, 511 with 2 x 512, 714 with 1 x 768; 128x64x64 with 8
+    // (512 a tile) 76 us with 5 x 256, 93 with 4 x 512; 64x48x48 (1,090 a tile)
+    // 77 us with 3 x 512, 94 with 3 x 768; 80x92x52 with 500,000 photoions, up to
+    // 23,500 in a tile, 203 us with 1,024, 663 with 256.  The results
+    // do not depend on the choice.
     struct PushShape { int round, threads, parts; };
     PushShape choose_push(Species& S_) const {
         const bool looked = S_.fill_np > 0 && S_.np_est < 1.5 * S_.fill_np;
@@ -926,28 +942,41 @@ public:
         one[fill_class((uint32_t)std::min(mean, 1e6))] = 5;
         one[fill_class((uint32_t)std::min(mean + 3.0 * std::sqrt(mean), 1e6))] += 1;
         const auto& fill = looked ? S_.tile_fill : one;
-        double tiles = 0, np = 0;
-        for (int c = 1; c < FILL_CLASSES; ++c) { tiles += fill[c]; np += fill[c] * (64.0 * c - 32.0); }
+        const auto in_class = [&](int c) {  // particles of a tile of class c
+            return c == FILL_CLASSES - 1 && S_.fill_max ? 0.5 * (64.0 * c + S_.fill_max) : 64.0 * c - 32.0;
+        };
+        double sampled = fill[0], live = 0, np = 0, most = 0;
+        for (int c = 1; c < FILL_CLASSES; ++c) {
+            if (!fill[c]) continue;
+            live += fill[c]; np += fill[c] * in_class(c);
+            most = std::max(64.0 * c, (double)S_.fill_max);
+        }
+        sampled += live;
         // parts of a slot with four to eight particles each
         int lq = 0;
-        const double per_slot = tiles > 0 ? np / tiles / (8.0 * g.tc) : 0;
+        const double per_slot = live > 0 ? np / live / (8.0 * g.tc) : 0;
         while ((g.nslot + 1) << (lq + 1) <= 1 << SLOT_BITS && per_slot >= (16 << lq)) ++lq;
         PushShape best{256, 256, lq};
-        double best_cost = 1e300;
+        double best_us = 1e300;
         for (int k = 8; k >= 1; --k) {
             const size_t lds = std::min(lds_limit, (size_t)PUSH_MAX_LDS) / k - 1024;
             int round = 64 * (FILL_CLASSES - 2);
             while (round > 256 && push_lds<Real>(g, round, lq).bytes > lds) round -= 64;
             if (push_lds<Real>(g, round, lq).bytes > lds && k > 1) continue;
             for (int threads : {256, 512, 768, 1024}) {
+                const auto passes = [&](double n, double round_passes) {
+                    const double p = std::ceil(n / threads);
+                    return n <= round ? p + 1 : 1.8 * p + 1 + std::ceil(n / round) * round_passes;
+                };
+                double units = 0;
+                for (int c = 1; c < FILL_CLASSES; ++c)
+                    if (fill[c]) units += fill[c] * passes(c == FILL_CLASSES - 1 || 64 * c > round ? std::max(in_class(c), round + 1.0) : in_class(c), 1.0);
                 const double waves = std::min(24.0, k * threads / 64.0);
-                double cost = 0;
-                for (int c = 1; c < FILL_CLASSES; ++c) {
-                    const double passes = std::ceil((64.0 * c - 32.0) / threads);
-                    cost += fill[c] * (64 * c <= round && c < FILL_CLASSES - 1 ? passes + 1 : 3 * passes + 1);
-                }
-                cost *= threads * std::pow(24.0 / waves, 0.65);
-                if (cost < best_cost) { best_cost = cost; best = {round, threads, lq}; }
+                const double all_us = (units * threads * std::pow(24.0 / waves, 0.65) / 124e3 + fill[0] * 1.5 / (256 * k)) *
+                                      (g.ntiles / std::max(sampled, 1.0));
+                const double last_us = 2.0 * passes(most, 2.0);
+                const double us = std::max(all_us, last_us) + 0.25 * std::min(all_us, last_us);
+                if (us < best_us) { best_us = us; best = {round, threads, lq}; }
             }
         }
         return best;
@@ -989,6 +1018,7 @@ public:
 
     // The tiles' lists of the store as it is now, and the next segments.
     void tile_lists(Species& S_, const char* name) {
+        S_.has_lists = true;
         launch(name, k_tile_lists, cdiv(g.ntiles, TILES_PER_LIST_BLOCK), LIST_THREADS, 0, g, (const uint32_t*)S_.dtab.p,
                S_.tile_list.p, S_.seg_loc.p, S_.seg_blk.p, S_.scal.p);
     }
@@ -997,6 +1027,7 @@ public:
     // without pushing anything.
     void merge(Species& S_) {
         if (S_.pushed) throw StateError("injected particles pending between propagate and wait_particle_sends");
+        if (S_.has_lists && ++S_.since_look >= LOOK_EVERY) look_at_fill(S_);
         PushParams pp{};
         pp.still = 1;
         push(S_, pp, "sort_still");
@@ -1022,8 +1053,11 @@ public:
         launch("tile_fill", k_tile_fill, 1, FILL_THREADS, 0, g, (const uint32_t*)S_.tile_list.p, S_.scal.p);
         RH_HIP(hipMemcpyAsync(sc, S_.scal.p, sizeof(sc), hipMemcpyDeviceToHost, stream));
         RH_HIP(hipStreamSynchronize(stream));
+        S_.since_look = 0;
+        if (!sc[SC_NP]) return;  // (injected ones may be waiting)
         std::copy(sc + SC_FILL, sc + SC_N, S_.tile_fill.begin());
         S_.np_est = S_.fill_np = (double)sc[SC_NP];
+        S_.fill_max = sc[SC_FILL_MAX];
     }
 
     uint32_t scalar(Species& S_, int id) {
@@ -1355,6 +1389,8 @@ public:
     }
 
     void step(int n) override {
+        for (auto& s_ : sp)
+            if (s_->since_look >= NEVER && s_->has_lists && !s_->pushed) look_at_fill(*s_);
         for (int it = 0; it < n; ++it) {
             ++tstep;
             if (species_streams && sp.size() > 1) {
@@ -1374,10 +1410,8 @@ public:
             propagate_B_impl(it == n - 1);
         }
         check_overflow();
-        // for the next call's choice of the push's workgroups
-        for (auto& s_ : sp) {
-            look_at_fill(*s_);
-        }
+        for (auto& s_ : sp)
+            if ((s_->since_look += n) >= LOOK_EVERY) look_at_fill(*s_);
     }
 
     // propagate, wait_particle_sends and accumulate of every species, each

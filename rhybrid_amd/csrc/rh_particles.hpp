@@ -220,7 +220,8 @@ enum DevScalar {
     SC_NP = 0,   // particles in the segments (removed ones included until the next push)
     SC_END,      // store indices in use by the segments
     SC_TICKET,   // blocks of k_tile_lists that are done
-    SC_FILL,     // k_tile_fill's FILL_CLASSES counts
+    SC_FILL_MAX, // k_tile_fill's fullest tile, and its FILL_CLASSES counts
+    SC_FILL,
     SC_N = SC_FILL + 128
 };
 
@@ -436,23 +437,27 @@ __global__ __launch_bounds__(LIST_THREADS) void k_tile_lists(Geom g, const uint3
 // How full the tiles are, for the choice of the push's workgroups: of about
 // FILL_SAMPLE tiles spread over the grid the number that hold
 // 64c-63 .. 64c particles, per class c (the last class also fuller ones;
-// empty tiles are not counted).  One block, once per run of steps.
+// empty tiles are class 0), and the most that one holds.  One block, once per
+// run of steps.
 constexpr int FILL_CLASSES = SC_N - SC_FILL, FILL_SAMPLE = 4096, FILL_THREADS = 1024;
 RH_HD int fill_class(uint32_t n) { return n >= 64u * (FILL_CLASSES - 1) ? FILL_CLASSES - 1 : (int)((n + 63u) / 64u); }
 
 __global__ __launch_bounds__(FILL_THREADS) void k_tile_fill(Geom g, const uint32_t* __restrict__ lists,
                                                             uint32_t* __restrict__ scal) {
-    __shared__ uint32_t h[FILL_CLASSES];
+    __shared__ uint32_t h[FILL_CLASSES], most;
     const int tid = threadIdx.x, stride = (g.ntiles + FILL_SAMPLE - 1) / FILL_SAMPLE;
     if (tid < FILL_CLASSES) h[tid] = 0;
+    if (tid == 0) most = 0;
     __syncthreads();
     for (int T = tid * stride; T < g.ntiles; T += FILL_THREADS * stride) {
         const uint32_t* L = lists + (size_t)T * LIST_WORDS;
         const uint32_t n = L[LIST_PREF + 27] + L[LIST_OWN + 1];
-        if (n) atomicAdd(&h[fill_class(n)], 1u);
+        atomicAdd(&h[fill_class(n)], 1u);
+        if (n >= 64u * (FILL_CLASSES - 1)) atomicMax(&most, n);
     }
     __syncthreads();
     if (tid < FILL_CLASSES) scal[SC_FILL + tid] = h[tid];
+    if (tid == 0) scal[SC_FILL_MAX] = most;
 }
 
 // A Geom whose tile shape is known to the compiler: sides 2^LX, 2^LY, 2^LZ
@@ -557,15 +562,23 @@ struct Particle {
     Real X, Y, Z, vx, vy, vz;
 };
 
+// The particle's code from its extended cell (g.next: removed) and place in it.
+template <typename Real>
+__device__ __forceinline__ uint32_t particle_code(const uint32_t* codes, int e, const Particle<Real>& q) {
+    const uint32_t code = codes[e];
+    const uint32_t o = (q.X >= Real(0.5)) + 2 * (q.Y >= Real(0.5)) + 4 * (q.Z >= Real(0.5));
+    return (code & ~(7u << CODE_OCT_SHIFT)) + (o & (code >> CODE_OCT_SHIFT & 7u));
+}
+
 // One particle: push, move, code.  fl is the tile's field block, codes its
-// extended cells' codes; edge: the tile holds cells without all neighbours.
+// extended cells' codes, e the extended cell it ends in; edge: the tile holds cells without all neighbours.
 // PLAIN: accelerated, without gravity, and moved (the parameters of most
 // runs; the others are tested for).  Without branches except for the speed
 // limit, so that several particles' LDS reads are in flight.
 template <typename Real, bool PLAIN>
 __device__ __forceinline__ uint32_t push_particle(const Geom& g, const PushParams& pp, const int (&org)[3], bool edge,
                                                   const Real* fl, const uint32_t* codes, Particle<Real>& q, int lc,
-                                                  uint32_t& n_clamped, uint32_t& n_dropped) {
+                                                  int& e, uint32_t& n_clamped, uint32_t& n_dropped) {
     const bool act = q.X >= Real(0);
     const int hx = g.tx + 1, hy = g.ty + 1, nh = (g.tx + 1) * (g.ty + 1) * (g.tz + 1);
     const Real* sbx = fl;  // faceB of local cells -1..t-1 (halo on the low side)
@@ -644,11 +657,11 @@ __device__ __forceinline__ uint32_t push_particle(const Geom& g, const PushParam
         Y = Y < Real(1) ? Y : below_one<Real>();
         Z = Z < Real(1) ? Z : below_one<Real>();
     }
-    const uint32_t code = codes[act && ok ? (li + sx + 1) + g.ex * ((lj + sy + 1) + g.ey * (lk + sz + 1)) : g.next];
-    const uint32_t o = (X >= Real(0.5)) + 2 * (Y >= Real(0.5)) + 4 * (Z >= Real(0.5));
-    n_dropped += act && (code & SLOT_MASK) == (uint32_t)g.nslot;
+    e = act && ok ? (li + sx + 1) + g.ex * ((lj + sy + 1) + g.ey * (lk + sz + 1)) : g.next;
     q.X = X; q.Y = Y; q.Z = Z; q.vx = vx; q.vy = vy; q.vz = vz;
-    return (code & ~(7u << CODE_OCT_SHIFT)) + (o & (code >> CODE_OCT_SHIFT & 7u));
+    const uint32_t code = particle_code(codes, e, q);
+    n_dropped += act && (code & SLOT_MASK) == (uint32_t)g.nslot;
+    return code;
 }
 
 // How many of the slot's list entries (from `part`, c of them, padded with
@@ -671,8 +684,11 @@ __device__ __forceinline__ uint32_t list_rank(const uint16_t* part, uint32_t c, 
 // counted (integer LDS atomics) and scanned, and is then written to its
 // place, a wave writing 64 places in a row (written by the particles' own
 // order instead, a wave's places lie in up to twice as many cache lines and
-// the address units bound the kernel).  A fuller tile is pushed three times:
-// to count, then round by round for the codes and to write.  A particle's
+// the address units bound the kernel).  A fuller tile is pushed
+// once too, for the counts, but waits in place of its input, and is then
+// ranked and written round by round (pushed again in every round, for the code
+// and to be written, the photoions of 160x128x128, up to 12,000 in a tile, take
+// 429 us instead of 333).  A particle's
 // rank in its slot is the number of the round's particles of that slot that
 // come before it: the atomics hand out places of a list by slot in any order,
 // and each particle then counts the smaller entries of its slot's few, so the
@@ -749,8 +765,10 @@ __global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
     }
     if (tid < LIST_WORDS) L[tid] = lw;
     // the others: arrivals, then injected particles
+    auto other_place = [&](uint32_t v) { return v < na ? arrival_index(L, v) : a0 + (v - na); };
+    auto place = [&](uint32_t u) { return u < n0 ? p0 + u : other_place(u - n0); };
     auto other = [&](uint32_t v, Particle<Real>& q, int& lc) {
-        const uint32_t p = v < na ? arrival_index(L, v) : a0 + (v - na);
+        const uint32_t p = other_place(v);
         q.X = A.x[p]; q.Y = A.y[p]; q.Z = A.z[p];
         q.vx = A.vx[p]; q.vy = A.vy[p]; q.vz = A.vz[p];
         lc = A.lc[p];
@@ -839,11 +857,6 @@ __global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
         for (uint32_t u = total + tid; u < N; u += NT)
             if (u < places) (D.x + seg)[u] = Real(-1);
     };
-    auto store = [&](uint32_t dst, const Particle<Real>& q, uint32_t c) {
-        (D.x + seg)[dst] = q.X; (D.y + seg)[dst] = q.Y; (D.z + seg)[dst] = q.Z;
-        (D.vx + seg)[dst] = q.vx; (D.vy + seg)[dst] = q.vy; (D.vz + seg)[dst] = q.vz;
-        (D.lc + seg)[dst] = (uint8_t)(c >> CELL_SHIFT);
-    };
     if (one) {
         for (int i = tid; i < (int)N; i += NT) {
             if (i >= (int)n0) other((uint32_t)i - n0, nq, nlc);
@@ -851,7 +864,8 @@ __global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
             const int lc = nlc;
             const uint32_t u = (uint32_t)(i + NT);
             if (u < n0) own(u, nq, nlc);  // the next own one is loaded ahead
-            uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, n_clamped, n_dropped);
+            int e;
+            uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, e, n_clamped, n_dropped);
             S4[i] = Real4<Real>{{q.X, q.Y, q.Z, q.vx}};
             S2[i] = Real2<Real>{{q.vy, q.vz}};
             c = part_code(c, i);
@@ -892,16 +906,23 @@ __global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
             }
         }
     } else {
-        auto any = [&](uint32_t u, Particle<Real>& q, int& lc) {
-            if (u < n0) own(u, q, lc);
-            else other(u - n0, q, lc);
-        };
+        // Pushed for the counts, and written back where it came from (no other
+        // tile reads those places): its extended cell e in lc, the ninth bit
+        // of e as the sign of Y.  A removed one keeps its old state.
         for (uint32_t u = tid; u < N; u += NT) {
-            Particle<Real> q;
-            int lc;
-            any(u, q, lc);
-            const uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, n_clamped, n_dropped);
+            if (u >= n0) other(u - n0, nq, nlc);
+            Particle<Real> q = nq;
+            const int lc = nlc;
+            if (u + NT < n0) own(u + NT, nq, nlc);  // the next own one is loaded ahead
+            const Particle<Real> was = q;
+            int e;
+            const uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, e, n_clamped, n_dropped);
+            if ((c & SLOT_MASK) == (uint32_t)K) { q = was; e = g.next; }
             atomicAdd(&cnt[part_code(c, (int)u) & SLOT_MASK], 1u);
+            const uint32_t p = place(u);
+            A.x[p] = q.X; A.y[p] = e & 256 ? -q.Y : q.Y; A.z[p] = q.Z;
+            A.vx[p] = q.vx; A.vy[p] = q.vy; A.vz[p] = q.vz;
+            A.lc[p] = (uint8_t)e;
         }
         __syncthreads();
         const uint32_t total = scan_slots(true);
@@ -909,18 +930,20 @@ __global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
         __syncthreads();
         for (int e = tid; e < KT; e += NT) cnt[e] = 0u;
         __syncthreads();
-        // each round's particles are pushed for their codes, and again to be
-        // written at their places (their input is still in the caches)
+        // each round's particles then wait in LDS for their ranks
         for (uint32_t ub = 0; ub < N; ub += round) {
             const int n = (int)min((uint32_t)round, N - ub);
-            uint32_t unused0 = 0, unused1 = 0;
             for (int i = tid; i < n; i += NT) {
+                const uint32_t p = place(ub + i);
                 Particle<Real> q;
-                int lc;
-                any(ub + i, q, lc);
-                uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, unused0, unused1);
-                c = part_code(c, i);
+                q.X = A.x[p]; q.Y = A.y[p]; q.Z = A.z[p];
+                q.vx = A.vx[p]; q.vy = A.vy[p]; q.vz = A.vz[p];
+                int e = A.lc[p];
+                if (__builtin_signbit(q.Y)) { q.Y = -q.Y; e |= 256; }
+                uint32_t c = part_code(q.X >= Real(0) ? particle_code(codes, e, q) : (uint32_t)K, i);
                 c |= atomicAdd(&cnt[c & SLOT_MASK], 1u) << RANK_SHIFT;
+                S4[i] = Real4<Real>{{q.X, q.Y, q.Z, q.vx}};
+                S2[i] = Real2<Real>{{q.vy, q.vz}};
                 scode[i] = c;
             }
             __syncthreads();
@@ -932,15 +955,15 @@ __global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
             }
             __syncthreads();
             for (int i = tid; i < n; i += NT) {
-                const uint32_t s = scode[i] & SLOT_MASK;
+                const uint32_t c = scode[i], s = c & SLOT_MASK;
                 if (s >= (uint32_t)KQ) continue;
-                Particle<Real> q;
-                int lc;
-                any(ub + i, q, lc);
-                const uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, unused0, unused1);
                 const uint32_t dst = goff[s] + list_rank(list + loff[s], cnt[s], (uint32_t)i);
                 if (dst < places) {
-                    store(dst, q, c);
+                    const Real4<Real> a = S4[i];
+                    const Real2<Real> b = S2[i];
+                    (D.x + seg)[dst] = a.v[0]; (D.y + seg)[dst] = a.v[1]; (D.z + seg)[dst] = a.v[2];
+                    (D.vx + seg)[dst] = a.v[3]; (D.vy + seg)[dst] = b.v[0]; (D.vz + seg)[dst] = b.v[1];
+                    (D.lc + seg)[dst] = (uint8_t)(c >> CELL_SHIFT);
                 } else {
                     atomicAdd(counters + C_RANK_OVERFLOW, 1ull);  // slot 0
                 }
