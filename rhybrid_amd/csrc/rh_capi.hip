@@ -1109,12 +1109,13 @@ public:
         S_.deposited = true;
     }
 
-    // A cell has at most two candidate tiles per axis: tiles (also the last,
-    // partial one) of at least two cells, and no wrap onto the same tile.
+    // A cell has at most two candidate tiles per axis: tiles of at least two
+    // cells (but the last of an axis without wrap, which has no next one), and
+    // no wrap onto the same tile.  75x54x49: 20 -> 14 us.
     bool fold_two_per_axis() const {
         const int n[3] = {g.nx, g.ny, g.nz}, lt[3] = {g.ltx, g.lty, g.ltz}, nt[3] = {g.ntx, g.nty, g.ntz};
         for (int d = 0; d < 3; ++d)
-            if (lt[d] == 0 || tile_width(n[d], lt[d], nt[d] - 1) < 2 || (g.per[d] && nt[d] < 3)) return false;
+            if (lt[d] == 0 || (g.per[d] && (nt[d] < 3 || tile_width(n[d], lt[d], nt[d] - 1) < 2))) return false;
         return true;
     }
 
@@ -1374,7 +1375,7 @@ public:
             fill(fld[RH_CELL_J].p, Real(0), fld[RH_CELL_J].n);
         }
         if (P.use_gaussian) {
-            RH_HIP(hipMemcpyAsync(tmpv.p, fld[RH_NODE_E].p, sizeof(Real) * 3 * g.nc, hipMemcpyDeviceToDevice, stream));
+            std::swap(fld[RH_NODE_E].p, tmpv.p);
             V3<Real> old{tmpv.p, tmpv.p + g.nc, tmpv.p + 2 * (size_t)g.nc};
             launch("node_avg", k_node_avg<Real>, cb, bb, 0, g, old, v3(RH_NODE_E), (Real)P.gauss_coeffs[0],
                    (Real)P.gauss_coeffs[1], (Real)P.gauss_coeffs[2], (Real)P.gauss_coeffs[3]);
@@ -1408,6 +1409,10 @@ public:
             // only the last step's update writes the arrays nothing in
             // between reads
             propagate_B_impl(it == n - 1);
+            // (particles that a first step has only now sorted)
+            if (it == 0 && n > 1)
+                for (auto& s_ : sp)
+                    if (s_->since_look >= NEVER) look_at_fill(*s_);
         }
         check_overflow();
         for (auto& s_ : sp)
