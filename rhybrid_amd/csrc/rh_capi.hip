@@ -971,7 +971,8 @@ public:
                 double units = 0;
                 for (int c = 1; c < FILL_CLASSES; ++c)
                     if (fill[c]) units += fill[c] * passes(c == FILL_CLASSES - 1 || 64 * c > round ? std::max(in_class(c), round + 1.0) : in_class(c), 1.0);
-                const double waves = std::min(24.0, k * threads / 64.0);
+                // (the registers of the kernel are made for 24 waves a CU)
+                const double waves = std::min(k, 1536 / threads) * threads / 64.0;
                 const double all_us = (units * threads * std::pow(24.0 / waves, 0.65) / 124e3 + fill[0] * 1.5 / (256 * k)) *
                                       (g.ntiles / std::max(sampled, 1.0));
                 const double last_us = 2.0 * passes(most, 2.0);
@@ -1053,7 +1054,7 @@ public:
         launch("tile_fill", k_tile_fill, 1, FILL_THREADS, 0, g, (const uint32_t*)S_.tile_list.p, S_.scal.p);
         RH_HIP(hipMemcpyAsync(sc, S_.scal.p, sizeof(sc), hipMemcpyDeviceToHost, stream));
         RH_HIP(hipStreamSynchronize(stream));
-        S_.since_look = 0;
+        S_.since_look = sc[SC_NP] || !S_.np_est ? 0 : NEVER;
         if (!sc[SC_NP]) return;  // (injected ones may be waiting)
         std::copy(sc + SC_FILL, sc + SC_N, S_.tile_fill.begin());
         S_.np_est = S_.fill_np = (double)sc[SC_NP];
