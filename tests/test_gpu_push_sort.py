@@ -98,3 +98,36 @@ def test_partial_tiles_obstacle_inflow(gpu_mod, oracle_mod, prec, dims):
         print("%s rel L2 %.3e" % (name, r), flush=True)
         assert r < (1e-9 if prec else 1e-5), (name, r)
     ctx.close()
+
+
+# many particles that enter one subcell of a tile from its neighbour in one
+# step: a list of every length around the four that the deposit takes at a
+# time, and more than it links in one chunk
+@pytest.mark.parametrize("prec", [1, 0])
+@pytest.mark.parametrize("counts", [(1, 2, 3, 4, 5, 6, 7), (8, 9, 12, 13, 16, 17, 0), (800,)])
+def test_arrivals_of_one_subcell(gpu_mod, oracle_mod, prec, counts):
+    print("case %s precision %d" % (counts, prec), flush=True)
+    pr = P.config_periodic(n=8, ppc=8, seed=57)
+    g, rng = pr.grid, np.random.default_rng(58)
+    speed = 0.3 * g.dx / pr.params.dt
+    pr.params.max_ion_speed2 = (10.0 * speed) ** 2
+    cells, states = [pr.particles[0].cell], [pr.particles[0].state]
+    for q, n in enumerate(counts):  # from cell (3, q, 1) to the lower octants of (4, q, 1)
+        st = np.zeros((n, states[0].shape[1]))
+        st[:, 6:] = states[0][0, 6:]
+        st[:, 0] = rng.uniform(0.75, 0.95, n) * g.dx
+        st[:, 1:3] = rng.uniform(0.1, 0.4, (n, 2)) * g.dx
+        st[:, 3] = speed
+        cells.append(np.full(n, 3 + 8 * (q + 8), dtype=cells[0].dtype))
+        states.append(st)
+    pr.particles[0] = P.Particles(np.concatenate(cells), np.concatenate(states))
+    ora = oracle_mod.Oracle(pr)
+    ora.step(1)
+    ctx = gpu_mod.Context(pr, precision=prec, tile=(4, 4, 4))
+    ctx.step(1)
+    assert ctx.num_particles(0) == ora.num_particles(0)
+    for name in ("cellRhoQi", "cellJi"):
+        r = rel(ctx.field(name), ora.field(name))
+        print("%s rel L2 %.3e" % (name, r), flush=True)
+        assert r < (1e-9 if prec else 1e-5), (name, r)
+    ctx.close()
