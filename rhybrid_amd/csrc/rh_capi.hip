@@ -791,6 +791,14 @@ public:
         Species& S_ = S(s);
         if (n < 0 || (n > 0 && (!cell || !st))) throw ArgError("bad particle arrays");
         if ((uint64_t)n >= 0xFFFFFFFFull) throw CapError("too many particles for 32-bit indices");
+        if (n == 0) {  // (no tables are read where no tile is live)
+            ensure_capacity(S_, (size_t)std::max<int64_t>(S_.d.capacity, 0));
+            fill(S_.live.p, (uint8_t)0, S_.live.n);
+            fill(S_.dtab.p, 0u, S_.dtab.n);
+            fill(S_.scal.p, 0u, S_.scal.n);
+            uploaded(S_);
+            return;
+        }
         // keys and a stable counting sort on the host
         std::vector<uint32_t> key((size_t)n);
         std::vector<Real> u[3];
@@ -843,6 +851,10 @@ public:
         sc[SC_END] = (uint32_t)n;
         RH_HIP(hipMemcpyAsync(S_.scal.p, sc, sizeof(sc), hipMemcpyHostToDevice, stream));
         RH_HIP(hipMemcpyAsync(S_.dtab.p, dtab.data(), sizeof(uint32_t) * dtab.size(), hipMemcpyHostToDevice, stream));
+        uploaded(S_);
+    }
+
+    void uploaded(Species& S_) {
         tile_lists(S_, "sort_still");
         look_at_fill(S_);
         S_.pushed = false;

@@ -131,3 +131,21 @@ def test_arrivals_of_one_subcell(gpu_mod, oracle_mod, prec, counts):
         print("%s rel L2 %.3e" % (name, r), flush=True)
         assert r < (1e-9 if prec else 1e-5), (name, r)
     ctx.close()
+
+
+@pytest.mark.parametrize("prec", [1, 0])
+def test_empty_upload_over_a_stepped_store(gpu_mod, oracle_mod, prec):
+    pr = P.config_periodic(n=8, ppc=8, seed=59)
+    ctx = gpu_mod.Context(pr, precision=prec)
+    ctx.step(2)
+    full = ctx.particles(0)
+    ctx.upload_particles(0, full[0][:0], full[1][:0])
+    assert ctx.num_particles(0) == 0 and len(ctx.particles(0)[0]) == 0
+    ctx.upload_particles(0, *full)
+    again = ctx.particles(0)
+    assert np.array_equal(full[0], again[0]) and np.array_equal(full[1], again[1])
+    ctx.upload_particles(0, full[0][:0], full[1][:0])
+    ctx.step(1)
+    assert ctx.num_particles(0) == 0
+    assert not ctx.field("cellJi").any()
+    ctx.close()
