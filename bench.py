@@ -45,26 +45,23 @@ def kernel_bytes(name: str, ctx, np_total: float, nspecies: int, npp: float = No
     lay = ctx.layout()
     nc, ntiles = lay["ncells"], lay["ntiles"]
     next_ = (lay["tx"] + 2) * (lay["ty"] + 2) * (lay["tz"] + 2)
-    extk = next_ * 8
-    nkeys = ntiles * lay["tx"] * lay["ty"] * lay["tz"] * 8
     if npp is None:
         npp = np_total / nspecies  # particles per species launch (mean)
     nh = (lay["tx"] + 1) * (lay["ty"] + 1) * (lay["tz"] + 1)
     tc = lay["tx"] * lay["ty"] * lay["tz"]
+    kt = (7 * tc + next_ + 4) & ~3               # places of a tile's slot table
     fblock = 4.0 * (3 * nh + 7 * tc) * ntiles   # per-tile field blocks (FP32 + neighbourhood masks)
     if name == "push_fields":  # read 9 f32 fields per cell, write the per-tile blocks
         return 36.0 * nc + fblock
-    if name == "push":       # pass 0: read 6 f32 + local cell byte and the field blocks; write 16-bit slot counts
-        return 25.0 * npp + fblock + 2.0 * extk * ntiles + 8.0 * ntiles
-    if name == "move":       # pass 1: read and write 6 f32 + local cell byte; field blocks; 16-bit slot
-        # offsets and the 32-bit starts of the extended region's subcells
-        return 50.0 * npp + fblock + 6.0 * extk * ntiles + 8.0 * ntiles
-    if name == "deposit":    # read 6 f32 per particle and the subcell starts; write the f32 tile ghosts
-        return 24.0 * npp + 4.0 * nkeys + 16.0 * next_ * ntiles
+    if name == "move":       # push and sort: read and write 6 f32 + local cell byte; field blocks; slot tables,
+        # direction tables and the lists of the tile's particles
+        return 50.0 * npp + fblock + 4.0 * (kt + 32 + 64) * ntiles
+    if name == "deposit":    # read 6 f32 per particle, the subcell starts and the lists; write the f32 tile ghosts
+        return 24.0 * npp + (32.0 * tc + 256.0) * ntiles + 16.0 * next_ * ntiles
     if name == "fold":       # read the f32 tile ghosts once, write rho + J (f32)
         return 16.0 * next_ * ntiles + 16.0 * nc
-    if name == "sort_slots":  # read and write the 16-bit slot table, write the totals
-        return 4.0 * extk * ntiles + 4.0 * nkeys
+    if name == "sort_slots":  # read the direction tables, write the lists and the segments' places
+        return 4.0 * (32 + 64 + 1) * ntiles
     if name == "field_update":  # fused propagateB: read faceB, rho, Ji, eta (32 B), flags (3 B); write faceB,
         # cellUe, cellEp (36 B) and the per-tile push-field blocks (the last step of a call also writes the
         # reference's other arrays; not counted)
@@ -72,9 +69,8 @@ def kernel_bytes(name: str, ctx, np_total: float, nspecies: int, npp: float = No
     return 0.0
 
 
-PROFILE_KERNELS = {"push": "rh::k_push_move<float>_[pass_0:_push]", "move": "rh::k_push_move<float>_[pass_1:_move]",
-                   "deposit": "rh::k_deposit<float>", "fold": "rh::k_fold<float>",
-                   "sort_slots": "rh::k_slot_offsets"}
+PROFILE_KERNELS = {"move": "rh::k_push_sort<float>", "deposit": "rh::k_deposit<float>", "fold": "rh::k_fold<float>",
+                   "sort_slots": "rh::k_tile_lists"}
 
 
 def measured_traffic(kernel: str, profile: str = "hbm_traffic_obstacle128x96x96_ppc32_inflow.txt",
@@ -145,8 +141,8 @@ def gpu_bench(args, pr):
     ctx.step(nb)
     ctx.synchronize()
     ctx.set_timing(False)
-    names = ["push_fields", "push", "sort_slots", "sort_count", "scan", "sort_base", "move", "deposit",
-             "deposit_dense", "fold", "boundary", "inject_slots", "inject_count", "inject_fill", "sort_still",
+    # ("push" names the same launches as "move")
+    names = ["push_fields", "sort_slots", "scan", "move", "deposit", "fold", "boundary", "inject_slots", "inject_count", "inject_fill", "sort_still",
              "cell_B_bc", "neumann", "imf", "cell2node", "node_J", "node2cell", "cell_J_Ue", "node_Ue_B_E",
              "node_avg", "face_curl_Ep", "field_update", "fill", "diag"]
     ktimes = {}
@@ -155,8 +151,7 @@ def gpu_bench(args, pr):
         if n:
             ktimes[nm] = (ms, n)
     total_k = sum(v[0] for v in ktimes.values())
-    pd_names = ("push_fields", "push", "sort_slots", "sort_count", "scan", "sort_base", "move", "deposit",
-                "deposit_dense", "fold")
+    pd_names = ("push_fields", "sort_slots", "scan", "move", "deposit", "fold")
     t_pd = sum(ktimes[k][0] for k in pd_names if k in ktimes) / 1e3
     dom = max(ktimes, key=lambda k: ktimes[k][0])
     per_kernel = {}
@@ -561,7 +556,7 @@ def exosphere_bench(steps: int = 10, warmup: int = 2, prefill: int = 600, tune_s
     for s, sp in enumerate(("H+", "O+")):
         npp = 0.5 * (n0[s] + n1[s])
         row = {}
-        for nm in ("push", "sort_slots", "move", "deposit", "boundary", "inject_count", "inject_fill",
+        for nm in ("sort_slots", "move", "deposit", "boundary", "inject_count", "inject_fill",
                    "inject_slots"):
             ms, n = ctx.kernel_time("%s:%d" % (nm, s))
             if n:
