@@ -142,8 +142,8 @@ def gpu_bench(args, pr):
     ctx.synchronize()
     ctx.set_timing(False)
     # ("push" names the same launches as "move")
-    names = ["push_fields", "sort_slots", "scan", "move", "deposit", "fold", "boundary", "inject_slots", "inject_count", "inject_fill", "sort_still",
-             "cell_B_bc", "neumann", "imf", "cell2node", "node_J", "node2cell", "cell_J_Ue", "node_Ue_B_E",
+    names = ["push_fields", "sort_slots", "scan", "move", "deposit", "fold", "boundary",
+             "inject_slots", "inject_count", "inject_fill", "sort_still", "cell_B_bc", "neumann", "imf", "cell2node", "node_J", "node2cell", "cell_J_Ue", "node_Ue_B_E",
              "node_avg", "face_curl_Ep", "field_update", "fill", "diag"]
     ktimes = {}
     for nm in names:
