@@ -1442,8 +1442,8 @@ __global__ __launch_bounds__(512, sizeof(Real) == 8 ? 4 : 8) void k_deposit(Geom
     // are staged; a thread takes those of its list, in ascending order, after
     // its own.  The loops over the tile's own particles hold nothing of the
     // arrivals in registers (64 of them let four workgroups share a CU): 128x96x96
-    // with 35.5 M particles takes 314 us a launch (2.9 TB/s; 280 without
-    // arrivals), and took 370 with both kinds in one loop, 332 with the list
+    // with 35.5 M particles takes 314 us a launch (2.9 TB/s; 280 where
+    // every particle lies in its own tile's segment), and took 370 with both kinds in one loop, 332 with the list
     // read before the own ones, 392 with three own particles' loads in flight.
     const int CH = deposit_chunk<Real>(g);
     Real4<Real>* L4 = reinterpret_cast<Real4<Real>*>(S);          // x, y, z, vx
