@@ -330,7 +330,7 @@ public:
         RH_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         ls = stream;
         RH_HIP(hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming));
-        RH_HIP(hipHostMalloc(&staging, READBACK_SLOTS * READBACK_SLOT_BYTES, hipHostMallocDefault));
+        RH_HIP(hipHostMalloc(&ring.mem, READBACK_SLOTS * READBACK_SLOT_BYTES, hipHostMallocDefault));
         for (auto& e : staging_ev) RH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         for (int f = 0; f < RH_N_FIELDS; ++f) {
             fld[f].alloc((size_t)g.nc * FIELD_DIM[f]);
@@ -392,9 +392,9 @@ public:
         }
         // the staging ring's pages and the stream's copy queue, ready for the
         // first read-back (1 ms otherwise)
-        memset(staging, 0, READBACK_SLOTS * READBACK_SLOT_BYTES);
+        memset(ring.mem, 0, READBACK_SLOTS * READBACK_SLOT_BYTES);
         for (auto& e : staging_ev) {
-            RH_HIP(hipMemcpyAsync(staging, fld[RH_FACE_B].p, std::min(READBACK_SLOT_BYTES, fld[RH_FACE_B].n * sizeof(Real)),
+            RH_HIP(hipMemcpyAsync(ring.mem, fld[RH_FACE_B].p, std::min(READBACK_SLOT_BYTES, fld[RH_FACE_B].n * sizeof(Real)),
                                   hipMemcpyDeviceToHost, stream));
             RH_HIP(hipEventRecord(e, stream));
         }
@@ -424,7 +424,7 @@ public:
         for (auto e : event_pool) (void)hipEventDestroy(e);
         if (fork_ev) (void)hipEventDestroy(fork_ev);
         for (auto e : staging_ev) if (e) (void)hipEventDestroy(e);
-        if (staging) (void)hipHostFree(staging);
+        if (ring.mem) (void)hipHostFree(ring.mem);
         sp.clear();
         if (stream) (void)hipStreamDestroy(stream);
     }
@@ -742,19 +742,14 @@ public:
     void download_field(int id, double* data) override {
         if (id < 0 || id >= RH_N_FIELDS || !data) throw ArgError("bad field id or null data");
         const int dim = FIELD_DIM[id];
-        const size_t chunk = std::min((size_t)g.nc, READBACK_SLOT_BYTES / (dim * sizeof(Real)));
-        Real* slot[READBACK_SLOTS];
-        for (int q = 0; q < READBACK_SLOTS; ++q)
-            slot[q] = reinterpret_cast<Real*>(static_cast<char*>(staging) + q * READBACK_SLOT_BYTES);
-        readback<Real>(
-            (size_t)g.nc, dim, data, slot, chunk,
-            [&](size_t c, size_t first, size_t n) {
-                Real* to = slot[c % READBACK_SLOTS];
+        ring.read<Real>(
+            (size_t)g.nc, dim, data,
+            [&](size_t c, Real* to, size_t stride, size_t first, size_t n) {
                 if (n == (size_t)g.nc)  // the planes follow each other
                     RH_HIP(hipMemcpyAsync(to, fld[id].p, dim * n * sizeof(Real), hipMemcpyDeviceToHost, stream));
                 else
                     for (int l = 0; l < dim; ++l)
-                        RH_HIP(hipMemcpyAsync(to + l * chunk, fld[id].p + (size_t)l * g.nc + first, n * sizeof(Real),
+                        RH_HIP(hipMemcpyAsync(to + l * stride, fld[id].p + (size_t)l * g.nc + first, n * sizeof(Real),
                                               hipMemcpyDeviceToHost, stream));
                 RH_HIP(hipEventRecord(staging_ev[c % READBACK_SLOTS], stream));
             },
@@ -1182,7 +1177,7 @@ public:
         fill(S_.ave_v.p, 0.0, S_.ave_v.n);
     }
 
-    void* staging = nullptr;  // download_field's pinned ring
+    ReadbackRing ring;  // download_field's, pinned; its slots' events, used by who holds it
     hipEvent_t staging_ev[READBACK_SLOTS] = {};
     DevBuf<float> dn_in, dn_out, dn_filt;  // denoiser volumes, filtered density (allocated on first use)
     DevBuf<uint32_t> pf_tile;     // push fields, one block per tile (k_push_fields)

@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <cstddef>
+#include <mutex>
 
 namespace rh {
 
@@ -50,5 +51,31 @@ void readback(size_t nc, int dim, double* data, const Real* const* slot, size_t 
         if (n < chunks) copy(n, n * chunk, cells(n));
     }
 }
+
+// A context's staging ring for every array it reads back.  Host threads may
+// read arrays of one context side by side: a read holds the ring, and the
+// events of its slots, until its last chunk is converted, and the others wait
+// for it (they would share the one stream and its copy engine anyway).
+class ReadbackRing {
+public:
+    void* mem = nullptr;  // READBACK_SLOTS * READBACK_SLOT_BYTES
+
+    // copy(c, to, stride, first cell, cells) enqueues chunk c's planes to `to`,
+    // `stride` values apart; wait(c) as above.
+    template <typename Real, typename Copy, typename Wait>
+    void read(size_t nc, int dim, double* data, Copy&& copy, Wait&& wait) {
+        std::lock_guard<std::mutex> held(mu);
+        const size_t chunk = std::min(nc, READBACK_SLOT_BYTES / (dim * sizeof(Real)));
+        Real* slot[READBACK_SLOTS];
+        for (int q = 0; q < READBACK_SLOTS; ++q)
+            slot[q] = reinterpret_cast<Real*>(static_cast<char*>(mem) + q * READBACK_SLOT_BYTES);
+        readback<Real>(
+            nc, dim, data, slot, chunk,
+            [&](size_t c, size_t first, size_t n) { copy(c, slot[c % READBACK_SLOTS], chunk, first, n); }, wait);
+    }
+
+private:
+    std::mutex mu;
+};
 
 }  // namespace rh
