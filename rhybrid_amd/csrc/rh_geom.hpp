@@ -183,6 +183,35 @@ RH_HD void tile_origin(const Geom& g, int T, int& ox, int& oy, int& oz) {
     oz = (T / (g.ntx * g.nty)) * g.tz;
 }
 
+// A pushed particle that waits in place of its input keeps its extended cell
+// e < 512 there: the low eight bits as its cell byte, the ninth as the top
+// exponent bit of x, which is clear for every x a stored particle has (0 <= x
+// <= 1 or -0.0, and -1 for a removed one), so nothing else of x is lost.  No
+// sign can hold it: a position may be -0.0, and y and z may be no number.
+template <typename Real> struct TopExponent;
+template <> struct TopExponent<float> { using Bits = uint32_t; static constexpr Bits mask = 1u << 30; };
+template <> struct TopExponent<double> { using Bits = uint64_t; static constexpr Bits mask = 1ull << 62; };
+
+template <typename Real>
+RH_HD uint8_t put_ext_cell(int e, Real& x) {
+    typename TopExponent<Real>::Bits b;
+    __builtin_memcpy(&b, &x, sizeof(b));
+    if (e & 256) b |= TopExponent<Real>::mask;
+    __builtin_memcpy(&x, &b, sizeof(b));
+    return (uint8_t)e;
+}
+
+// The extended cell put there; x as it was.
+template <typename Real>
+RH_HD int take_ext_cell(uint8_t low, Real& x) {
+    typename TopExponent<Real>::Bits b;
+    __builtin_memcpy(&b, &x, sizeof(b));
+    const int e = (int)low | (b & TopExponent<Real>::mask ? 256 : 0);
+    b &= ~TopExponent<Real>::mask;
+    __builtin_memcpy(&x, &b, sizeof(b));
+    return e;
+}
+
 RH_HD uint32_t cell_key(const Geom& g, int i, int j, int k) {
     const int T = tile_of(g, i, j, k);
     const int lc = (i & (g.tx - 1)) + ((j & (g.ty - 1)) << g.ltx) + ((k & (g.tz - 1)) << (g.ltx + g.lty));

@@ -650,8 +650,10 @@ __device__ __forceinline__ uint32_t push_particle(const Geom& g, const PushParam
         // difference from its floor, which rounds to one, has after the limit)
         X = (Real)__builtin_amdgcn_fract(Xd); Y = (Real)__builtin_amdgcn_fract(Yd); Z = (Real)__builtin_amdgcn_fract(Zd);
     }
-    // at most one cell along each axis, and nothing that is not a number
-    const bool ok = (unsigned)(sx + 1) <= 2u && (unsigned)(sy + 1) <= 2u && (unsigned)(sz + 1) <= 2u && X + Y + Z >= Real(0);
+    // at most one cell along each axis, and nothing that is not a number (a
+    // still pass keeps that too)
+    const bool ok = (unsigned)(sx + 1) <= 2u && (unsigned)(sy + 1) <= 2u && (unsigned)(sz + 1) <= 2u &&
+                    (X + Y + Z >= Real(0) || (!PLAIN && pp.still));
     if (PLAIN || !pp.still) {
         X = X < Real(1) ? X : below_one<Real>();
         Y = Y < Real(1) ? Y : below_one<Real>();
@@ -907,22 +909,24 @@ __global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
         }
     } else {
         // Pushed for the counts, and written back where it came from (no other
-        // tile reads those places): its extended cell e in lc, the ninth bit
-        // of e as the sign of Y.  A removed one keeps its old state.
+        // tile reads those places) with its extended cell; a removed one is
+        // only marked, whatever its state was.
         for (uint32_t u = tid; u < N; u += NT) {
             if (u >= n0) other(u - n0, nq, nlc);
             Particle<Real> q = nq;
             const int lc = nlc;
             if (u + NT < n0) own(u + NT, nq, nlc);  // the next own one is loaded ahead
-            const Particle<Real> was = q;
             int e;
             const uint32_t c = push_particle<Real, PLAIN>(g, pp, org, edge, fl, codes, q, lc, e, n_clamped, n_dropped);
-            if ((c & SLOT_MASK) == (uint32_t)K) { q = was; e = g.next; }
             atomicAdd(&cnt[part_code(c, (int)u) & SLOT_MASK], 1u);
             const uint32_t p = place(u);
-            A.x[p] = q.X; A.y[p] = e & 256 ? -q.Y : q.Y; A.z[p] = q.Z;
+            if ((c & SLOT_MASK) == (uint32_t)K) {
+                A.x[p] = Real(-1);
+                continue;
+            }
+            A.lc[p] = put_ext_cell(e, q.X);
+            A.x[p] = q.X; A.y[p] = q.Y; A.z[p] = q.Z;
             A.vx[p] = q.vx; A.vy[p] = q.vy; A.vz[p] = q.vz;
-            A.lc[p] = (uint8_t)e;
         }
         __syncthreads();
         const uint32_t total = scan_slots(true);
@@ -938,8 +942,7 @@ __global__ __launch_bounds__(NT, sizeof(Real) == 8 ? 4 : 6) void k_push_sort(
                 Particle<Real> q;
                 q.X = A.x[p]; q.Y = A.y[p]; q.Z = A.z[p];
                 q.vx = A.vx[p]; q.vy = A.vy[p]; q.vz = A.vz[p];
-                int e = A.lc[p];
-                if (__builtin_signbit(q.Y)) { q.Y = -q.Y; e |= 256; }
+                const int e = take_ext_cell(A.lc[p], q.X);
                 uint32_t c = part_code(q.X >= Real(0) ? particle_code(codes, e, q) : (uint32_t)K, i);
                 c |= atomicAdd(&cnt[c & SLOT_MASK], 1u) << RANK_SHIFT;
                 S4[i] = Real4<Real>{{q.X, q.Y, q.Z, q.vx}};
