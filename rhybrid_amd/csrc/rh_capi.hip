@@ -959,7 +959,7 @@ public:
             most = std::max(64.0 * c, (double)S_.fill_max);
         }
         sampled += live;
-        // parts of a slot with four to eight particles each
+        // parts of a slot that count apart, about 8 to 16 particles each
         int lq = 0;
         const double per_slot = live > 0 ? np / live / (8.0 * g.tc) : 0;
         while ((g.nslot + 1) << (lq + 1) <= 1 << SLOT_BITS && per_slot >= (16 << lq)) ++lq;
