@@ -867,41 +867,78 @@ public:
         return (int64_t)t[0];
     }
 
+    // The live particles by tile and subcell, in each subcell the tile's own
+    // ones first, then its arrivals and its waiting injected ones: the order
+    // that the next push reads them in and a merge would store them in.  The
+    // store is only read (a merge here would change the order, and with it the
+    // rounding, of the steps that follow).
     void download_particles(int s, int64_t capn, int64_t* cell, double* st) override {
         Species& S_ = S(s);
         if (S_.pushed) throw StateError("download between propagate and wait_particle_sends");
-        if (S_.lists || S_.inj_pending) merge(S_);  // every particle in its own tile's segment
-        std::vector<uint32_t> tab((size_t)g.ntiles * g.kt);
-        std::vector<uint8_t> live((size_t)g.ntiles);
-        RH_HIP(hipMemcpyAsync(tab.data(), S_.tab.p, sizeof(uint32_t) * tab.size(), hipMemcpyDeviceToHost, stream));
-        RH_HIP(hipMemcpyAsync(live.data(), S_.live.p, live.size(), hipMemcpyDeviceToHost, stream));
-        const uint32_t end = scalar(S_, SC_END);
-        std::vector<Real> h[6];
-        for (int q = 0; q < 6; ++q) {
-            h[q].resize(end);
-            if (end) RH_HIP(hipMemcpy(h[q].data(), S_.a[q].p, sizeof(Real) * end, hipMemcpyDeviceToHost));
+        std::vector<uint32_t> lists((size_t)g.ntiles * LIST_WORDS), cbeg, off;
+        uint32_t sc[SC_END + 1];
+        RH_HIP(hipMemcpyAsync(lists.data(), S_.tile_list.p, sizeof(uint32_t) * lists.size(), hipMemcpyDeviceToHost, stream));
+        RH_HIP(hipMemcpyAsync(sc, S_.scal.p, sizeof(sc), hipMemcpyDeviceToHost, stream));
+        if (S_.inj_pending) {
+            cbeg.resize((size_t)g.ntiles + 1);
+            off.resize((size_t)S_.inj_ncell + 1);
+            RH_HIP(hipMemcpyAsync(cbeg.data(), S_.inj_cbeg.p, sizeof(uint32_t) * cbeg.size(), hipMemcpyDeviceToHost, stream));
+            RH_HIP(hipMemcpyAsync(off.data(), S_.inj_off.p, sizeof(uint32_t) * off.size(), hipMemcpyDeviceToHost, stream));
         }
-        // in slot order; the cell of a particle follows from the slots holding it
+        RH_HIP(hipStreamSynchronize(stream));
+        // the segments, then the appendix, as far as the push takes it
+        const InjAppendix app = S_.appendix();
+        const uint32_t np = sc[SC_NP], end = sc[SC_END];
+        const uint32_t room = std::min(S_.cap > np ? (uint32_t)S_.cap - np : 0u, app.places);
+        const uint32_t waiting = S_.inj_pending ? std::min(off.back(), room) : 0u;
+        const size_t base = app.at_end ? np : S_.cap;
+        auto fetch = [&](auto& h, const auto* a) {
+            h.resize((size_t)end + waiting);
+            if (end) RH_HIP(hipMemcpy(h.data(), a, sizeof(*a) * end, hipMemcpyDeviceToHost));
+            if (waiting) RH_HIP(hipMemcpy(h.data() + end, a + base, sizeof(*a) * waiting, hipMemcpyDeviceToHost));
+        };
+        std::vector<Real> h[6];
+        std::vector<uint8_t> hl;
+        for (int q = 0; q < 6; ++q) fetch(h[q], S_.a[q].p);
+        fetch(hl, S_.a_lc.p);
+        const size_t ns = (size_t)g.tc * 8;
+        std::vector<uint32_t> seq, sorted;   // a tile's live particles as the push reads them, and by subcell
+        std::vector<uint16_t> key;
+        std::vector<size_t> at(ns + 1);
         int64_t out = 0;
         for (int T = 0; T < g.ntiles; ++T) {
-            if (!live[T]) continue;
+            const uint32_t* L = lists.data() + (size_t)T * LIST_WORDS;
+            seq.clear();
+            key.clear();
+            std::fill(at.begin(), at.end(), 0);
+            auto take = [&](uint32_t p) {
+                if (h[0][p] < Real(0)) return;
+                const int o = (h[0][p] >= Real(0.5)) + 2 * (h[1][p] >= Real(0.5)) + 4 * (h[2][p] >= Real(0.5));
+                seq.push_back(p);
+                key.push_back((uint16_t)(8 * hl[p] + o));
+                ++at[(size_t)key.back() + 1];
+            };
+            for (uint32_t v = 0; v < L[LIST_OWN + 1]; ++v) take(L[LIST_OWN] + v);
+            for (int j = 0; j < 27; ++j)
+                for (uint32_t v = L[LIST_PREF + j]; v < L[LIST_PREF + j + 1]; ++v) take(L[LIST_START + j] + v);
+            if (waiting)
+                for (uint32_t v = std::min(off[cbeg[T]], waiting); v < std::min(off[cbeg[T + 1]], waiting); ++v) take(end + v);
+            for (size_t q = 0; q < ns; ++q) at[q + 1] += at[q];
+            sorted.resize(seq.size());
+            for (size_t q = 0; q < seq.size(); ++q) sorted[at[key[q]]++] = seq[q];
             int ox, oy, oz;
             tile_origin(g, T, ox, oy, oz);
-            for (int lc = 0; lc < g.tc; ++lc) {
-                const uint32_t* t = tab.data() + (size_t)T * g.kt + 8 * lc;
-                const int c = cell_index(g, ox + lc % g.tx, oy + (lc / g.tx) % g.ty, oz + lc / (g.tx * g.ty));
-                for (uint32_t p = t[0]; p < t[8]; ++p) {
-                    if (h[0][p] < Real(0)) continue;
-                    if (out >= capn) throw CapError("download buffer too small");
-                    if (cell) cell[out] = c;
-                    if (st) {
-                        double* q = st + 7 * out;
-                        q[0] = (double)h[0][p] * g.dx; q[1] = (double)h[1][p] * g.dx; q[2] = (double)h[2][p] * g.dx;
-                        q[3] = (double)h[3][p]; q[4] = (double)h[4][p]; q[5] = (double)h[5][p];
-                        q[6] = S_.d.w;
-                    }
-                    ++out;
+            for (uint32_t p : sorted) {
+                if (out >= capn) throw CapError("download buffer too small");
+                const int lc = hl[p];
+                if (cell) cell[out] = cell_index(g, ox + lc % g.tx, oy + (lc / g.tx) % g.ty, oz + lc / (g.tx * g.ty));
+                if (st) {
+                    double* q = st + 7 * out;
+                    q[0] = (double)h[0][p] * g.dx; q[1] = (double)h[1][p] * g.dx; q[2] = (double)h[2][p] * g.dx;
+                    q[3] = (double)h[3][p]; q[4] = (double)h[4][p]; q[5] = (double)h[5][p];
+                    q[6] = S_.d.w;
                 }
+                ++out;
             }
         }
     }
@@ -1066,13 +1103,6 @@ public:
         std::copy(sc + SC_FILL, sc + SC_N, S_.tile_fill.begin());
         S_.np_est = S_.fill_np = (double)sc[SC_NP];
         S_.fill_max = sc[SC_FILL_MAX];
-    }
-
-    uint32_t scalar(Species& S_, int id) {
-        uint32_t v = 0;
-        RH_HIP(hipMemcpyAsync(&v, S_.scal.p + id, sizeof(v), hipMemcpyDeviceToHost, stream));
-        RH_HIP(hipStreamSynchronize(stream));
-        return v;
     }
 
     void scan(const uint32_t* in, uint32_t n, uint32_t* out, std::vector<DevBuf<uint32_t>>& lv, size_t level) {
