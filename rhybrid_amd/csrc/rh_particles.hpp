@@ -1274,9 +1274,9 @@ RH_HD int deposit_chunk(const Geom& g) {
     return ((16 * 8 * deposit_octant_block(g)) / 6) & ~63;
 }
 
-
 // The deposit of a crowded tile (k_deposit sends tiles with at least
-// dense_min particles here): eight lanes share a subcell and read eight
+// dense_min particles here, whether its own or arrivals; tab null: none of
+// its own): eight lanes share a subcell and read eight
 // consecutive particles per array (one cache line per group instead of one
 // per lane), then add their sums in a fixed butterfly order; blockDim/8
 // subcells per round.  Within the same LDS as the sparse path, the two
@@ -1294,8 +1294,8 @@ __device__ void deposit_dense_tile(const Geom& g, const PArrays<Real>& A, const 
         if (half) __syncthreads();  // the first half's reads are done
         for (int base = 0; base < NS; base += ngrp) {
             const int ls = base + grp;
-            const bool valid = ls < NS;
-            const uint32_t p0 = valid ? tab[ls] : 0u, p1 = valid ? tab[ls + 1] : 0u;
+            const bool valid = ls < NS, some = valid && tab;
+            const uint32_t p0 = some ? tab[ls] : 0u, p1 = some ? tab[ls + 1] : 0u;
             const int o = ls & 7, cell = ls >> 3;
             const bool hx = o & 1, hy = (o >> 1) & 1, hz = (o >> 2) & 1;
             Real acc[2][8];
@@ -1439,7 +1439,7 @@ __global__ __launch_bounds__(512, sizeof(Real) == 8 ? 4 : 8) void k_deposit(Geom
     uint32_t p0 = 0, p1 = 0;
     if (n0) { p0 = tab[ls]; p1 = tab[ls + 1]; }
     for (int e = ls; e < LIST_WORDS; e += blockDim.x) L[e] = lists[(size_t)T * LIST_WORDS + e];
-    if (n0 >= dense_min) {
+    if (n0 + na >= dense_min) {
         if (na) {
             __syncthreads();
             deposit_arrivals(g, A, L, S, R);
@@ -1447,7 +1447,7 @@ __global__ __launch_bounds__(512, sizeof(Real) == 8 ? 4 : 8) void k_deposit(Geom
             Real* Rw = reinterpret_cast<Real*>(R);
             for (int e = ls; e < 4 * g.next; e += blockDim.x) Rw[e] = Real(0);
         }
-        deposit_dense_tile(g, A, tab, glist, gcount, partial, T, S, R);
+        deposit_dense_tile(g, A, n0 ? tab : nullptr, glist, gcount, partial, T, S, R);
         return;
     }
     const int o = ls & 7, cell = ls >> 3;
@@ -1462,20 +1462,29 @@ __global__ __launch_bounds__(512, sizeof(Real) == 8 ? 4 : 8) void k_deposit(Geom
     // subcell's particles of the chunk, in particle order.  A particle is
     // staged as (x, y, z, vx) and (vy, vz): two LDS reads instead of six.
     // The arrivals, about 3 % of the particles, are linked by subcell as they
-    // are staged; a thread takes those of its list, in ascending order, after
-    // its own.  The loops over the tile's own particles hold nothing of the
-    // arrivals in registers (64 of them let four workgroups share a CU): 128x96x96
-    // with 35.5 M particles takes 314 us a launch (2.9 TB/s; 280 where
-    // every particle lies in its own tile's segment), and took 370 with both kinds in one loop, 332 with the list
+    // are staged, in any order; then each walks its subcell's list once for
+    // the one that follows it, and a thread takes those of its list in
+    // ascending order after its own (a thread that walks its list again for
+    // every four it takes needs 21 ms for 2,000 arrivals of one subcell instead
+    // of 0.48, and 313 us on the box below).  The loops over the tile's own
+    // particles hold nothing of the arrivals in registers (64 of them let four
+    // workgroups share a CU): 128x96x96 with 35.5 M particles takes 309 us a
+    // launch (2.9 TB/s; 280 where every particle lies in its own tile's
+    // segment), and took 370 with both kinds in one loop, 332 with the list
     // read before the own ones, 392 with three own particles' loads in flight.
     const int CH = deposit_chunk<Real>(g);
     Real4<Real>* L4 = reinterpret_cast<Real4<Real>*>(S);          // x, y, z, vx
     Real2<Real>* L2 = reinterpret_cast<Real2<Real>*>(S + 4 * CH);  // vy, vz
     constexpr uint32_t NONE = 0xFFFFu;
-    uint32_t* head = reinterpret_cast<uint32_t*>(R);               // per subcell its list's first entry
-    uint16_t* next = reinterpret_cast<uint16_t*>(head + NS);       // per arrival of the chunk the next one
-    const uint32_t AR = (uint32_t)((4 * sizeof(Real) * g.next - 4 * (size_t)NS) / 2);  // arrivals of one chunk
-    head[ls] = NONE;
+    // per subcell its list's first entry as linked, and above it in order
+    uint32_t* head = reinterpret_cast<uint32_t*>(R);
+    uint16_t* lowest = reinterpret_cast<uint16_t*>(R) + 1;
+    uint16_t* next = reinterpret_cast<uint16_t*>(head + NS);  // per arrival of the chunk the next one as linked
+    // arrivals of one chunk: one a thread at most
+    const uint32_t AR = min((uint32_t)((4 * sizeof(Real) * g.next - 4 * (size_t)NS) / 4), (uint32_t)NS);
+    uint16_t* follow = next + AR;                             // and the next one in order
+    constexpr uint32_t EMPTY = NONE | NONE << 16;
+    head[ls] = EMPTY;
     uint32_t n = 0;
     for (uint32_t cs = 0; cs < n0 + na; cs += n) {
         const uint32_t qa = n0 > cs ? n0 - cs : 0u;  // the chunk's first arrival
@@ -1491,18 +1500,35 @@ __global__ __launch_bounds__(512, sizeof(Real) == 8 ? 4 : 8) void k_deposit(Geom
             L4[q] = r;
             L2[q] = t;
         }
-        for (uint32_t q = no + ls; q < n; q += blockDim.x) {
-            const uint32_t p = arrival_index(L, cs + q - n0);
+        const uint32_t mine = no + ls;               // the thread's arrival
+        uint32_t to = 0, old = NONE;                 // its subcell, and what it was linked before
+        if (mine < n) {
+            const uint32_t p = arrival_index(L, cs + mine - n0);
             Real4<Real> r;
             r.v[0] = A.x[p]; r.v[1] = A.y[p]; r.v[2] = A.z[p]; r.v[3] = A.vx[p];
             Real2<Real> t;
             t.v[0] = A.vy[p]; t.v[1] = A.vz[p];
-            L4[q] = r;
-            L2[q] = t;
+            L4[mine] = r;
+            L2[mine] = t;
             const int oct = (r.v[0] >= Real(0.5)) + 2 * (r.v[1] >= Real(0.5)) + 4 * (r.v[2] >= Real(0.5));
-            next[q - qa] = (uint16_t)atomicExch(&head[A.lc[p] * 8 + oct], q);
+            to = A.lc[p] * 8u + (uint32_t)oct;
+            old = atomicExch(&head[to], mine | NONE << 16) & 0xFFFFu;
+            next[mine - qa] = (uint16_t)old;
         }
         __syncthreads();
+        if (n > no) {
+            if (mine < n) {
+                uint32_t above = NONE;
+                bool first = true;
+                for (uint32_t h = head[to] & 0xFFFFu; h != NONE; h = h == mine ? old : next[h - qa]) {
+                    if (h > mine) above = min(above, h);
+                    first = first && h >= mine;
+                }
+                follow[mine - qa] = (uint16_t)above;
+                if (first) lowest[2 * to] = (uint16_t)mine;
+            }
+            __syncthreads();
+        }
         const uint32_t a = max(p0, t0 + cs) - t0 - cs, b = min(p1, t0 + cs + n) - t0 - cs;
         const int own = p1 > t0 + cs && p0 < t0 + cs + n && p1 > p0 ? (int)(b - a) : 0;
         for (int it = 0; it < own; ++it) {
@@ -1511,31 +1537,12 @@ __global__ __launch_bounds__(512, sizeof(Real) == 8 ? 4 : 8) void k_deposit(Geom
             cic_accumulate(acc, hx, hy, hz, r.v[0], r.v[1], r.v[2], r.v[3], t.v[0], t.v[1]);
         }
         if (n == no) continue;
-        // the list's entries above `last`, four at a time (16 bits each)
-        int last = -1;
-        for (bool more = head[ls] != NONE; more;) {
-            uint64_t four = ~0ull;
-            for (uint32_t h = head[ls]; h != NONE; h = next[h - qa]) {
-                uint32_t v = (int)h > last ? h : NONE;
-                uint64_t s = 0;
-#pragma unroll
-                for (int d = 0; d < 64; d += 16) {
-                    const uint32_t w = (uint32_t)(four >> d) & 0xFFFFu;
-                    s |= (uint64_t)min(v, w) << d;
-                    v = max(v, w);
-                }
-                four = s;
-            }
-            int k = 0;
-            for (; k < 4 && ((uint32_t)four & 0xFFFFu) != NONE; ++k, four >>= 16) {
-                last = (int)((uint32_t)four & 0xFFFFu);
-                const Real4<Real> r = L4[last];
-                const Real2<Real> t = L2[last];
-                cic_accumulate(acc, hx, hy, hz, r.v[0], r.v[1], r.v[2], r.v[3], t.v[0], t.v[1]);
-            }
-            more = k == 4;
+        for (uint32_t h = head[ls] >> 16; h != NONE; h = follow[h - qa]) {
+            const Real4<Real> r = L4[h];
+            const Real2<Real> t = L2[h];
+            cic_accumulate(acc, hx, hy, hz, r.v[0], r.v[1], r.v[2], r.v[3], t.v[0], t.v[1]);
         }
-        head[ls] = NONE;
+        head[ls] = EMPTY;
     }
     // the eight octant lanes of each cell: 64 corner sums -> 27 targets
 #pragma unroll
