@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <numeric>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -203,7 +204,7 @@ public:
     // the destination of the next push (dst, tab_new, live_new), swapped after
     // it.  `cap` places hold the segments; app_cap more, after them, the
     // appendix of injected particles that wait for their first push.
-    static constexpr int NEVER = 1 << 20, LOOK_EVERY = 8;  // steps
+    static constexpr int LOOK_EVERY = 8;  // pushes
     struct Species {
         rh_species_desc d;
         size_t cap = 0;
@@ -218,10 +219,16 @@ public:
         bool compact = true;   // the segments hold no empty places
         double np_est = 0;     // about how many particles there are
         std::array<uint32_t, FILL_CLASSES> tile_fill{};  // of the store as last looked at (k_tile_fill)
-        double fill_np = 0;    // np_est then
+        double fill_np = 0;    // particles then
         uint32_t fill_max = 0; // the most particles in a tile then, 0 if the classes tell
-        int since_look = NEVER;  // steps since then
-        bool has_lists = false;  // k_tile_lists has run
+        // the look under way: its words in pinned memory, its end, np_est at
+        // its start, the pushes since then, and how many until it is taken
+        uint32_t* look = nullptr;
+        hipEvent_t looked = nullptr;
+        bool look_pending = false;
+        double look_est = 0;
+        int since_look = 0;
+        int look_wait = 1;
         DevBuf<Real> partial;  // deposit: per-tile ghost partials (ntiles x next x 4)
         DevBuf<double> ave_n, ave_v;  // temporal averages: running charge and current sums (FP64)
         bool deposited = false;
@@ -231,6 +238,7 @@ public:
         // offset of its new particles past the store's end
         InjParams inj{};
         int inj_ncell = 0;
+        double inj_mean = 0;  // particles a step, about
         int inj_slots = 0;  // solar wind: fixed places per listed cell (ceil of the rate)
         DevBuf<int> inj_cells;
         DevBuf<double> inj_rate;
@@ -270,6 +278,9 @@ public:
         Species& operator=(const Species&) = delete;
         ~Species() {
             if (ss) (void)hipStreamSynchronize(ss);
+            if (look_pending) (void)hipEventSynchronize(looked);
+            if (looked) (void)hipEventDestroy(looked);
+            if (look) (void)hipHostFree(look);
             if (done) (void)hipEventDestroy(done);
             if (ss) (void)hipStreamDestroy(ss);
         }
@@ -685,6 +696,8 @@ public:
         RH_HIP(hipMemsetAsync(s->pcount.p, 0, sizeof(unsigned long long) * C_N * COUNTER_SLOTS, stream));
         s->bc_acc.alloc((size_t)std::max(n_bc, 1) * 4);
         fill(s->bc_acc.p, 0.0, s->bc_acc.n);
+        RH_HIP(hipHostMalloc((void**)&s->look, LOOK_WORDS * sizeof(uint32_t), hipHostMallocDefault));
+        RH_HIP(hipEventCreateWithFlags(&s->looked, hipEventDisableTiming));
         ensure_capacity(*s, (size_t)std::max<int64_t>(d->capacity, 0));
         ensure_averages(*s);
         sp.push_back(std::move(s));
@@ -851,7 +864,11 @@ public:
 
     void uploaded(Species& S_) {
         tile_lists(S_, "sort_still");
-        look_at_fill(S_);
+        take_look(S_);
+        S_.np_est = 0;
+        start_look(S_);
+        take_look(S_);
+        if (!S_.fill_np) S_.look_wait = 1;  // look again after the first push
         S_.pushed = false;
         S_.inj_pending = false;
         S_.lists = false;
@@ -1063,7 +1080,6 @@ public:
 
     // The tiles' lists of the store as it is now, and the next segments.
     void tile_lists(Species& S_, const char* name) {
-        S_.has_lists = true;
         launch(name, k_tile_lists, cdiv(g.ntiles, TILES_PER_LIST_BLOCK), LIST_THREADS, 0, g, (const uint32_t*)S_.dtab.p,
                S_.tile_list.p, S_.seg_loc.p, S_.seg_blk.p, S_.scal.p);
     }
@@ -1072,7 +1088,6 @@ public:
     // without pushing anything.
     void merge(Species& S_) {
         if (S_.pushed) throw StateError("injected particles pending between propagate and wait_particle_sends");
-        if (S_.has_lists && ++S_.since_look >= LOOK_EVERY) look_at_fill(S_);
         PushParams pp{};
         pp.still = 1;
         push(S_, pp, "sort_still");
@@ -1091,18 +1106,37 @@ public:
         S_.inj_pending = false;
         S_.lists = true;
         S_.compact = false;
+        keep_looking(S_);
     }
 
-    void look_at_fill(Species& S_) {
-        uint32_t sc[SC_N];
-        launch("tile_fill", k_tile_fill, 1, FILL_THREADS, 0, g, (const uint32_t*)S_.tile_list.p, S_.scal.p);
-        RH_HIP(hipMemcpyAsync(sc, S_.scal.p, sizeof(sc), hipMemcpyDeviceToHost, stream));
-        RH_HIP(hipStreamSynchronize(stream));
-        S_.since_look = sc[SC_NP] || !S_.np_est ? 0 : NEVER;
-        if (!sc[SC_NP]) return;  // (injected ones may be waiting)
-        std::copy(sc + SC_FILL, sc + SC_N, S_.tile_fill.begin());
-        S_.np_est = S_.fill_np = (double)sc[SC_NP];
-        S_.fill_max = sc[SC_FILL_MAX];
+    // The fill of the tiles, looked at after every LOOK_EVERY pushes whoever
+    // drives them, and taken that many later: the host then waits for what it
+    // enqueued long before, with the pushes since then still queued behind it
+    // (the first look: after the next push).
+    void keep_looking(Species& S_) {
+        if (++S_.since_look < S_.look_wait) return;
+        take_look(S_);
+        start_look(S_);
+    }
+
+    void start_look(Species& S_) {
+        launch("tile_fill", k_tile_fill, 1, FILL_THREADS, 0, g, (const uint32_t*)S_.tile_list.p, (const uint32_t*)S_.scal.p,
+               S_.look);
+        RH_HIP(hipEventRecord(S_.looked, ls));
+        S_.look_pending = true;
+        S_.look_est = S_.np_est;
+        S_.since_look = 0;
+    }
+
+    void take_look(Species& S_) {
+        if (!S_.look_pending) return;
+        RH_HIP(hipEventSynchronize(S_.looked));
+        S_.look_pending = false;
+        S_.look_wait = LOOK_EVERY;
+        std::copy(S_.look + LOOK_CLASS, S_.look + LOOK_WORDS, S_.tile_fill.begin());
+        S_.fill_np = (double)S_.look[LOOK_NP];
+        S_.fill_max = S_.look[LOOK_MOST];
+        S_.np_est = S_.fill_np + (S_.np_est - S_.look_est);  // and those injected since
     }
 
     void scan(const uint32_t* in, uint32_t n, uint32_t* out, std::vector<DevBuf<uint32_t>>& lv, size_t level) {
@@ -1429,7 +1463,7 @@ public:
 
     void step(int n) override {
         for (auto& s_ : sp)
-            if (s_->since_look >= NEVER && s_->has_lists && !s_->pushed) look_at_fill(*s_);
+            if (s_->look_wait == 1) take_look(*s_);
         for (int it = 0; it < n; ++it) {
             ++tstep;
             if (species_streams && sp.size() > 1) {
@@ -1450,11 +1484,9 @@ public:
             // (particles that a first step has only now sorted)
             if (it == 0 && n > 1)
                 for (auto& s_ : sp)
-                    if (s_->since_look >= NEVER) look_at_fill(*s_);
+                    if (s_->look_wait == 1) take_look(*s_);
         }
         check_overflow();
-        for (auto& s_ : sp)
-            if ((s_->since_look += n) >= LOOK_EVERY) look_at_fill(*s_);
     }
 
     // propagate, wait_particle_sends and accumulate of every species, each
@@ -1664,6 +1696,8 @@ public:
         S_.inj = ip;
         S_.inj_ncell = (int)hc.size();
         S_.inj_slots = slots;
+        S_.inj_mean = (double)hc.size() * ip.rate;
+        if (ip.kind == INJ_EXOSPHERE) S_.inj_mean = std::accumulate(hr.begin(), hr.end(), 0.0);
     }
 
     // ParticleInjectorBase::inject for the current timestep (nothing at
@@ -1692,7 +1726,7 @@ public:
                        (const uint32_t*)(S_.scal.p + SC_NP), ip.kind == INJ_UNIFORM ? 1 : 0, S_.A(), (uint32_t)S_.cap,
                        S_.inj_total.p, dcount.p, S_.inj_acc.p);
             S_.inj_pending = S_.inj_slots > 0;
-            S_.np_est += (double)S_.inj_ncell * S_.inj.rate;
+            S_.np_est += S_.inj_mean;
             return;
         }
         const unsigned nb = cdiv(S_.inj_ncell, 256);
@@ -1704,6 +1738,7 @@ public:
                (const uint32_t*)S_.inj_off.p, (const uint32_t*)(S_.scal.p + SC_NP), S_.A(), (uint32_t)S_.cap,
                (uint32_t)S_.app_cap, S_.inj_total.p, dcount.p, S_.inj_acc.p);
         S_.inj_pending = true;
+        S_.np_est += S_.inj_mean;
     }
 
     // ---- logs (logWriteParticleField, src/diagnostics.h:407-813) -------------

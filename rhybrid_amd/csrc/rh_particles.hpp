@@ -220,9 +220,7 @@ enum DevScalar {
     SC_NP = 0,   // particles in the segments (removed ones included until the next push)
     SC_END,      // store indices in use by the segments
     SC_TICKET,   // blocks of k_tile_lists that are done
-    SC_FILL_MAX, // k_tile_fill's fullest tile, and its FILL_CLASSES counts
-    SC_FILL,
-    SC_N = SC_FILL + 128
+    SC_N
 };
 
 // Per tile DIR_WORDS store indices: where its halo slots of direction d begin
@@ -437,13 +435,15 @@ __global__ __launch_bounds__(LIST_THREADS) void k_tile_lists(Geom g, const uint3
 // How full the tiles are, for the choice of the push's workgroups: of about
 // FILL_SAMPLE tiles spread over the grid the number that hold
 // 64c-63 .. 64c particles, per class c (the last class also fuller ones;
-// empty tiles are class 0), and the most that one holds.  One block, once per
-// run of steps.
-constexpr int FILL_CLASSES = SC_N - SC_FILL, FILL_SAMPLE = 4096, FILL_THREADS = 1024;
+// empty tiles are class 0), and the most that one holds.  One block, every few
+// pushes; it writes to pinned memory of the host (words LOOK_*), which waits
+// for an event after it: no copy that the next kernels would queue behind.
+constexpr int FILL_CLASSES = 128, FILL_SAMPLE = 4096, FILL_THREADS = 1024;
+enum LookWord { LOOK_NP = 0, LOOK_MOST, LOOK_CLASS, LOOK_WORDS = LOOK_CLASS + FILL_CLASSES };
 RH_HD int fill_class(uint32_t n) { return n >= 64u * (FILL_CLASSES - 1) ? FILL_CLASSES - 1 : (int)((n + 63u) / 64u); }
 
 __global__ __launch_bounds__(FILL_THREADS) void k_tile_fill(Geom g, const uint32_t* __restrict__ lists,
-                                                            uint32_t* __restrict__ scal) {
+                                                            const uint32_t* __restrict__ scal, uint32_t* __restrict__ look) {
     __shared__ uint32_t h[FILL_CLASSES], most;
     const int tid = threadIdx.x, stride = (g.ntiles + FILL_SAMPLE - 1) / FILL_SAMPLE;
     if (tid < FILL_CLASSES) h[tid] = 0;
@@ -456,8 +456,11 @@ __global__ __launch_bounds__(FILL_THREADS) void k_tile_fill(Geom g, const uint32
         if (n >= 64u * (FILL_CLASSES - 1)) atomicMax(&most, n);
     }
     __syncthreads();
-    if (tid < FILL_CLASSES) scal[SC_FILL + tid] = h[tid];
-    if (tid == 0) scal[SC_FILL_MAX] = most;
+    if (tid < FILL_CLASSES) look[LOOK_CLASS + tid] = h[tid];
+    if (tid == 0) {
+        look[LOOK_NP] = scal[SC_NP];
+        look[LOOK_MOST] = most;
+    }
 }
 
 // A Geom whose tile shape is known to the compiler: sides 2^LX, 2^LY, 2^LZ
