@@ -23,8 +23,8 @@
 //    channels, K = 32 voxels.  The workgroups are persistent; each stages
 //    16x4x4 voxel tiles into LDS as they lie in memory (channels last), reads
 //    the fragments' voxel runs with LDS transpose reads, and keeps its taps'
-//    partial sums in registers; k_wgrad_reduce adds the per-workgroup
-//    partials in a fixed order.
+//    partial sums in registers; k_wgrad_reduce adds the partials in FP64, in a
+//    fixed order.
 //
 // Fragment lane layouts (checked on the device): for 16x16x32, lane l holds
 // A[l%16][8*(l/16) .. +7], B[8*(l/16) .. +7][l%16] and D[4*(l/16) + i][l%16].
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(64 * TZ_) void k_conv(ConvArgs a) {
 // 16-channel halves lie apart and a row is WPX = 20 voxels long: then a read
 // of two rows meets each bank twice, the least that 512 bytes can.  Bound by
 // LDS reads and MFMA alike (about 2,000 cycles each per tile and CU).
-// 8 volumes of 32^3, 32 -> 32 channels: 26 us; 59 to 67 with a tile transposed by
+// 8 volumes of 32^3, 32 -> 32 channels: 27 us; 59 to 67 with a tile transposed by
 // 2-byte LDS writes into three shifted copies, two workgroups of four waves a CU.
 constexpr int WX = 16, WY = 4, WZ = 4, WK = WX * WY * WZ;
 constexpr int WHY = WY + 2, WHZ = WZ + 2, WPX = 20;
@@ -231,6 +231,7 @@ constexpr int WHV = (WX + 2) * WHY * WHZ, WPV = WPX * WHY * WHZ;  // the halo's 
 constexpr int WTAPS = 7;       // taps per wave (27 = 7+7+7+6)
 constexpr int WG_THREADS = 512;
 constexpr int WGRAD_BLOCKS = 256;  // persistent workgroups, one per CU
+constexpr int WGRAD_PARTS = 2 * WGRAD_BLOCKS;  // their partial sums, one per half of the planes
 
 typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
 
@@ -251,9 +252,7 @@ __global__ __launch_bounds__(WG_THREADS, 2) void k_wgrad(const bf16* __restrict_
     constexpr int BI = CIN < 16 ? 16 : 32, BO = COUT < 16 ? 16 : 32;  // bytes of a voxel's 8 or 16 channels
     constexpr int CHI = CIN / 8, CHG = COUT / 8;
     constexpr int X_BYTES = MT * WPV * BI, BUF = X_BYTES + NT * WK * BO;
-    constexpr int ACC_BYTES = 4 * WTAPS * MT * NT * 64 * 16;
-    constexpr int LDS = 2 * BUF > ACC_BYTES ? 2 * BUF : ACC_BYTES;
-    __shared__ __attribute__((aligned(16))) unsigned char lds[LDS];
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * BUF];
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), wt = w & 3, wh = w >> 2;
     const int m = lane & 15, kg = lane >> 4;
     const int ntx = X / WX, nty = Y / WY, ntz = Z / WZ;
@@ -346,19 +345,10 @@ __global__ __launch_bounds__(WG_THREADS, 2) void k_wgrad(const bf16* __restrict_
         if (more) store(lds + cur * BUF);
         __syncthreads();  // the next tile is there, and this one's buffer is free
     }
-    // the two halves of the planes added through LDS
-    floatx4* sum = reinterpret_cast<floatx4*>(lds);
-#pragma unroll
-    for (int t = 0; t < WTAPS; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                if (wh == 1) sum[(((wt * WTAPS + t) * MT + mt) * NT + nt) * 64 + lane] = acc[t][mt][nt];
-    __syncthreads();
-    if (wh == 1) return;
-    // partial[block][tap][ci][co]; lane holds D[ci = 4*kg + i][co = m] of each tile
-    float* out = part + (size_t)blockIdx.x * NTAP * CI * CO;
+    // partial[block][half of the planes][tap][ci][co] without the padding; lane
+    // holds D[ci = 4*kg + i][co = m] of each tile
+    if ((CIN < 16 && kg >= CIN / 4) || (COUT < 16 && m >= COUT)) return;
+    float* out = part + ((size_t)blockIdx.x * 2 + wh) * NTAP * CIN * COUT;
 #pragma unroll
     for (int t = 0; t < WTAPS; ++t) {
         const int tap = wt + 4 * t;
@@ -366,23 +356,22 @@ __global__ __launch_bounds__(WG_THREADS, 2) void k_wgrad(const bf16* __restrict_
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const floatx4 o = sum[(((wt * WTAPS + t) * MT + mt) * NT + nt) * 64 + lane];
+            for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    out[((size_t)tap * CI + mt * 16 + 4 * kg + i) * CO + nt * 16 + m] = acc[t][mt][nt][i] + o[i];
-            }
+                    out[((size_t)tap * CIN + mt * 16 + 4 * kg + i) * COUT + nt * 16 + m] = acc[t][mt][nt][i];
     }
 }
 
-// grad[offset + (co*cin + ci)*27 + tap] = sum over workgroups in a fixed
-// order, all layers in one launch: a block takes 64 consecutive entries of a
-// layer's partials (256 bytes of each workgroup's) x RED_G groups of
-// workgroups; group g sums workgroups g, g+RED_G, ... and the group sums are
-// added in order of g.  Entries of padding channels are not read.  Bound by
-// the partials' 85 MB, which are still in the last-level cache: 23 us for 256
-// workgroups; 100 in four launches that read 32 bytes at a time of 512.
-constexpr int RED_W = 64, RED_G = 16;
+// grad[offset + (co*cin + ci)*27 + tap] = sum over the partials in a fixed
+// order, in FP64, all layers in one launch: a block takes RED_E consecutive
+// entries of a layer's partials, four a thread, x RED_G groups of partials;
+// group g sums partials g, g+RED_G, ... and the group sums are added in order
+// of g.  The two halves of a workgroup's planes are partials of their own (an
+// FP32 sum of them lost what FP64 keeps).  Bound by the partials' 142 MB, 26 us
+// for 256 workgroups (5.5 TB/s); 47 with one entry a thread and the padding
+// channels stored (170 MB), 100 in four launches that read 32 bytes at a time.
+constexpr int RED_W = 32, RED_G = 32, RED_E = 4 * RED_W;
 struct WgradLayer {
     int ci, co, cin, cout, offset, block0;  // padded and real channels, first weight, first block
     const float* part;
@@ -390,30 +379,37 @@ struct WgradLayer {
 struct WgradLayers {
     WgradLayer l[4];
 };
-constexpr int wgrad_words(int l) {  // of one workgroup's partials
-    return NTAP * (LAYERS[l].cin < 16 ? 16 : LAYERS[l].cin) * (LAYERS[l].cout < 16 ? 16 : LAYERS[l].cout);
-}
+// channels of a layer's arrays: 7 and 4 are padded to 8
+constexpr int padded(int channels) { return channels < 8 ? 8 : channels; }
+constexpr int wgrad_words(int l) { return NTAP * padded(LAYERS[l].cin) * padded(LAYERS[l].cout); }  // of one partial
 
-__global__ __launch_bounds__(RED_W * RED_G) void k_wgrad_reduce(WgradLayers a, int nblk, float* __restrict__ grad) {
-    __shared__ double red[RED_G][RED_W];
+static_assert(wgrad_words(0) % RED_E == 0 && wgrad_words(1) % RED_E == 0 && wgrad_words(3) % RED_E == 0, "whole blocks");
+
+__global__ __launch_bounds__(RED_W * RED_G) void k_wgrad_reduce(WgradLayers a, int nparts, float* __restrict__ grad) {
+    __shared__ double red[RED_G][RED_E];
     int q = 0;
     while (q < 3 && (int)blockIdx.x >= a.l[q + 1].block0) ++q;
     const WgradLayer L = a.l[q];
     const int wl = threadIdx.x % RED_W, gi = threadIdx.x / RED_W;
-    const int e = ((int)blockIdx.x - L.block0) * RED_W + wl;
-    const int co = e % L.co, ci = e / L.co % L.ci, tap = e / (L.co * L.ci);
+    const int e0 = ((int)blockIdx.x - L.block0) * RED_E;
     const size_t stride = (size_t)NTAP * L.ci * L.co;
-    const bool real = co < L.cout && ci < L.cin && tap < NTAP;
-    double s = 0.0;
-    if (real)
-        for (int b = gi; b < nblk; b += RED_G) s += L.part[b * stride + e];
-    red[gi][wl] = s;
-    __syncthreads();
-    if (gi == 0 && real) {
-        double t = 0.0;
-        for (int g = 0; g < RED_G; ++g) t += red[g][wl];
-        grad[L.offset + ((size_t)co * L.cin + ci) * NTAP + tap] = (float)t;
+    const float* from = L.part + e0 + 4 * wl;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+    for (int b = gi; b < nparts; b += RED_G) {
+        const floatx4 v = *reinterpret_cast<const floatx4*>(from + b * stride);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] += v[j];
     }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) red[gi][4 * wl + j] = s[j];
+    __syncthreads();
+    if (threadIdx.x >= RED_E) return;
+    const int e = e0 + (int)threadIdx.x, co = e % L.co, ci = e / L.co % L.ci, tap = e / (L.co * L.ci);
+    if (co >= L.cout || ci >= L.cin) return;  // padding
+    double t = 0.0;
+    for (int g = 0; g < RED_G; ++g) t += red[g][threadIdx.x];
+    grad[L.offset + ((size_t)co * L.cin + ci) * NTAP + tap] = (float)t;
 }
 
 // packed B fragments of one layer.  KP = 32: fragment f = tap*NT + nt,
@@ -671,7 +667,7 @@ struct rh_denoiser {
         g2.alloc(V * 32);
         g1.alloc(V * 32);
         y.alloc(V * 4);
-        part.alloc((size_t)WGRAD_BLOCKS * (wgrad_words(0) + wgrad_words(1) + wgrad_words(2) + wgrad_words(3)));
+        part.alloc((size_t)WGRAD_PARTS * (wgrad_words(0) + wgrad_words(1) + wgrad_words(2) + wgrad_words(3)));
         lpart.alloc(1024);
         DN_HIP(hipMemsetAsync(w.p, 0, RH_DN_N_WEIGHTS * sizeof(float), stream));
         reset_adam();
@@ -752,7 +748,7 @@ struct rh_denoiser {
 
     float* wgrad_part(int layer) {
         size_t at = 0;
-        for (int l = 0; l < layer; ++l) at += (size_t)WGRAD_BLOCKS * wgrad_words(l);
+        for (int l = 0; l < layer; ++l) at += (size_t)WGRAD_PARTS * wgrad_words(l);
         return part.p + at;
     }
     static int wgrad_blocks(int P, int X, int Y, int Z) {
@@ -769,10 +765,10 @@ struct rh_denoiser {
         int blocks = 0;
         for (int l = 0; l < 4; ++l) {
             const Layer& L = LAYERS[l];
-            a.l[l] = {L.cin < 16 ? 16 : L.cin, L.cout < 16 ? 16 : L.cout, L.cin, L.cout, L.offset, blocks, wgrad_part(l)};
-            blocks += (int)cdiv(wgrad_words(l), RED_W);
+            a.l[l] = {padded(L.cin), padded(L.cout), L.cin, L.cout, L.offset, blocks, wgrad_part(l)};
+            blocks += wgrad_words(l) / RED_E;
         }
-        launch("wgrad_reduce", k_wgrad_reduce, dim3(blocks), dim3(RED_W * RED_G), a, wgrad_blocks(P, X, Y, Z), g.p);
+        launch("wgrad_reduce", k_wgrad_reduce, dim3(blocks), dim3(RED_W * RED_G), a, 2 * wgrad_blocks(P, X, Y, Z), g.p);
     }
 
     // forward + loss + backward into g; loss left in `loss`
