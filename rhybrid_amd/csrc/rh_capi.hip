@@ -1070,8 +1070,11 @@ public:
     void push_launch(Species& S_, const PushParams& pp, const char* name, int round, int lq) {
         const size_t lds = push_lds<Real>(g, round, lq).bytes;
         auto kernel = k_push_sort<Real, NT, LX, LY, LZ, PLAIN>;
+        // (the same value in every call: the attribute is the kernel's, and
+        // contexts of several threads share the kernel)
         if (lds > 65536)
-            RH_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            RH_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)std::min(lds_limit, (size_t)PUSH_MAX_LDS)));
         launch(name, kernel, tile_grid(), NT, lds, g, pp,
                (const uint32_t*)pf_tile.p, S_.A(), S_.Dst(), (const uint16_t*)slot_dir.p, (const uint16_t*)slot_of.p,
                (const uint32_t*)slot_code.p, S_.tab_new.p, S_.dtab.p, S_.live_new.p, (const uint32_t*)S_.tile_list.p, (const uint32_t*)S_.seg_loc.p,
