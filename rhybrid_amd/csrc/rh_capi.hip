@@ -412,9 +412,9 @@ public:
         RH_HIP(hipStreamSynchronize(stream));
     }
 
-    // block sums of a scan over nkeys elements, per level
+    // block sums of a scan over the injection's cells (at most all), per level
     void alloc_scan_levels(std::vector<DevBuf<uint32_t>>& lv) {
-        size_t n = (size_t)g.nkeys;
+        size_t n = (size_t)g.nc;
         while (n > (size_t)SCAN_TILE) {
             const size_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
             lv.emplace_back();
@@ -510,7 +510,7 @@ public:
         g.next = g.ex * g.ey * g.ez;
         g.extk = g.next * 8;
         set_slots(g);
-        if (g.extk > MAX_EXTK) throw ArgError("tile extended region too large");
+        if (g.next > MAX_NEXT || g.nslot > (int)SLOT_MASK) throw ArgError("tile extended region too large");
         const uint64_t nk = (uint64_t)g.ntiles * g.tc * 8;
         if (nk >= 0xFFFFFFFFull) throw ArgError("grid too large for 32-bit subcell keys");
         if ((uint64_t)g.ntiles * std::max(g.extk, g.kt) >= 0xFFFFFFFFull) throw ArgError("tiles too small for this grid (slot table)");
@@ -655,7 +655,7 @@ public:
 
     static unsigned cdiv(size_t a, size_t b) { return (unsigned)((a + b - 1) / b); }
     // per-tile launches: one workgroup per tile in XCD-aware order (xcd_tile)
-    dim3 tile_grid() const { return dim3(N_XCD * g.xchunk); }
+    dim3 tile_grid() const { return dim3(N_XCD * cdiv(g.ntiles, N_XCD)); }
     dim3 cell_grid() const { return dim3(cdiv(g.nx, 32), cdiv(g.ny, 8), g.nz); }
     static dim3 cell_block() { return dim3(32, 8, 1); }
 
@@ -1251,7 +1251,7 @@ public:
     bool pf_dirty = true;         // fields changed since the blocks were written
 
     // The blocks of the push fields are rewritten when the fields have
-    // changed; both passes of every species then read the same blocks.
+    // changed; the pushes of all species then read the same blocks.
     void alloc_push_fields() {
         if (pf_tile.p) return;
         pf_tile.alloc((size_t)g.ntiles * push_field_words<Real>(g));

@@ -48,7 +48,7 @@ typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
 typedef __attribute__((__vector_size__(4 * sizeof(__bf16)))) __bf16 bf16x4;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float floatx4;
 
-constexpr int TX = 16, HX = TX + 2;  // x extent of a convolution's output tile, and with its halo
+constexpr int TX = 16, TY = 4, HX = TX + 2, HY = TY + 2;  // extents of a convolution's output tile, and with its halo
 constexpr int NTAP = 27;
 
 struct Layer {
@@ -76,10 +76,10 @@ __device__ __forceinline__ floatx4 mfma(bf16x8 a, bf16x8 b, floatx4 c) {
 // Convolution over zero-padded volumes; CIN in {8, 32}, NT output tiles of 16.
 // A workgroup computes a 16x4xTZ_ tile, one wave per z plane (TZ_ = 4 or 8:
 // the taller tile stages 10 halo planes for 8 output planes instead of 6 for 4).
-template <int CIN, int NT, int EP, int TY, int TZ_>
+template <int CIN, int NT, int EP, int TZ_>
 __global__ __launch_bounds__(64 * TZ_) void k_conv(ConvArgs a) {
     constexpr int CH = CIN / 8;  // 16-byte chunks per voxel
-    constexpr int HY = TY + 2, HZ_ = TZ_ + 2, HV_ = HX * HY * HZ_, NTH = 64 * TZ_;
+    constexpr int HZ_ = TZ_ + 2, HV_ = HX * HY * HZ_, NTH = 64 * TZ_;
     __shared__ bf16x8 tile[HV_ * CH];
     // the first weight group of the 32-channel path, loaded while the halo is staged
     bf16x8 bnx[3][NT];
@@ -717,14 +717,14 @@ struct rh_denoiser {
         a.yout = yo;
         a.xres = xres;
         for (int c = 0; c < 4; ++c) a.s[c] = scale[c];
-        if (Z % 8 == 0) conv_launch<CIN, NT, EP, 4, 8>(name, a, P);
-        else conv_launch<CIN, NT, EP, 4, 4>(name, a, P);
+        if (Z % 8 == 0) conv_launch<CIN, NT, EP, 8>(name, a, P);
+        else conv_launch<CIN, NT, EP, 4>(name, a, P);
     }
 
-    template <int CIN, int NT, int EP, int TY, int TZ>
+    template <int CIN, int NT, int EP, int TZ>
     void conv_launch(const char* name, ConvArgs& a, int P) {
         a.nzb = a.Z / TZ;
-        launch(name, k_conv<CIN, NT, EP, TY, TZ>, dim3(a.X / TX, a.Y / TY, P * a.nzb), dim3(64 * TZ), a);
+        launch(name, k_conv<CIN, NT, EP, TZ>, dim3(a.X / TX, a.Y / TY, P * a.nzb), dim3(64 * TZ), a);
     }
 
     // The forward pass with the packed input in bx8 and the activations of

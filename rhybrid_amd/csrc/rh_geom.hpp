@@ -1,20 +1,24 @@
 // rh_geom.hpp -- grid and tile geometry shared by host and device code.
 //
 // Cells are numbered as in the reference, n = i + nx*(j + ny*k) (ParGrid
-// global ids with x fastest, src/particle_list_hybrid.h:89-91).  Particles are
-// kept sorted by *subcell key* in tile-major order:
+// global ids with x fastest, src/particle_list_hybrid.h:89-91).  The grid is cut
+// into tiles of tx*ty*tz cells, and every cell into eight subcells: the octant
+// says in which half of the cell a particle sits along each axis (bit0: x >=
+// dx/2, bit1: y, bit2: z).  The *subcell key* is
 //   key = ((tile * tc) + local_cell) * 8 + octant
-// where the grid is cut into tiles of tx*ty*tz cells, local_cell is the cell's
-// index inside its tile (x fastest) and the octant says in which half of the
-// cell the particle sits along each axis (bit0: x >= dx/2, bit1: y, bit2: z).
-// A tile's particles are one contiguous range, each cell's particles are one
-// contiguous range, and each subcell's particles share one 2x2x2 cloud-in-
-// cell footprint, which is what the deposit exploits.
+// with local_cell the cell's index inside its tile (x fastest).  A subcell's
+// particles share one 2x2x2 cloud-in-cell footprint, which is what the deposit
+// exploits.
 //
 // The "extended region" of a tile is the tile grown by one cell on every side,
 // (tx+2)*(ty+2)*(tz+2) cells with local coordinates -1..t.  A particle pushed
 // out of a cell of the tile lands in the extended region (moves are at most
 // one cell per step), and a deposit from the tile's subcells only touches it.
+//
+// A tile owns one contiguous segment of the particle store, in slot order: the
+// slots are the tile's subcells, then the extended region's other cells.  After
+// a push a segment holds the particles that stayed in the tile, by subcell,
+// then those that left it, by the cell they left to (rh_particles.hpp).
 #pragma once
 
 #include <cstdint>
@@ -29,11 +33,7 @@
 
 namespace rh {
 
-constexpr uint32_t DEAD_CELL = 0xFFFFFFFFu;  // particle marked for removal
-constexpr uint32_t DEAD_PACKED = 0xFFFFFFFFu;
-constexpr int RANK_BITS = 20;
-constexpr uint32_t RANK_MASK = (1u << RANK_BITS) - 1u;
-constexpr int MAX_EXTK = 4095;               // ext cells * 8 must fit 12 bits (4095 = dead)
+constexpr int MAX_NEXT = 511;  // cells of an extended region, and one index past them: nine bits (put_ext_cell)
 
 struct Geom {
     int nx, ny, nz, nc;
@@ -47,7 +47,7 @@ struct Geom {
     int extk;                  // next * 8 subcell slots in the extended region
     uint32_t nkeys;            // ntiles * tc * 8
     int nslot, kt;             // subcell and halo-cell slots of a tile; entries per tile of the slot tables
-    int xpx, xpy, xpz, xchunk; // XCD bricks: parts per axis (product 8), most tiles in one brick
+    int xpx, xpy, xpz, xchunk; // XCD bricks: parts per axis (product 8), workgroups per XCD that cover either order
 };
 
 // slots of the tile shape: 8 subcells per cell of the tile, one per halo cell
@@ -116,20 +116,16 @@ RH_HD void local_ijk(const Geom& g, int lc, int& li, int& lj, int& lk) {
 
 // XCD-aware tile orders.  The hardware deals the workgroups of a launch to
 // the eight XCDs (each with its own L2) in turn, workgroup b to XCD b % 8.
-// Per-tile launches use a 1D grid of 8 * xchunk workgroups (xchunk covers
-// both orders); a result >= ntiles is no tile.
+// A result >= ntiles is no tile.
 //   xcd_tile: XCD x takes the contiguous range [x * chunk, (x + 1) * chunk)
 //   of the x-fastest tile order (slabs of whole tile layers), so that tiles
-//   neighbouring in memory run on one XCD close in time.  The push and the
-//   deposit, which read each tile's particle range, run in this order.
+//   neighbouring in memory run on one XCD close in time.  Every per-tile
+//   launch runs in this order, with 8 * chunk workgroups.
 //   xcd_brick_tile: the tile grid cut into eight bricks (xpx x xpy x xpz
-//   parts per axis), XCD x taking brick x, x-fastest.  The move writes the
-//   particles that cross into a neighbour tile into that tile's subcell
-//   ranges, in cache lines the neighbour's own workgroup also writes; within
-//   a brick those two workgroups share an L2 and run closer in time than in
-//   slabs, and bricks share fewer faces between XCDs (the move 519 -> 500 us
-//   per launch on the 128x96x96 box; the deposit and the push were slower
-//   in this order, 289 -> 307 us).
+//   parts per axis), XCD x taking brick x, x-fastest.  For kernels that write
+//   into their neighbours' cache lines, which two workgroups of a brick do in
+//   one L2; none does now, and the deposit, which does not, took 307 us in
+//   this order instead of 289 (128x96x96 cells).
 constexpr int N_XCD = 8;
 RH_HD int xcd_tile(const Geom& g, int b) {
     const int chunk = (g.ntiles + N_XCD - 1) / N_XCD;

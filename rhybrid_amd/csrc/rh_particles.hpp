@@ -9,7 +9,7 @@
 //            segment that holds none
 //   vx,vy,vz velocity in m/s
 //   lc       the particle's cell inside its tile (implied by the sort order,
-//            kept so that kernels need not search the subcell ranges)
+//            kept so that kernels need not search the slots' ranges)
 // in one segment per tile, sorted inside it by slot; TileTables says where
 // each slot's particles are.
 #pragma once
@@ -45,7 +45,6 @@ struct PushParams {
     double GMdt;
     int accelerate, use_e_pressure, use_gravity, initial_flow_through;
     int still;           // sort only: no acceleration, no move
-    uint8_t* live;       // pass 0 writes, per tile, whether it holds particles
 };
 
 enum DevCounter { C_MAX_VI = 0, C_MIN_CELL_RHO, C_MAX_CELL_UE, C_MIN_NODE_RHO, C_MAX_NODE_UE,
