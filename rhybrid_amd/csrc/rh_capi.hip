@@ -1032,7 +1032,8 @@ public:
                 double units = 0;
                 for (int c = 1; c < FILL_CLASSES; ++c)
                     if (fill[c]) units += fill[c] * passes(c == FILL_CLASSES - 1 || 64 * c > round ? std::max(in_class(c), round + 1.0) : in_class(c), 1.0);
-                // (the registers of the kernel are made for 24 waves a CU)
+                // (the registers of the FP32 kernel are held to 24 waves a CU;
+                // those of the FP64 one to 16, and the same model serves it)
                 const double waves = std::min(k, 1536 / threads) * threads / 64.0;
                 const double all_us = (units * threads * std::pow(24.0 / waves, 0.65) / 124e3 + fill[0] * 1.5 / (256 * k)) *
                                       (g.ntiles / std::max(sampled, 1.0));
